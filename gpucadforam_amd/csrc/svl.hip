@@ -16,10 +16,9 @@
 //     round trip) and one fused pass upsamples the three phase fields and
 //     sums every harmonic per fine point as products of e^{i Phi_x},
 //     e^{i Phi_y}, e^{i Phi_z}.
-//   * the unit-cell Fourier coefficients by direct DFT (FP64 accumulation)
+//   * the unit-cell Fourier coefficients by separable direct DFT (FP64 accumulation)
 //     for exactly the (2r+1)^3 coefficients the reference keeps.
 #include <cmath>
-#include <vector>
 
 #include "gc_common.hpp"
 #include "gc_math.hpp"
@@ -327,6 +326,28 @@ __device__ __forceinline__ double block_sum(double v) {
         __syncthreads();
     }
     return s[0];
+}
+
+// one step of the wave sum: v plus the DPP-moved v (0 where no lane is the source)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+    return v + __longlong_as_double((long long)((uint64_t)(uint32_t)hi << 32 | (uint32_t)lo));
+}
+// sum over the 64 lanes, the same in every lane (DPP moves: no LDS)
+__device__ __forceinline__ double wave_sum_d(double v) {
+    v = dpp_add<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8 within rows of 16 lanes
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15, 31: lane 63 holds the sum
+    v = dpp_add<0x143, 0xc>(v);
+    const long long b = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)b, 63);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
 }
 
 // the same fixed-order sum of G partials in every block (so every block
@@ -679,40 +700,98 @@ __global__ void svl_field_kernel(const float *phix, const float *phiy, const flo
 // (1/N) sum f(x,y,z) e^{-2 pi i (i x/nx + j y/ny + k z/nz)}, the forward R2C
 // transform scaled as fft_scalar does (Fft_lattice.cu) and picked as
 // unit_lattice does (src/main.cu:3578-3711: loop k, j, i over [-r, r])
+//
+// Separable: the x sums of every row for i = 0..r (the cell is real, so -i is
+// the conjugate), then one workgroup per (i >= 0, j, k) over the rows.  Sums
+// and twiddles in FP64.  Bound by latency, the cell is small: 61^3,
+// r = 2 took 290 us with a workgroup per coefficient over the whole cell, the
+// two passes take 5.1 + 6.1 us.
 // ---------------------------------------------------------------------------
-__global__ void dft_kernel(const float *cell, int nx, int ny, int nz, int range,
-                           const double2 *tw /* (nx+ny+nz) * (2r+1) twiddles */, float2 *out) {
-    const int side = 2 * range + 1;
-    const int h = blockIdx.x;
-    const int i = h % side, j = (h / side) % side, k = h / (side * side);
-    const double2 *tx = tw + (uint64_t)i * nx;
-    const double2 *ty = tw + (uint64_t)side * nx + (uint64_t)j * ny;
-    const double2 *tz = tw + (uint64_t)side * (nx + ny) + (uint64_t)k * nz;
-    const uint64_t n = (uint64_t)nx * ny * nz;
-    double re = 0.0, im = 0.0;
-    for (uint64_t t = threadIdx.x; t < n; t += blockDim.x) {
-        int x, y, z;
-        point_xyz(t, nx, ny, &x, &y, &z);
-        const double2 a = tx[x], b = ty[y], c = tz[z];
-        const double abr = a.x * b.x - a.y * b.y, abi = a.x * b.y + a.y * b.x;
-        const double er = abr * c.x - abi * c.y, ei = abr * c.y + abi * c.x;
-        const double f = cell[t];
-        re += f * er;
-        im += f * ei;
-    }
-    __shared__ double sr[256], si[256];
-    sr[threadIdx.x] = re;
-    si[threadIdx.x] = im;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            sr[threadIdx.x] += sr[threadIdx.x + w];
-            si[threadIdx.x] += si[threadIdx.x + w];
+// (cos, -sin)(2 pi num / n), num < n
+__device__ __forceinline__ double2 twiddle(uint32_t num, uint32_t n) {
+    double s, c;
+    sincospi(2.0 * (double)num / (double)n, &s, &c);
+    return make_double2(c, -s);
+}
+__device__ __forceinline__ double2 cmuld(double2 a, double2 b) {
+    return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
+}
+constexpr int kDftRows = 4;  // rows per wave: a wave's twiddles serve all of them
+
+// rows[i * nrows + row] = sum over x of f(x, row) e^{-2 pi i ix/nx}, i = 0..R
+template <int R>
+__global__ void __launch_bounds__(256) dft_rows_kernel(const float *cell, int nx, uint32_t nrows,
+                                                       double2 *rows) {
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * kDftRows;
+    if (row0 >= nrows) return;
+    double2 acc[kDftRows][R + 1];
+#pragma unroll
+    for (int q = 0; q < kDftRows; ++q)
+#pragma unroll
+        for (int i = 0; i <= R; ++i) acc[q][i] = make_double2(0.0, 0.0);
+    for (uint32_t x = lane; x < (uint32_t)nx; x += 64) {
+        double2 e[R + 2];  // powers of e^{-2 pi i x/nx}
+        e[0] = make_double2(1.0, 0.0);
+        if constexpr (R > 0) e[1] = twiddle(x, (uint32_t)nx);
+#pragma unroll
+        for (int i = 2; i <= R; ++i) e[i] = cmuld(e[i - 1], e[1]);
+#pragma unroll
+        for (int q = 0; q < kDftRows; ++q) {
+            const uint32_t row = row0 + q < nrows ? row0 + q : row0;
+            const double f = cell[(uint64_t)row * nx + x];
+#pragma unroll
+            for (int i = 0; i <= R; ++i) {
+                acc[q][i].x = fma(f, e[i].x, acc[q][i].x);
+                acc[q][i].y = fma(f, e[i].y, acc[q][i].y);
+            }
         }
-        __syncthreads();
     }
-    if (threadIdx.x == 0)
-        out[h] = make_float2((float)(sr[0] / (double)n), (float)(si[0] / (double)n));
+#pragma unroll
+    for (int q = 0; q < kDftRows; ++q)
+#pragma unroll
+        for (int i = 0; i <= R; ++i) {
+            const double2 v = make_double2(wave_sum_d(acc[q][i].x), wave_sum_d(acc[q][i].y));
+            if (lane == 0 && row0 + q < nrows) rows[(uint64_t)i * nrows + row0 + q] = v;
+        }
+}
+
+// workgroup (i, j, k): the rows' sums over y and z; writes (i, j, k) and its
+// mirror image (-i, -j, -k)
+__global__ void __launch_bounds__(256) dft_planes_kernel(const double2 *rows, int ny, int nz,
+                                                         int range, double cells, float2 *out) {
+    const int side = 2 * range + 1;
+    const int j = (int)(blockIdx.x % side) - range, k = (int)(blockIdx.x / side) - range;
+    const int i = (int)blockIdx.y;
+    const uint32_t nrows = (uint32_t)ny * (uint32_t)nz;
+    double re = 0.0, im = 0.0;
+    for (uint32_t t = threadIdx.x; t < nrows; t += 256) {
+        const uint32_t z = t / (uint32_t)ny, y = t - z * (uint32_t)ny;
+        // the angle in periods (at most 2 range of them, so rounded to about 1e-15)
+        const double a = (double)((int64_t)j * y) / (double)ny + (double)((int64_t)k * z) / (double)nz;
+        double s, c;
+        sincospi(2.0 * a, &s, &c);
+        const double2 v = cmuld(rows[(uint64_t)i * nrows + t], make_double2(c, -s));
+        re += v.x;
+        im += v.y;
+    }
+    __shared__ double sr[4], si[4];
+    re = wave_sum_d(re);
+    im = wave_sum_d(im);
+    if ((threadIdx.x & 63) == 0) {
+        sr[threadIdx.x >> 6] = re;
+        si[threadIdx.x >> 6] = im;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const float vr = (float)(((sr[0] + sr[1]) + (sr[2] + sr[3])) / cells);
+        const float vi = (float)(((si[0] + si[1]) + (si[2] + si[3])) / cells);
+        auto at = [=](int a, int b, int c) {
+            return (a + range) + side * ((b + range) + side * (c + range));
+        };
+        out[at(i, j, k)] = make_float2(vr, vi);
+        if (i > 0) out[at(-i, -j, -k)] = make_float2(vr, -vi);
+    }
 }
 
 // fft_fill_kernel (Fft_lattice.cu): the half spectrum (nx/2+1 columns) into
@@ -1105,26 +1184,21 @@ int gpucad_unit_spectrum(const float *d_cell, int32_t nx, int32_t ny, int32_t nz
     if (st) return st;
     GC_ARG(range >= 0 && range <= kMaxRange, "range must be in [0, %d]", kMaxRange);
     const int side = 2 * range + 1;
-    // twiddles e^{-2 pi i m x / n} for m = -r..r on each axis, in double
-    std::vector<double2> tw((uint64_t)side * (nx + ny + nz));
-    const int dims[3] = {nx, ny, nz};
-    uint64_t o = 0;
-    for (int a = 0; a < 3; ++a) {
-        for (int m = -range; m <= range; ++m) {
-            for (int x = 0; x < dims[a]; ++x) {
-                // reduce m x mod n first so the angle stays in one period
-                const long long q = (((long long)m * x) % dims[a] + dims[a]) % dims[a];
-                const double ang = -kTwoPi * (double)q / (double)dims[a];
-                tw[o++] = make_double2(std::cos(ang), std::sin(ang));
-            }
-        }
-    }
+    const uint32_t nrows = (uint32_t)((uint64_t)ny * nz);
     void *ws = nullptr;
-    st = scratch_arena(tw.size() * sizeof(double2), &ws);
+    st = scratch_arena((uint64_t)(range + 1) * nrows * sizeof(double2), &ws);
     if (st) return st;
-    GC_HIP(hipMemcpy(ws, tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(dft_kernel, dim3((unsigned)(side * side * side)), dim3(256), 0, 0, d_cell,
-                       nx, ny, nz, range, (const double2 *)ws, (float2 *)d_coeffs);
+    double2 *rows = (double2 *)ws;
+    typedef void (*RowsKernel)(const float *, int, uint32_t, double2 *);
+    static const RowsKernel kRows[kMaxRange + 1] = {dft_rows_kernel<0>, dft_rows_kernel<1>,
+                                                    dft_rows_kernel<2>, dft_rows_kernel<3>,
+                                                    dft_rows_kernel<4>};
+    hipLaunchKernelGGL(kRows[range], dim3((nrows - 1) / (4 * kDftRows) + 1), dim3(256), 0, 0, d_cell,
+                       nx, nrows, rows);
+    GC_CHECK_LAUNCH();
+    hipLaunchKernelGGL(dft_planes_kernel, dim3((unsigned)(side * side), (unsigned)(range + 1)),
+                       dim3(256), 0, 0, rows, ny, nz, range, (double)nx * ny * nz,
+                       (float2 *)d_coeffs);
     GC_CHECK_LAUNCH();
     GC_HIP(hipStreamSynchronize(0));
     return GPUCAD_OK;
