@@ -489,66 +489,675 @@ __global__ void cg_b_kernel(CgArgs a, int it) {
     if (threadIdx.x == 0) a.prr[((uint64_t)((it + 1) & 1) * m + s) * a.G + blockIdx.x] = tot;
 }
 
-// Solves A x = b for m right-hand sides (b: m vectors of n, x written over
-// b when x == b).  Iterations run in chunks between host checks of the done
-// flags; a finished right-hand side leaves the kernels at their first test.
-int cg_solve(const float *b, float *x, int m, int nx, int ny, int nz, int max_iter, float end_res,
-             int *iters, float *res, hipStream_t st) {
-    const uint64_t n = (uint64_t)nx * ny * nz;
-    CgArgs a;
-    a.nx = nx;
-    a.ny = ny;
-    a.nz = nz;
-    a.n = n;
-    a.dnx = make_div32((uint32_t)nx);
-    a.dplane = make_div32((uint32_t)nx * (uint32_t)ny);
+// ---------------------------------------------------------------------------
+// The same iteration in one launch, for grids whose vectors fit on the chip
+// ---------------------------------------------------------------------------
+// The two-launch form moves ten vectors through memory per iteration and pays
+// two launches.  Here a workgroup keeps a tile of one right-hand side for
+// the whole solve: r, phi and q in registers (a thread owns a column of the
+// tile, one (x, y), and its z run), d in LDS with two points around the tile.
+// Tiles span the grid along x and split y and z.  Per iteration the tiles
+// exchange r on their faces (two layers; each tile updates its halo of d by the
+// same d = r + beta d as the owner, so d needs no exchange) and meet twice, in
+// the sums d.q and r.r.  Every element sees the arithmetic of the two-launch
+// form in the same order; the sums are FP64 over the same products.
+//
+// There are no fences: an exchanged value travels in one 8-byte word with the
+// number of its iteration, written and read by relaxed agent-scope atomics,
+// so a word is valid as soon as its number is the expected one.  A face or sum
+// word is written again only after its writer passed a sum that every reader
+// posted to after reading the word's last value.
+//
+// All workgroups must be resident together: at most one per CU is launched.
+// Every wait is bounded in time: should other work hold the CUs that long, the
+// waiting workgroups leave, nothing has been written to x, and the caller
+// solves by the two-launch form.
+//
+// Measured (us per iteration, two-launch form -> this): three right-hand
+// sides of 120^3 41 -> 20.4; one of 120^3 26.8 -> 12.4, of 61 x 57 x 70 13.7 -> 8.1, of
+// 12^3 (one tile) 13.1 -> 7.2.  What is left is latency: two exchanges of about 2 us each
+// and the barriers of a workgroup that fills its CU.
+constexpr int kChipThreads = 1024;            // most threads of a tile's workgroup
+constexpr int kChipZ = 24;                    // longest z run of a tile
+constexpr int kYPass = 3;                     // most passes over a halo layer of a y side
+constexpr size_t kChipLds = 160 * 1024 - 1024;  // LDS of a tile's d (1 KB: the sums)
+constexpr int64_t kChipWaitTicks = 20000000;  // longest wait: 0.2 s of the 100 MHz clock
+
+struct ChipArgs {
+    int nx, ny, nz, m, ty, tz, G;  // G = ty * tz tiles per right-hand side
+    uint64_t n;
+    const float *b;             // m right-hand sides
+    float *phi;                 // their solutions, complete when every `done` is set
+    uint64_t *faces;            // [m][G][4][face_words]: r, iteration
+    uint64_t *sums;             // [m][2][G][2]: FP64 halves, iteration
+    uint32_t face_words;
+    uint32_t *abort;            // set by a workgroup whose wait ran out
+    CgState *st;
+    int max_iter;
+    float term;
+};
+
+// The same value, unknown to the optimiser: what is computed from it inside the
+// iteration stays there instead of being held in registers throughout.
+__device__ __forceinline__ int here(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ int here_uniform(int v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+struct ChipShared {
+    double part[kChipThreads / 64], total[kChipThreads / 64];
+    int abort;
+};
+
+__device__ __forceinline__ void post_word(uint64_t *p, uint32_t value, uint32_t it) {
+    __hip_atomic_store(p, (uint64_t)it << 32 | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t read_word(const uint64_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A bounded wait: false once the time has run out or another workgroup gave up.
+struct ChipWait {
+    int64_t start = 0;
+    uint32_t turns = 0;
+    __device__ __forceinline__ bool again(uint32_t *abort) {
+        if ((++turns & 63u) != 0) return true;
+        const int64_t now = (int64_t)wall_clock64();
+        if (start == 0) start = now;
+        if (now - start > kChipWaitTicks)
+            __hip_atomic_store(abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+    }
+};
+
+// Sum of v over the workgroups of a right-hand side, the same bits in every
+// one (each sums all of them in the same order), in two halves: the
+// workgroup's own sum is posted, and then all of them are collected (false
+// when a wait ran out).  One barrier each.
+__device__ __forceinline__ void chip_post(double v, uint64_t *slots, int g, uint32_t it,
+                                          ChipShared &sh) {
+    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6, waves = (int)blockDim.x >> 6;
+    v = wave_sum_d(v);
+    if (lane == 0) sh.part[wave] = v;
+    __syncthreads();
+    if (wave == 0) {
+        const double w = wave_sum_d(lane < waves ? sh.part[lane] : 0.0);
+        if (lane == 0 && sh.abort == 0) {  // (a sum without its halo is not posted)
+            const uint64_t bits = (uint64_t)__double_as_longlong(w);
+            post_word(slots + 2 * g, (uint32_t)(bits >> 32), it);
+            post_word(slots + 2 * g + 1, (uint32_t)bits, it);
+        }
+    }
+}
+__device__ __forceinline__ bool chip_collect(const uint64_t *slots, int G, uint32_t it,
+                                             uint32_t *abort, ChipShared &sh, double *total) {
+    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6, used = (G + 63) >> 6;
+    if (wave < used) {
+        double w = 0.0;
+        bool ok = true;
+        if (t < G) {
+            ChipWait wait;
+            uint64_t hi, lo;
+            for (;;) {
+                hi = read_word(slots + 2 * t);
+                lo = read_word(slots + 2 * t + 1);
+                if ((uint32_t)(hi >> 32) == it && (uint32_t)(lo >> 32) == it) break;
+                if (!wait.again(abort)) {
+                    ok = false;
+                    break;
+                }
+            }
+            w = __longlong_as_double((long long)(hi << 32 | (lo & 0xffffffffull)));
+        }
+        if (!ok) sh.abort = 1;
+        w = wave_sum_d(w);
+        if (lane == 0) sh.total[wave] = w;
+    }
+    __syncthreads();
+    double s = 0.0;
+    for (int i = 0; i < used; ++i) s += sh.total[i];
+    *total = s;
+    return sh.abort == 0;
+}
+
+// the two neighbour terms of coordinate c of n (axis_terms): offsets in points and weights
+struct AxisTerms {
+    int o2, o3;
+    float w, k2, k3;
+};
+__device__ __forceinline__ AxisTerms axis_terms_at(int c, int n) {
+    const bool lo = c <= 1, hi1 = c == n - 2, hi0 = c == n - 1;
+    AxisTerms a;
+    a.w = (lo || hi1 || hi0) ? 1.25f : 0.5f;
+    a.o2 = c == 0 ? 1 : (c == 1 ? -1 : -2);
+    a.k2 = lo ? -1.0f : -0.25f;
+    a.o3 = lo ? 2 : (hi1 ? 1 : (hi0 ? -1 : 2));
+    a.k3 = lo ? -0.25f : ((hi1 || hi0) ? -1.0f : -0.25f);
+    return a;
+}
+
+// A tile's z runs are held in registers: KZ is the tiles' longest run rounded
+// up to 4, and every run is at least KZ - 4.  The z loops are unrolled over KZ
+// with the arrays assigned in every step and no branch around a step (steps
+// past the run compute on its last plane and are not stored, summed or sent):
+// branches that merge the arrays made the compiler spill them.
+template <int KZ>
+__global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
+    extern __shared__ float lds_d[];
+    __shared__ ChipShared sh;
+    // workgroups are dispatched to the 8 XCDs round robin: each XCD gets a
+    // contiguous run of tiles (y fastest), so most faces are exchanged through
+    // its own L2
+    const int tile = (int)((blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3));
+    if (tile >= a.G * a.m) return;
+    const int s = tile / a.G, g = tile - s * a.G, t = (int)threadIdx.x;
+    const int iy = g % a.ty, iz = g / a.ty, nx = a.nx;
+    const int y0 = (int)((int64_t)a.ny * iy / a.ty), y1 = (int)((int64_t)a.ny * (iy + 1) / a.ty);
+    const int z0 = (int)((int64_t)a.nz * iz / a.tz), z1 = (int)((int64_t)a.nz * (iz + 1) / a.tz);
+    const int by = y1 - y0, bz = z1 - z0;
+    const bool ylo = iy > 0, yhi = iy + 1 < a.ty, zlo = iz > 0, zhi = iz + 1 < a.tz;
+    const int rows = (int)blockDim.x / nx;  // tile rows a pass of the workgroup covers
+    const int row = t / nx, x = t - row * nx;
+    const bool own = row < by;              // (rows >= by)
+    const int ty = own ? row : 0;           // threads without a column follow column 0's
+    const float *b = a.b + (uint64_t)s * a.n;
+    if (t == 0) sh.abort = 0;
+    __syncthreads();
+
+    // d in LDS: the tile's planes with two rows before and after, then two
+    // planes below and two above (by rows each)
+    const int ps = (by + 4) * nx, zoff = bz * ps;
+    // (point of column offset xy = y nx + x in plane z, or in layer l, 0 next
+    // to the tile, of a z side)
+    auto at = [=](int xy, int z) { return z * ps + 2 * nx + xy; };
+    auto at_z = [=](int side, int l, int xy) { return zoff + (2 * side + l) * by * nx + xy; };
+    // The column offset and the position within the grid are taken through
+    // here() in every phase: what derives from them is computed there instead of
+    // being held in registers over the whole iteration.
+    const int column = ty * nx + x;
+    auto face = [=](int tile, int f) {
+        return a.faces + (((uint64_t)s * a.G + tile) * 4 + f) * a.face_words;
+    };
+    // Past the grid's ends along z the halo holds 4 d of the point whose -d the
+    // operator takes there (axis_terms: rows 0, 1, nz - 2, nz - 1 have -d(1),
+    // -d(0), -d(nz - 1), -d(nz - 2) in the place of -0.25 d two planes off), so
+    // every plane has the one form -0.25 d(-2) - 0.25 d(+2).
+    auto ghosts = [&](int n) {  // from the thread's own column
+        const int xy = here(column), c = at(xy, 0), cz = at_z(0, 0, xy);
+        if (!zlo && own) {
+            lds_d[cz] = 4.0f * lds_d[c];
+            lds_d[cz + by * nx] = 4.0f * lds_d[c + ps];
+        }
+        if (!zhi && own) {
+            lds_d[cz + 2 * by * nx] = 4.0f * lds_d[c + (n - 1) * ps];
+            lds_d[cz + 3 * by * nx] = 4.0f * lds_d[c + (n - 2) * ps];
+        }
+    };
+    // step z exists: only the last four steps can be past the run
+#define GC_IN_RUN(z, n) ((z) < KZ - 4 || (z) < (n))
+
+    float r[KZ], phi[KZ], q[KZ];
+    double acc = 0.0;
+    {
+        const float *bp = b + ((uint64_t)z0 * a.ny + (y0 + ty)) * nx + x;
+        const uint64_t plane = (uint64_t)a.ny * nx;
+#pragma unroll
+        for (int z = 0; z < KZ; ++z) {
+            phi[z] = 0.f;
+            r[z] = bp[(uint64_t)min(z, bz - 1) * plane];
+            if ((z & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int z = 0; z < KZ; ++z)
+            if (GC_IN_RUN(z, bz) && own) {
+                lds_d[at(column, z)] = r[z];
+                acc += (double)r[z] * (double)r[z];
+            }
+    }
+    ghosts(bz);
+    // The halo's rows: layer l of a y side has a row per z (thread row `row`
+    // takes rows row + p * rows, p < kYPass), layer l of a z side a row per y (its
+    // own column's).  Its first values come from b, later ones from the faces:
+    // face 0 / 1 holds the tile's first / last two rows, 2 / 3 its first / last two
+    // planes, layer by layer from the outside.
+    if (row < rows) {
+        for (int l = 0; l < 2; ++l)
+            for (int z = row; z < bz; z += rows) {
+                const float *p = b + ((uint64_t)(z0 + z) * a.ny + y0) * nx + x;
+                if (ylo) lds_d[at((-1 - l) * nx + x, z)] = p[-(1 + l) * nx];
+                if (yhi) lds_d[at((by + l) * nx + x, z)] = p[(by + l) * nx];
+            }
+        for (int l = 0; l < 2; ++l) {
+            const float *p = b + ((uint64_t)z0 * a.ny + y0 + ty) * nx + x;
+            const int64_t plane = (int64_t)a.ny * nx;
+            if (own && zlo) lds_d[at_z(0, l, column)] = p[-(1 + l) * plane];
+            if (own && zhi) lds_d[at_z(1, l, column)] = p[(bz + l) * plane];
+        }
+    }
+    uint64_t *const sums_dq = a.sums + (uint64_t)s * 4 * a.G, *const sums_rr = sums_dq + 2 * a.G;
+    const bool fetch = row < rows;
+
+    double tot;
+    chip_post(acc, sums_rr, g, 1u, sh);
+    if (!chip_collect(sums_rr, a.G, 1u, a.abort, sh, &tot)) return;
+    float delta = (float)tot, delta_prev = 0.f, beta = 0.f;
+    float hy[2][2][kYPass], hz[2][2];  // the halo's r: [side][layer][pass], [side][layer]
+    int it = 0;
+    for (;; ++it) {
+        if (!(it + 1 < a.max_iter && delta > a.term)) break;
+        if (it > 0) {
+            // d = r + beta d: the tile's own points, then its halo
+            const int n = here_uniform(bz), xy = here(column);
+            float *d = lds_d + at(xy, 0);
+            if (own) {
+#pragma unroll
+                for (int z = 0; z < KZ; ++z) {
+                    if (GC_IN_RUN(z, n)) *d = __builtin_fmaf(beta, *d, r[z]);
+                    d += ps;
+                    if ((z & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            ghosts(n);
+            if (fetch) {
+                const int hr = here(row), hx = here(x) + hr * ps;
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    if (!(side ? yhi : ylo)) continue;
+#pragma unroll
+                    for (int l = 0; l < 2; ++l) {
+                        float *h = lds_d + at(hx + (side ? by + l : -1 - l) * nx, 0);
+#pragma unroll
+                        for (int p = 0; p < kYPass; ++p) {
+                            if (hr + p * rows < n) *h = __builtin_fmaf(beta, *h, hy[side][l][p]);
+                            h += rows * ps;
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (own) {
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    if (!(side ? zhi : zlo)) continue;
+#pragma unroll
+                    for (int l = 0; l < 2; ++l) {
+                        float *h = lds_d + at_z(side, l, xy);
+                        *h = __builtin_fmaf(beta, *h, hz[side][l]);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        // q = A d and d.q; the z terms from a run of five d values
+        acc = 0.0;
+        {
+            const int n = here_uniform(bz), last = by * nx, xy = here(column);
+            const int cz = at_z(1, 0, xy);
+            int c = at(xy, 0);
+            const AxisTerms ax = axis_terms_at(here(x), nx);
+            const AxisTerms ay = axis_terms_at(y0 + here(ty), a.ny);
+            const int ox2 = ax.o2, ox3 = ax.o3, oy2 = ay.o2 * nx, oy3 = ay.o3 * nx;
+            const float wxy = ax.w + ay.w;
+            const int lo_edge = here_uniform(zlo ? -1 : 2), hi_edge = here_uniform(zhi ? KZ : bz - 2);
+            float dm2 = lds_d[at_z(0, 1, xy)], dm1 = lds_d[at_z(0, 0, xy)];
+            float dc = lds_d[c], dp1 = lds_d[c + ps];
+            // two planes up: in the tile, in its halo, then past both (not used)
+            int up = n > 2 ? c + 2 * ps : cz;
+#pragma unroll
+            for (int z = 0; z < KZ; ++z) {
+                const float dp2 = lds_d[up];
+                const float wz = z < lo_edge || z >= hi_edge ? 1.25f : 0.5f;
+                float v = __builtin_fmaf(wxy + wz, dc, ax.k2 * lds_d[c + ox2]);
+                v = v + ax.k3 * lds_d[c + ox3];
+                v = v + ay.k2 * lds_d[c + oy2];
+                v = v + ay.k3 * lds_d[c + oy3];
+                v = v + -0.25f * dm2;
+                v = v + -0.25f * dp2;
+                asm volatile("" : "+v"(v));  // (computed here, not where it is used)
+                q[z] = v;
+                if (GC_IN_RUN(z, n)) acc += (double)dc * (double)v;
+                dm2 = dm1;
+                dm1 = dc;
+                dc = dp1;
+                dp1 = dp2;
+                c += GC_IN_RUN(z + 1, n) ? ps : 0;
+                up = z + 3 < n ? up + ps : (z + 3 == n ? cz : cz + last);
+                // (the later steps' reads stay behind: the state fills the registers)
+                if (z & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!own) acc = 0.0;
+        }
+        chip_post(acc, sums_dq, g, (uint32_t)it + 1u, sh);
+        if (!chip_collect(sums_dq, a.G, (uint32_t)it + 1u, a.abort, sh, &tot)) return;
+        const float alpha = delta / (float)tot;
+        // phi += alpha d, r -= alpha q, the new r on the faces, r.r
+        acc = 0.0;
+        const uint32_t tag = (uint32_t)it + 1u;
+        {
+            const int n = here_uniform(bz), fstep = by * nx, xy = here(column), y = here(ty);
+            int c = at(xy, 0);
+            const bool send_lo = own && y < 2 && ylo, send_hi = own && y >= by - 2 && yhi;
+            // 32-bit offsets from the tile's faces
+            uint64_t *const f = face(g, 0);
+            const uint32_t fw = a.face_words, hx = (uint32_t)here(x), fz = 2 * fw + (uint32_t)xy;
+            uint32_t lo = (uint32_t)(y * n * nx) + hx;
+            uint32_t hi = fw + (uint32_t)((by - 1 - y) * n * nx) + hx;
+#pragma unroll
+            for (int z = 0; z < KZ; ++z) {
+                const float d = lds_d[c];
+                phi[z] = __builtin_fmaf(alpha, d, phi[z]);
+                r[z] = __builtin_fmaf(-alpha, q[z], r[z]);
+                asm volatile("" : "+v"(phi[z]), "+v"(r[z]));  // (not vectors of them)
+                if (GC_IN_RUN(z, n)) {
+                    acc += (double)r[z] * (double)r[z];
+                    const uint32_t bits = __float_as_uint(r[z]);
+                    if (send_lo) post_word(f + lo, bits, tag);
+                    if (send_hi) post_word(f + hi, bits, tag);
+                    if (z < 2 && zlo && own) post_word(f + (fz + (uint32_t)(z * fstep)), bits, tag);
+                    if (z >= KZ - 6 && z >= n - 2 && zhi && own)
+                        post_word(f + (fz + fw + (uint32_t)((n - 1 - z) * fstep)), bits, tag);
+                }
+                c += GC_IN_RUN(z + 1, n) ? ps : 0;
+                lo += nx;
+                hi += nx;
+                if (z & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!own) acc = 0.0;
+        }
+        chip_post(acc, sums_rr, g, (uint32_t)it + 2u, sh);
+        // the neighbours' new r, all words in flight at once and together with
+        // the sum's
+        bool ok = true;
+        {
+            const int n = here_uniform(bz);
+            uint64_t vy[2][2][kYPass], vz[2][2];
+            const uint64_t none = (uint64_t)tag << 32;  // nothing to read: as read
+            // (uniform addresses plus 32-bit lane offsets)
+            const int hr = here(row);
+            const uint32_t xr = (uint32_t)(hr * nx + here(x)), xy = (uint32_t)here(column);
+            const uint64_t *py[2] = {face(ylo ? g - 1 : g, 1), face(yhi ? g + 1 : g, 0)};
+            const uint64_t *pz[2] = {face(zlo ? g - a.ty : g, 3), face(zhi ? g + a.ty : g, 2)};
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                const bool hasy = fetch && (side ? yhi : ylo), hasz = own && (side ? zhi : zlo);
+#pragma unroll
+                for (int l = 0; l < 2; ++l) {
+#pragma unroll
+                    for (int p = 0; p < kYPass; ++p)
+                        vy[side][l][p] = hasy && hr + p * rows < n
+                                             ? read_word(py[side] + (l * n + p * rows) * nx + xr)
+                                             : none;
+                    vz[side][l] = hasz ? read_word(pz[side] + l * by * nx + xy) : none;
+                }
+            }
+            ChipWait wait;
+            auto settle = [&](uint64_t v, const uint64_t *w) {
+                while ((uint32_t)(v >> 32) != tag) {
+                    if (!wait.again(a.abort)) {
+                        ok = false;
+                        break;
+                    }
+                    v = read_word(w);
+                }
+                uint32_t bits = (uint32_t)v;
+                asm volatile("" : "+v"(bits));  // (one register each, not vectors of them)
+                return __uint_as_float(bits);
+            };
+#pragma unroll
+            for (int side = 0; side < 2; ++side)
+#pragma unroll
+                for (int l = 0; l < 2; ++l) {
+#pragma unroll
+                    for (int p = 0; p < kYPass; ++p)
+                        hy[side][l][p] =
+                            settle(vy[side][l][p], py[side] + (l * n + p * rows) * nx + xr);
+                    hz[side][l] = settle(vz[side][l], pz[side] + l * by * nx + xy);
+                }
+        }
+        if (!ok) sh.abort = 1;  // (read after the next barrier)
+        if (!chip_collect(sums_rr, a.G, (uint32_t)it + 2u, a.abort, sh, &tot)) return;
+        delta_prev = delta;
+        delta = (float)tot;
+        beta = delta / delta_prev;
+    }
+    if (own) {
+        float *o = a.phi + (uint64_t)s * a.n + ((uint64_t)z0 * a.ny + (y0 + ty)) * nx + x;
+        const uint64_t plane = (uint64_t)a.ny * nx;
+#pragma unroll
+        for (int z = 0; z < KZ; ++z)
+            if (z < bz) o[z * plane] = phi[z];
+    }
+    if (g == 0 && t == 0) {
+        a.st[s].iters = it + 1;
+        a.st[s].res = sqrtf(delta);
+        a.st[s].done = 1;
+    }
+#undef GC_IN_RUN
+}
+
+// zeroes the exchange words (a stale iteration number must not be read) and
+// the states and abort flag behind them
+__global__ void chip_clear_kernel(uint64_t *p, uint64_t words) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words;
+         i += (uint64_t)gridDim.x * blockDim.x)
+        p[i] = 0;
+}
+
+// The tiles of one right-hand side, or ty = 0 when the grid does not fit.
+struct ChipPlan {
+    int ty = 0, tz = 0, threads = 0;
+    uint32_t face_words = 0;
+    size_t lds = 0;
+};
+
+// Every tile at least two points along y and z (a halo reaches one tile), its
+// columns one per thread, its z run in registers, its d in LDS, all tiles of
+// all right-hand sides on `cus` workgroups.  Of these the split with the
+// least work per iteration: a z step of the tile, the halo rows a pass of the
+// workgroup fetches, and the sums' words (weights from timings).
+ChipPlan chip_plan(int nx, int ny, int nz, int m, int cus) {
+    ChipPlan best;
+    double best_cost = 1e30;
+    if (nx * 2 > kChipThreads) return best;
+    for (int ty = 1; ty <= ny / 2 && ty * m <= cus; ++ty) {
+        const int by = (ny + ty - 1) / ty;
+        if (by * nx > kChipThreads) continue;
+        const int threads = std::min(kChipThreads, std::max(256, (by * nx + 63) / 64 * 64));
+        for (int tz = 1; tz <= nz / 2 && ty * tz * m <= cus; ++tz) {
+            const int bz = (nz + tz - 1) / tz;
+            if (bz > kChipZ) continue;
+            const size_t lds = ((size_t)bz * (by + 4) + 4 * (size_t)by) * nx * sizeof(float);
+            if (lds > kChipLds) continue;
+            const int rows = threads / nx;
+            if (ty > 1 && (bz + rows - 1) / rows > kYPass) continue;
+            const int halo = (ty > 1 ? (4 * bz + rows - 1) / rows : 0) +
+                             (tz > 1 ? (4 * by + rows - 1) / rows : 0);
+            const double cost = 60.0 * bz * threads / 1024 + 40.0 * halo + 4.0 * ty * tz;
+            if (cost < best_cost) {
+                best_cost = cost;
+                best.ty = ty;
+                best.tz = tz;
+                best.threads = threads;
+                best.face_words = (uint32_t)(2 * std::max(by, bz) * nx);
+                best.lds = lds;
+            }
+        }
+    }
+    return best;
+}
+
+int cg_cus(int *cus) {
+    int dev = 0;
+    GC_HIP(hipGetDevice(&dev));
+    GC_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
+    return GPUCAD_OK;
+}
+
+struct ChipLayout {
+    uint64_t faces, sums, state, bytes;  // offsets, the first word 0
+};
+ChipLayout chip_layout(const ChipPlan &p, int m) {
+    const uint64_t G = (uint64_t)p.ty * p.tz;
+    ChipLayout l;
+    l.faces = 0;
+    l.sums = l.faces + (uint64_t)m * G * 4 * p.face_words * 8;
+    l.state = l.sums + (uint64_t)m * G * 4 * 8;
+    l.bytes = l.state + kMaxRhs * sizeof(CgState) + 64;
+    return l;
+}
+
+// Vectors of the two-launch form: 5 slots of m vectors, partial sums, states.
+struct CgLayout {
+    uint64_t slot, bytes;
+    int G;
+    uint64_t C;
+};
+CgLayout cg_layout(uint64_t n, int m) {
+    CgLayout l;
     // about kCgResident workgroups in all (one wave of them, none waiting),
     // fewer when ranges of one step per thread cover the grid
     const uint64_t steps = (n + kCgStep - 1) / kCgStep;
-    a.G = (int)std::min<uint64_t>((steps + 7) & ~uint64_t(7), std::max(8, (kCgResident / m) & ~7));
-    a.C = ((n + a.G - 1) / a.G + kCgThreads - 1) / kCgThreads * kCgThreads;
+    l.G = (int)std::min<uint64_t>((steps + 7) & ~uint64_t(7), std::max(8, (kCgResident / m) & ~7));
+    l.C = ((n + l.G - 1) / l.G + kCgThreads - 1) / kCgThreads * kCgThreads;
+    l.slot = (m * n * sizeof(float) + 255) & ~uint64_t(255);  // 256-byte aligned vectors
+    l.bytes = 5 * l.slot + (uint64_t)m * l.G * 8 * 3 + kMaxRhs * sizeof(CgState) + 1024;
+    return l;
+}
+
+// The solve on the chip: m right-hand sides b, solutions into x (x may be b),
+// ws holding m * n floats and the exchange words.  *solved says whether it
+// ran to its end.
+int cg_chip_solve(const ChipPlan &p, const float *b, float *x, int m, int nx, int ny, int nz,
+                  int max_iter, float end_res, CgState *h, void *ws, bool *solved, hipStream_t st) {
+    const ChipLayout l = chip_layout(p, m);
+    const uint64_t n = (uint64_t)nx * ny * nz;
+    const uint64_t vec = (m * n * sizeof(float) + 255) & ~uint64_t(255);
+    char *w = (char *)ws + vec;
+    ChipArgs a;
+    a.nx = nx;
+    a.ny = ny;
+    a.nz = nz;
+    a.m = m;
+    a.ty = p.ty;
+    a.tz = p.tz;
+    a.G = p.ty * p.tz;
+    a.n = n;
+    a.b = b;
+    a.phi = (float *)ws;
+    a.faces = (uint64_t *)(w + l.faces);
+    a.sums = (uint64_t *)(w + l.sums);
+    a.face_words = p.face_words;
+    a.st = (CgState *)(w + l.state);
+    a.abort = (uint32_t *)(w + l.state + kMaxRhs * sizeof(CgState));
     a.max_iter = max_iter;
     a.term = end_res * end_res;
-    const uint64_t vec = m * n * sizeof(float);
-    const uint64_t slot = (vec + 255) & ~uint64_t(255);  // 256-byte aligned vectors
-    const uint64_t bytes = 5 * slot + (uint64_t)m * a.G * 8 * 3 + kMaxRhs * sizeof(CgState) + 1024;
-    void *ws = nullptr;
-    int rc = scratch_arena(bytes, &ws);
-    if (rc) return rc;
-    char *w = (char *)ws;
-    a.phi = (float *)w;
-    a.r = (float *)(w + slot);
-    a.q = (float *)(w + 2 * slot);
-    a.d0 = (float *)(w + 3 * slot);
-    a.d1 = (float *)(w + 4 * slot);
-    a.pq = (double *)(w + 5 * slot);
-    a.prr = a.pq + (uint64_t)m * a.G;
-    a.st = (CgState *)(a.prr + 2 * (uint64_t)m * a.G);
-    const dim3 grid((unsigned)a.G, (unsigned)m);
-    hipLaunchKernelGGL(cg_init_kernel, grid, dim3(kCgThreads), 0, st, b, a);
+    *solved = false;
+    typedef void (*ChipKernel)(ChipArgs);
+    const int bz = (nz + p.tz - 1) / p.tz;
+    static_assert(kChipZ == 24, "one kernel per four planes");
+    static const ChipKernel kernels[6] = {cg_chip_kernel<4>,  cg_chip_kernel<8>,
+                                          cg_chip_kernel<12>, cg_chip_kernel<16>,
+                                          cg_chip_kernel<20>, cg_chip_kernel<24>};
+    const ChipKernel kernel = kernels[(bz + 3) / 4 - 1];
+    GC_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)kChipLds));
+    const uint64_t words = l.bytes / 8;
+    hipLaunchKernelGGL(chip_clear_kernel, dim3((unsigned)std::min<uint64_t>((words + 255) / 256, 2048)),
+                       dim3(256), 0, st, (uint64_t *)w, words);
     GC_CHECK_LAUNCH();
-    constexpr int kChunk = 16;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((a.G * m + 7) / 8 * 8)), dim3(p.threads), p.lds, st, a);
+    GC_CHECK_LAUNCH();
+    GC_HIP(hipMemcpyAsync(h, a.st, m * sizeof(CgState), hipMemcpyDeviceToHost, st));
+    GC_HIP(hipStreamSynchronize(st));
+    for (int s = 0; s < m; ++s)
+        if (!h[s].done) return GPUCAD_OK;
+    GC_HIP(hipMemcpyAsync(x, a.phi, m * n * sizeof(float), hipMemcpyDeviceToDevice, st));
+    *solved = true;
+    return GPUCAD_OK;
+}
+
+// Workspace of cg_solve.
+size_t cg_bytes(int m, int nx, int ny, int nz) {
+    const uint64_t n = (uint64_t)nx * ny * nz;
+    int cus = 0;
+    if (cg_cus(&cus)) cus = 0;
+    size_t bytes = cg_layout(n, m).bytes;
+    const ChipPlan p = chip_plan(nx, ny, nz, m, cus);
+    if (p.ty)
+        bytes = std::max<size_t>(bytes, ((m * n * sizeof(float) + 255) & ~uint64_t(255)) +
+                                            chip_layout(p, m).bytes);
+    return bytes;
+}
+
+// Solves A x = b for m right-hand sides (b: m vectors of n, x written over
+// b when x == b) in ws (cg_bytes).  On the chip when the grid fits there;
+// otherwise, or when that gave up waiting, iterations of two launches in
+// chunks between host checks of the done flags (a finished right-hand side
+// leaves the kernels at their first test).  x is complete in stream order.
+int cg_solve(const float *b, float *x, int m, int nx, int ny, int nz, int max_iter, float end_res,
+             int *iters, float *res, void *ws, hipStream_t st) {
+    const uint64_t n = (uint64_t)nx * ny * nz;
     CgState h[kMaxRhs];
-    for (int it0 = 0; it0 < max_iter; it0 += kChunk) {
-        for (int it = it0; it < std::min(max_iter, it0 + kChunk); ++it) {
-            hipLaunchKernelGGL(cg_a_kernel, grid, dim3(kCgThreads), 0, st, a, it);
-            hipLaunchKernelGGL(cg_b_kernel, grid, dim3(kCgThreads), 0, st, a, it);
-        }
+    int cus = 0;
+    int rc = cg_cus(&cus);
+    if (rc) return rc;
+    const ChipPlan chip = chip_plan(nx, ny, nz, m, cus);
+    bool solved = false;
+    if (chip.ty) {
+        rc = cg_chip_solve(chip, b, x, m, nx, ny, nz, max_iter, end_res, h, ws, &solved, st);
+        if (rc) return rc;
+    }
+    if (!solved) {
+        const CgLayout l = cg_layout(n, m);
+        CgArgs a;
+        a.nx = nx;
+        a.ny = ny;
+        a.nz = nz;
+        a.n = n;
+        a.dnx = make_div32((uint32_t)nx);
+        a.dplane = make_div32((uint32_t)nx * (uint32_t)ny);
+        a.G = l.G;
+        a.C = l.C;
+        a.max_iter = max_iter;
+        a.term = end_res * end_res;
+        char *w = (char *)ws;
+        a.phi = (float *)w;
+        a.r = (float *)(w + l.slot);
+        a.q = (float *)(w + 2 * l.slot);
+        a.d0 = (float *)(w + 3 * l.slot);
+        a.d1 = (float *)(w + 4 * l.slot);
+        a.pq = (double *)(w + 5 * l.slot);
+        a.prr = a.pq + (uint64_t)m * a.G;
+        a.st = (CgState *)(a.prr + 2 * (uint64_t)m * a.G);
+        const dim3 grid((unsigned)a.G, (unsigned)m);
+        hipLaunchKernelGGL(cg_init_kernel, grid, dim3(kCgThreads), 0, st, b, a);
         GC_CHECK_LAUNCH();
-        GC_HIP(hipMemcpyAsync(h, a.st, m * sizeof(CgState), hipMemcpyDeviceToHost, st));
-        GC_HIP(hipStreamSynchronize(st));
-        bool all = true;
-        for (int s = 0; s < m; ++s) all = all && h[s].done;
-        if (all) break;
+        constexpr int kChunk = 16;
+        for (int it0 = 0; it0 < max_iter; it0 += kChunk) {
+            for (int it = it0; it < std::min(max_iter, it0 + kChunk); ++it) {
+                hipLaunchKernelGGL(cg_a_kernel, grid, dim3(kCgThreads), 0, st, a, it);
+                hipLaunchKernelGGL(cg_b_kernel, grid, dim3(kCgThreads), 0, st, a, it);
+            }
+            GC_CHECK_LAUNCH();
+            GC_HIP(hipMemcpyAsync(h, a.st, m * sizeof(CgState), hipMemcpyDeviceToHost, st));
+            GC_HIP(hipStreamSynchronize(st));
+            bool all = true;
+            for (int s = 0; s < m; ++s) all = all && h[s].done;
+            if (all) break;
+        }
+        for (int s = 0; s < m; ++s)
+            if (!h[s].done)
+                return fail(GPUCAD_E_HIP, "internal: CG did not stop by iteration %d", max_iter);
+        GC_HIP(hipMemcpyAsync(x, a.phi, m * n * sizeof(float), hipMemcpyDeviceToDevice, st));
     }
     for (int s = 0; s < m; ++s) {
-        if (!h[s].done) return fail(GPUCAD_E_HIP, "internal: CG did not stop by iteration %d",
-                                    max_iter);
         if (iters) iters[s] = h[s].iters;
         if (res) res[s] = h[s].res;
     }
-    GC_HIP(hipMemcpyAsync(x, a.phi, vec, hipMemcpyDeviceToDevice, st));
-    GC_HIP(hipStreamSynchronize(st));
     return GPUCAD_OK;
 }
 
@@ -1017,8 +1626,11 @@ int gpucad_svl_cg(float *d_phi, int32_t nx, int32_t ny, int32_t nz, int32_t iter
     GC_ARG(iter >= 1, "iter must be >= 1");
     int it = 0;
     float res = 0.f;
-    st = cg_solve(d_phi, d_phi, 1, nx, ny, nz, iter, end_res, &it, &res, 0);
+    void *ws = nullptr;
+    if ((st = scratch_arena(cg_bytes(1, nx, ny, nz), &ws))) return st;
+    st = cg_solve(d_phi, d_phi, 1, nx, ny, nz, iter, end_res, &it, &res, ws, 0);
     if (st) return st;
+    GC_HIP(hipStreamSynchronize(0));
     if (final_iter) *final_iter = it;
     if (final_res) *final_res = res;
     return GPUCAD_OK;
@@ -1130,42 +1742,30 @@ int gpucad_svl_field(const gc_svl_params *p, const float *d_period, const gc_flo
     // the three unit right-hand sides, solved together; a harmonic's residual
     // is at most (|i| + |j| + |k|) times theirs, so they are solved to
     // cg_end_res / (3 range) to meet cg_end_res for every harmonic
+    const uint64_t vec = (3 * n * sizeof(float) + 255) & ~uint64_t(255);
     void *ws = nullptr;
-    const uint64_t vec = 3 * n * sizeof(float);
-    hipError_t he = hipMalloc(&ws, vec);
-    if (he != hipSuccess) return fail(GPUCAD_E_OOM, "svl: allocation of %llu bytes failed",
-                                      (unsigned long long)vec);
+    if ((st = scratch_arena(vec + cg_bytes(3, p->nx, p->ny, p->nz), &ws))) return st;
     float *phi = (float *)ws;
     const int unit[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
     for (int a = 0; a < 3; ++a) {
         hipLaunchKernelGGL(finding_phi_kernel, stride_grid(n), dim3(256), 0, s, phi + a * n,
                            d_period, phi_args(p, unit[a][0], unit[a][1], unit[a][2]));
+        GC_CHECK_LAUNCH();
     }
     int iters[3] = {0, 0, 0};
     float res[3] = {0.f, 0.f, 0.f};
-    he = hipGetLastError();
-    if (he == hipSuccess) {
-        const float tol = p->cg_end_res / (float)(3 * std::max(1, p->range));
-        st = cg_solve(phi, phi, 3, p->nx, p->ny, p->nz, p->cg_max_iter, tol, iters, res, s);
-    } else {
-        st = fail(GPUCAD_E_HIP, "svl: launch failed: %s", hipGetErrorString(he));
-    }
-    if (!st) {
-        const Up u = {p->nx, p->ny, p->nz, p->fx, p->fy, p->fz, p->fine_dx, p->fine_dy, p->fine_dz};
-        const uint64_t fn = (uint64_t)p->fx * p->fy * p->fz;
-        hipLaunchKernelGGL(svl_field_kernel, stride_grid(fn), dim3(256),
-                           (size_t)std::max(1, p->harmonics) * (sizeof(float2) + sizeof(int)), s,
-                           phi, phi + n,
-                           phi + 2 * n, u, (const float2 *)d_coeffs, p->range, p->harmonics, d_svl);
-        he = hipGetLastError();
-        if (he != hipSuccess) st = fail(GPUCAD_E_HIP, "svl: launch failed: %s", hipGetErrorString(he));
-        else {
-            he = hipStreamSynchronize(s);
-            if (he != hipSuccess) st = fail(GPUCAD_E_HIP, "svl: %s", hipGetErrorString(he));
-        }
-    }
-    (void)hipFree(ws);
+    const float tol = p->cg_end_res / (float)(3 * std::max(1, p->range));
+    st = cg_solve(phi, phi, 3, p->nx, p->ny, p->nz, p->cg_max_iter, tol, iters, res,
+                  (char *)ws + vec, s);
     if (st) return st;
+    const Up u = {p->nx, p->ny, p->nz, p->fx, p->fy, p->fz, p->fine_dx, p->fine_dy, p->fine_dz};
+    const uint64_t fn = (uint64_t)p->fx * p->fy * p->fz;
+    hipLaunchKernelGGL(svl_field_kernel, stride_grid(fn), dim3(256),
+                       (size_t)std::max(1, p->harmonics) * (sizeof(float2) + sizeof(int)), s, phi,
+                       phi + n, phi + 2 * n, u, (const float2 *)d_coeffs, p->range, p->harmonics,
+                       d_svl);
+    GC_CHECK_LAUNCH();
+    GC_HIP(hipStreamSynchronize(s));
     if (result) {
         for (int a = 0; a < 3; ++a) {
             result->cg_iters[a] = iters[a];
