@@ -173,7 +173,7 @@ BatchExtract make_batch_extract(const HostPlan &h, const DevPlan &d, const float
     b.nseg = (uint32_t)h.segs.size();
     b.nb = h.nb;
     b.base = d.base;
-    b.twave = d.twave;
+    b.live = d.live;
     b.bsum = d.bsum;
     b.ctl = d.ctl;
     b.res = d.res;
@@ -447,7 +447,7 @@ int batch_create(const gc_lattice_params *grids, int n, const gc_batch_options *
     const Part p_consts = part(n * sizeof(FieldConsts)), p_segs = part(n * sizeof(Seg)),
                p_b2s = part(nb * 4), p_res = part(n * sizeof(SegResult)),
                p_base = part(nb * kBaseBytesPerBlock),
-               p_twave = part(nb * kTwaveBytesPerBlock), p_bsum = part(nb * 16),
+               p_live = part(nb * kLiveBytesPerBlock), p_bsum = part(nb * 16),
                p_ctl = part(64), p_fields = part(fo * 4),
                p_signs = part(so * 8);
     hipError_t he = hipMalloc(&b->arena, off);
@@ -462,7 +462,7 @@ int batch_create(const gc_lattice_params *grids, int n, const gc_batch_options *
     b->d.blk2seg = (uint32_t *)(A + p_b2s.off);
     b->d.res = (SegResult *)(A + p_res.off);
     b->d.base = (uint32_t *)(A + p_base.off);
-    b->d.twave = (uint32_t *)(A + p_twave.off);
+    b->d.live = (uint32_t *)(A + p_live.off);
     b->d.bsum = (uint64_t *)(A + p_bsum.off);
     b->d.ctl = (uint64_t *)(A + p_ctl.off);
     b->fields = (float *)(A + p_fields.off);

@@ -54,10 +54,10 @@ int device_tables(const DeviceTables **out) {
     DeviceState &ds = g_dev[dev];
     if (!ds.tables_ready) {
         DeviceTables t;
-        GC_HIP(hipMalloc(&t.tri_packed, 256 * sizeof(uint64_t)));
+        GC_HIP(hipMalloc(&t.emit, 5 * 256 * sizeof(uint32_t)));
         GC_HIP(hipMalloc(&t.num_verts, 256));
         GC_HIP(hipMalloc(&t.tri_table, 256 * 16));
-        GC_HIP(hipMemcpy(t.tri_packed, host_tri_packed(), 256 * sizeof(uint64_t),
+        GC_HIP(hipMemcpy(t.emit, host_emit_table(), 5 * 256 * sizeof(uint32_t),
                          hipMemcpyHostToDevice));
         GC_HIP(hipMemcpy(t.num_verts, host_num_verts(), 256, hipMemcpyHostToDevice));
         GC_HIP(hipMemcpy(t.tri_table, host_tri_table(), 256 * 16, hipMemcpyHostToDevice));
@@ -197,7 +197,7 @@ int gpucad_shutdown(void) {
     gc::DeviceState &ds = gc::g_dev[dev];
     GC_HIP(hipDeviceSynchronize());
     if (ds.tables_ready) {
-        GC_HIP(hipFree(ds.tables.tri_packed));
+        GC_HIP(hipFree(ds.tables.emit));
         GC_HIP(hipFree(ds.tables.num_verts));
         GC_HIP(hipFree(ds.tables.tri_table));
         ds.tables = gc::DeviceTables();

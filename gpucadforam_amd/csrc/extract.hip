@@ -10,48 +10,37 @@
 //
 // The grid is seen through its sign words: bit b of word w of row r = y+ny*z
 // is [f(64w+b, y, z) < iso].  A word (k = r*W + w) is the unit of
-// bookkeeping: the lane that owns it derives the crossing edges of its 64
-// points and the active cells of its 64 cells with 64-bit bit arithmetic.
-// Work on active cells is balanced by compacting them, per wave, into an LDS
-// list in canonical order and running one lane per active cell; a lane reads
-// the word-level data of its cell from the owning lane (ds_bpermute).
+// bookkeeping: the lane that owns it (or half of it) derives the crossing
+// edges of its points and the active cells with bit arithmetic.
 //
 // Launches (one stream, no host round trip, no inter-block waits):
 //   signs : ballot of f < iso per 64 points; skipped when the field kernel
 //           already produced the words
-//   count : blocks of 256 words: triangles per wave (case of each active
-//           cell), vertex and triangle sums per block, and each half word's
-//           first vertex number within its block
+//   count : blocks of 256 words: vertex and triangle sums per block, each
+//           word's first vertices and first triangle within its block, and
+//           which groups of 8 words have something to emit
 //   scan  : one workgroup scans the block sums (64-bit), writes the totals
-//           and the vertex/triangle range of each grid
-//   emit  : the vertex and triangle stages in one launch, their workgroups
-//           interleaved (both depend only on count and scan):
-//     vert: each wave compacts its 64 words' crossing edges into an LDS list
-//           in canonical order and emits them one lane per edge (loads of f0
-//           and f1, interpolation); a wave's vertices form one contiguous
-//           range, stored coalesced
-//     tri : one lane per active cell computes the 12 edge vertex numbers from
-//           popcounts of the crossing words of the four rows touching the cell
-//           (plus the rows' first vertex numbers) and writes its triangles; a
-//           wave's triangles form one contiguous range starting at the wave's
-//           scanned base
+//           and the vertex/triangle range of each grid; one grid of few
+//           blocks needs no such launch, its emission sums them itself
+//   emit  : a wave takes 8, 16 or 32 consecutive words, lists their cells (and
+//           the points with an edge but no cell) in canonical order and runs
+//           one lane per list entry: the 12 edge vertex numbers from popcounts
+//           of the crossings of the four rows touching the cell, its triangles
+//           and its own edges; then one lane per edge and one per triangle.
+//           A wave's vertices and triangles are contiguous ranges whose starts
+//           follow from count and scan.
 //
 // The kernels see grids as segments: a grid's words occupy a contiguous range
-// of global blocks.  Every launch runs one workgroup per block (three per
-// block for emit: its vertices and its two triangle halves); the many-grid
-// form (batched and served) finds each block's grid in a block -> grid table.
-// Both run the same block code, so a grid's mesh does not depend on what it
-// is launched with.
+// of global blocks; the many-grid form (batched and served) finds each block's
+// grid in a block -> grid table.  Both run the same code, so a grid's mesh
+// does not depend on what it is launched with.
 #include "extract_types.hpp"
 
 namespace gc {
 namespace {
 
-constexpr int kWaveVertCap = 1024; // per-wave LDS edge-list entries per round
-constexpr int kEdgeStep = 4;   // edges per thread and step of the vertex emission
-
 struct ExtractLayout {
-    uint64_t signs_off, base_off, twave_off, bsum_off, ctl_off, res_off, bytes;
+    uint64_t signs_off, base_off, live_off, bsum_off, ctl_off, res_off, bytes;
     uint64_t words, nb;
 };
 
@@ -66,8 +55,8 @@ ExtractLayout layout(int nx, int ny, int nz) {
     off = align256(off + L.words * 8);
     L.base_off = off;
     off = align256(off + L.nb * kBaseBytesPerBlock);
-    L.twave_off = off;
-    off = align256(off + L.nb * kTwaveBytesPerBlock);
+    L.live_off = off;
+    off = align256(off + L.nb * kLiveBytesPerBlock);
     L.bsum_off = off;
     off = align256(off + L.nb * 16);
     L.ctl_off = off;  // [0] n_vertices [1] n_triangles [2] vertex numbers overflow 32 bits
@@ -88,13 +77,6 @@ __device__ __forceinline__ uint64_t mask_below(int64_t n) {
     if (n <= 0) return 0ull;
     return (1ull << n) - 1ull;
 }
-__device__ __forceinline__ uint32_t bit_at(uint64_t w, uint32_t b) {
-    return (uint32_t)(w >> b) & 1u;
-}
-__device__ __forceinline__ uint32_t lane_id() {
-    return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-}
-
 __device__ __forceinline__ uint32_t gather32(uint32_t v, uint32_t src) {
     return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(src << 2), (int)v);
 }
@@ -137,11 +119,8 @@ __device__ __forceinline__ void store_nt(uint32_t *p, T3 t) {
 }
 
 __device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv &f) {
-    uint32_t q = (uint32_t)((double)n * f.inv);
-    const int64_t r = (int64_t)n - (int64_t)q * f.d;
-    if (r < 0) --q;
-    else if (r >= (int64_t)f.d) ++q;
-    return q;
+    const uint32_t q = __umulhi(n, f.m);  // n / d or one less
+    return q + (n - q * f.d >= f.d ? 1u : 0u);
 }
 
 // sign word `idx` of a grid (32-bit word index: a grid has fewer than 2^32
@@ -164,26 +143,6 @@ __device__ __forceinline__ WordPos word_pos(uint64_t k, const Grid &g) {
     p.z = (int)z;
     p.y = (int)(r - z * (uint32_t)g.ny);
     return p;
-}
-
-struct Cross {
-    uint64_t ex, ey, ez, sx, sy;
-};
-
-// Crossing words of the row with words (cur, nxt), +y neighbour (py, pyn) and
-// +z neighbour pz; sx/sy: the same for point b+1.
-__device__ __forceinline__ Cross row_cross(uint64_t cur, uint64_t nxt, uint64_t py, uint64_t pyn,
-                                           uint64_t pz, bool has_y, bool has_z, uint64_t ved,
-                                           uint64_t vpt, bool ved_n, bool vpt_n) {
-    Cross c;
-    c.ex = (cur ^ shift1(cur, nxt)) & ved;
-    c.ey = has_y ? (cur ^ py) & vpt : 0ull;
-    c.ez = has_z ? (cur ^ pz) & vpt : 0ull;
-    const uint64_t exn = ved_n ? ((nxt ^ (nxt >> 1)) & 1ull) : 0ull;
-    const uint64_t eyn = (has_y && vpt_n) ? ((nxt ^ pyn) & 1ull) : 0ull;
-    c.sx = shift1(c.ex, exn);
-    c.sy = shift1(c.ey, eyn);
-    return c;
 }
 
 // ---------------------------------------------------------------------------
@@ -269,9 +228,11 @@ __device__ __forceinline__ uint32_t word_triangles(uint64_t k0, uint64_t k1, uin
 
 struct CountArgs {
     const uint64_t *signs;  // sign buffer base
-    uint32_t *twave;
+    uint32_t *live;         // per block: bit i: its words 8i .. 8i + 7 have something to emit
     uint64_t *bsum;
-    uint32_t *base;  // block-local first vertex of each half word
+    // per word: first vertex of its two half words (16 bits each) and its
+    // first triangle, within the block (at most 49152 and 81920)
+    uint2 *base;
 };
 
 template <class Src>
@@ -320,20 +281,22 @@ __global__ void __launch_bounds__(kBlock) count_kernel(Src src, CountArgs a) {
         const uint32_t vincl = wave_scan_incl(vc);
         const uint32_t vw = readlane32(vincl, 63);
         const uint32_t tincl = wave_scan_incl(tc);
-        const uint32_t tlo = readlane32(tincl, 31), tw = readlane32(tincl, 63);
+        const uint32_t tw = readlane32(tincl, 63);
+        const uint64_t used = __ballot((vc | tc) != 0);
+        const uint64_t eights = __ballot(lane < 8 && ((used >> 8 * (lane & 7)) & 0xffu) != 0);
         if (lane == 0) {
             s_sum[wave][0] = vw;
             s_sum[wave][1] = tw;
-            // triangle counts of the wave's two groups of 32 words
-            a.twave[kGroups * (uint64_t)gb + 2 * wave] = tlo;
-            a.twave[kGroups * (uint64_t)gb + 2 * wave + 1] = tw - tlo;
+            ((uint8_t *)a.live)[4 * (uint64_t)gb + wave] = (uint8_t)eights;
         }
         __syncthreads();
         if (k < g.words) {
-            // the word's first vertex within the block, for each 32-point half
-            uint32_t v0 = vincl - vc;
-            for (uint32_t i = 0; i < 4; ++i) v0 += i < wave ? s_sum[i][0] : 0u;
-            *(uint2 *)(a.base + 2 * ((uint64_t)gb * kBlock + tid)) = make_uint2(v0, v0 + vlo);
+            uint32_t v0 = vincl - vc, t0 = tincl - tc;
+            for (uint32_t i = 0; i < 4; ++i) {
+                v0 += i < wave ? s_sum[i][0] : 0u;
+                t0 += i < wave ? s_sum[i][1] : 0u;
+            }
+            a.base[(uint64_t)gb * kBlock + tid] = make_uint2(v0 | (v0 + vlo) << 16, t0);
         }
         if (tid == 0) {
             a.bsum[2 * (uint64_t)gb] =
@@ -454,495 +417,505 @@ scan_blocks_kernel(uint64_t *bsum, uint64_t nb, uint64_t *ctl, uint64_t *d_count
 }
 
 // ---------------------------------------------------------------------------
-// vertices (+ per-word first vertex numbers)
+// emit: vertices and triangles
 // ---------------------------------------------------------------------------
-// vertex on the edge from point (xf, yf, zf) along axis ax with end values f0, f1:
-// t = (iso - f0)/(f1 - f0), p = fma(t, p1 - p0, p0) on that axis
-__device__ __forceinline__ V3 edge_vertex(const Seg &s, float xf, float yf, float zf, uint32_t ax,
+// Vertex on the edge from point (xf, yf, zf) along axis ax with end values f0,
+// f1: t = (iso - f0)/(f1 - f0), p = fma(t, p1 - p0, p0) on that axis.  The
+// three axes are interpolated and the edge's own one is kept (lanes of a wave
+// hold edges of all three): selects cost twice an FMA.
+struct Frame {
+    float iso, ox, oy, oz, sx, sy, sz;
+};
+__device__ __forceinline__ V3 edge_vertex(const Frame &s, float xf, float yf, float zf, uint32_t ax,
                                           float f0, float f1) {
     const float t = (s.iso - f0) / (f1 - f0);
     const float px = __builtin_fmaf(xf, s.sx, s.ox);
     const float py = __builtin_fmaf(yf, s.sy, s.oy);
     const float pz = __builtin_fmaf(zf, s.sz, s.oz);
-    // the edge's axis by selects (lanes of a wave hold edges of all three
-    // axes): its low end p0, its high end p1, and p0 + t (p1 - p0) on it
-    const float c = ax == 0 ? xf : (ax == 1 ? yf : zf);
-    const float sc = ax == 0 ? s.sx : (ax == 1 ? s.sy : s.sz);
-    const float oc = ax == 0 ? s.ox : (ax == 1 ? s.oy : s.oz);
-    const float p0 = ax == 0 ? px : (ax == 1 ? py : pz);
-    const float p1 = __builtin_fmaf(c + 1.0f, sc, oc);
-    const float pe = __builtin_fmaf(t, p1 - p0, p0);
-    return V3{ax == 0 ? pe : px, ax == 1 ? pe : py, ax == 2 ? pe : pz};
+    const float ex = __builtin_fmaf(t, __builtin_fmaf(xf + 1.0f, s.sx, s.ox) - px, px);
+    const float ey = __builtin_fmaf(t, __builtin_fmaf(yf + 1.0f, s.sy, s.oy) - py, py);
+    const float ez = __builtin_fmaf(t, __builtin_fmaf(zf + 1.0f, s.sz, s.oz) - pz, pz);
+    return V3{ax == 0 ? ex : px, ax == 1 ? ey : py, ax == 2 ? ez : pz};
 }
 
-struct VertArgs {
+constexpr int kEmitWaves = 4;          // waves per workgroup
+constexpr int kCellCap = 512;          // cells of a wave listed at a time
+constexpr int kRing = 256;             // edges waiting: at most 63 + a step's 192
+constexpr int kIdStride = kEmitStride; // vertex numbers of an edge: 64 cells + 1 (banks)
+// One grid of up to this many blocks needs no scan launch: every workgroup of
+// the emission sums the counts (two per thread).  203 x 149 x 181, 422 blocks:
+// 42.5 us for scan and emission (4.9 of them the scan, and its launch), 35.6 so.
+constexpr int kSelfBlocks = 512;
+
+struct EmitArgs {
     const float *field;     // field buffer base
     const uint64_t *signs;  // sign buffer base
-    const uint64_t *bsum;   // scanned block bases
+    const uint2 *base;      // per word: block-local numbers (count_kernel)
+    const uint32_t *live;   // per block: groups with something to emit
+    const uint64_t *bsum;   // first vertex and triangle of each block (kSelf: their counts)
     const SegResult *res;
+    const uint32_t *table;  // 5 x 256 triangle words (host_emit_table)
     float *vertices;
     uint64_t vcap;
-};
-
-// The vertex stage's LDS: one edge list per wave (a wave fills and emits its
-// own 64 words' edges, with no wait on the block's other waves).
-struct VertShared {
-    uint16_t list[kBlock / 64][kWaveVertCap + 64];  // + one discard slot per lane
-    uint64_t p0[kBlock];   // linear index of the word's first point
-    uint32_t xyz[kBlock];  // first x | y << 16
-    uint32_t z[kBlock];
-    uint32_t wsum[4];
-};
-
-// Vertices of count block gb.
-template <class Src>
-__device__ __forceinline__ void vert_block(const Src &src, const VertArgs &a, uint32_t gb,
-                                           VertShared &sh) {
-    uint64_t *s_p0 = sh.p0;
-    uint32_t *s_xyz = sh.xyz, *s_z = sh.z, *s_wsum = sh.wsum;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    {
-        const uint32_t si = src.seg_of(gb);
-        const Seg s = src.get(si);
-        const Grid &g = s.g;
-        const uint64_t *signs = a.signs + s.sign_off;
-        const uint64_t k = (uint64_t)(gb - s.block_off) * kBlock + tid;
-        // block base and grid range first: their loads overlap the sign loads
-        const uint64_t vblock = a.bsum[2 * (uint64_t)gb];
-        const uint32_t ovf = a.res[si].ovf;
-        uint64_t ex = 0, ey = 0, ez = 0;
-        if (k < g.words) {
-            const WordPos p = word_pos(k, g);
-            const bool has_y = p.y + 1 < g.ny, has_z = p.z + 1 < g.nz;
-            const uint32_t kk = (uint32_t)k, W = (uint32_t)g.W, RW = (uint32_t)g.ny * W;
-            // every load before any use (one round trip)
-            const uint64_t w0 = signs[kk], w0n = ldw(signs, kk + 1, p.w + 1 < g.W);
-            const uint64_t wy = ldw(signs, kk + W, has_y), wz = ldw(signs, kk + RW, has_z);
-            const uint64_t vpt = mask_below((int64_t)g.nx - 64 * p.w);
-            const uint64_t ved = mask_below((int64_t)g.nx - 1 - 64 * p.w);
-            ex = (w0 ^ shift1(w0, w0n)) & ved;
-            ey = has_y ? (w0 ^ wy) & vpt : 0ull;
-            ez = has_z ? (w0 ^ wz) & vpt : 0ull;
-            s_p0[tid] = ((uint64_t)p.z * g.ny + p.y) * g.nx + 64 * (uint64_t)p.w;
-            s_xyz[tid] = (uint32_t)(64 * p.w) | ((uint32_t)p.y << 16);
-            s_z[tid] = (uint32_t)p.z;
-        }
-        const uint32_t vc = popc64(ex) + popc64(ey) + popc64(ez);
-        const uint32_t incl = wave_scan_incl(vc);
-        const uint32_t wtot = readlane32(incl, 63);
-        if (lane == 63) s_wsum[wave] = incl;
-        __syncthreads();
-        uint32_t wbase = 0;
-        for (uint32_t i = 0; i < 4; ++i)
-            if (i < wave) wbase += s_wsum[i];
-        const uint32_t vexw = incl - vc;  // first vertex of this word within the wave
-        if (ovf) return;  // vertex numbers do not fit 32 bits: nothing is written
-        const float *field = a.field + s.field_off;
-        const uint64_t plane = (uint64_t)g.nx * g.ny;
-        uint16_t *list = sh.list[wave];
-        const uint64_t vwave = vblock + wbase;  // the wave's first vertex
-        for (uint32_t r0 = 0; r0 < wtot; r0 += kWaveVertCap) {
-            // this lane's edges, canonical order, that fall into the round's window
-            if (wtot <= kWaveVertCap) {
-                // one round holds the wave: no window tests, 32-bit halves;
-                // an edge a point lacks goes to the lane's discard slot
-                uint16_t *dump = list + kWaveVertCap + lane;
-                uint32_t i = vexw;
-#pragma unroll
-                for (uint32_t h = 0; h < 2; ++h) {
-                    const uint32_t hx = (uint32_t)(ex >> (32 * h));
-                    const uint32_t hy = (uint32_t)(ey >> (32 * h));
-                    const uint32_t hz = (uint32_t)(ez >> (32 * h));
-                    uint32_t pts = hx | hy | hz;
-                    while (pts) {
-                        const uint32_t b = (uint32_t)__builtin_ctz(pts);
-                        pts &= pts - 1;
-                        const uint32_t ent = (tid << 8) | ((b + 32 * h) << 2);
-                        const uint32_t bx = (hx >> b) & 1u, by = (hy >> b) & 1u, bz = (hz >> b) & 1u;
-                        *(bx ? list + i : dump) = (uint16_t)ent;
-                        i += bx;
-                        *(by ? list + i : dump) = (uint16_t)(ent | 1u);
-                        i += by;
-                        *(bz ? list + i : dump) = (uint16_t)(ent | 2u);
-                        i += bz;
-                    }
-                }
-            } else if (vc && vexw < r0 + kWaveVertCap && vexw + vc > r0) {
-                uint64_t pts = ex | ey | ez;
-                uint32_t i = vexw;
-                while (pts) {
-                    const uint32_t b = (uint32_t)__builtin_ctzll(pts);
-                    pts &= pts - 1;
-                    const uint32_t m =
-                        bit_at(ex, b) | (bit_at(ey, b) << 1) | (bit_at(ez, b) << 2);
-#pragma unroll
-                    for (uint32_t ax = 0; ax < 3; ++ax) {
-                        if (!((m >> ax) & 1)) continue;
-                        if (i >= r0 && i < r0 + kWaveVertCap)
-                            list[i - r0] = (uint16_t)((tid << 8) | (b << 2) | ax);
-                        ++i;
-                    }
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            const uint32_t n = min((uint32_t)kWaveVertCap, wtot - r0);
-            // kEdgeStep edges per lane and step, so that all their field
-            // loads are in flight before the first interpolation
-            for (uint32_t e0 = lane; e0 < n; e0 += kEdgeStep * 64) {
-                uint32_t ent[kEdgeStep];
-                float f0[kEdgeStep], f1[kEdgeStep];
-#pragma unroll
-                for (int q = 0; q < kEdgeStep; ++q) {
-                    const uint32_t e = e0 + q * 64;
-                    ent[q] = list[e < n ? e : e0];
-                    const uint32_t j = ent[q] >> 8, b = (ent[q] >> 2) & 63, ax = ent[q] & 3;
-                    const uint64_t pt = s_p0[j] + b;
-                    const uint64_t st = ax == 0 ? 1ull : (ax == 1 ? (uint64_t)g.nx : plane);
-                    f0[q] = field[pt];
-                    f1[q] = field[pt + st];
-                }
-#pragma unroll
-                for (int q = 0; q < kEdgeStep; ++q) {
-                    const uint32_t e = e0 + q * 64;
-                    const uint32_t j = ent[q] >> 8, b = (ent[q] >> 2) & 63, ax = ent[q] & 3;
-                    const uint32_t xy = s_xyz[j];
-                    const V3 v = edge_vertex(s, (float)((xy & 0xffff) + b), (float)(xy >> 16),
-                                             (float)s_z[j], ax, f0[q], f1[q]);
-                    const uint64_t id = vwave + r0 + e;
-                    if (e < n && id < a.vcap) store_nt(a.vertices + 3 * id, v);
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// triangles
-// ---------------------------------------------------------------------------
-// One thread per half word: 32 points of a row, bit b of half h of word w is
-// point 64w + 32h + b, and the sign buffer is read as 32-bit halves.  A
-// triangle block is half of a count block: 128 words, 4 waves of 32 words,
-// each wave one of the count stage's triangle groups.  32-bit halves halve
-// the gathers and the bit work per cell and the per-thread state.
-constexpr int kTriThreads = kBlock;
-constexpr int kTriWords = kTriThreads / 2;  // words per triangle block
-constexpr int kCellCap = 256;  // per-wave LDS cell-list entries per round
-
-__device__ __forceinline__ uint32_t sh1(uint32_t cur, uint32_t next) {
-    return (cur >> 1) | (next << 31);
-}
-// bits [0, n) of a 32-bit half
-__device__ __forceinline__ uint32_t below32(int64_t n) {
-    return n <= 0 ? 0u : (n >= 32 ? ~0u : (1u << n) - 1u);
-}
-// half `idx` when `ok`, else 0; unconditional load as ldw
-__device__ __forceinline__ uint32_t ldh(const uint32_t *s, uint32_t idx, bool ok) {
-    const uint32_t v = s[ok ? idx : 0u];
-    return ok ? v : 0u;
-}
-__device__ __forceinline__ uint32_t bit32(uint32_t w, uint32_t b) { return (w >> b) & 1u; }
-
-struct Cross32 {
-    uint32_t ex, ey, ez, sx, sy;
-};
-
-// Crossing bits of the row half with signs (cur, nxt = next half), +y
-// neighbour (py, pyn) and +z neighbour pz; sx/sy: the same for point b+1.
-__device__ __forceinline__ Cross32 row_cross32(uint32_t cur, uint32_t nxt, uint32_t py,
-                                               uint32_t pyn, uint32_t pz, bool has_y, bool has_z,
-                                               uint32_t ved, uint32_t vpt, bool ved_n,
-                                               bool vpt_n) {
-    Cross32 c;
-    c.ex = (cur ^ sh1(cur, nxt)) & ved;
-    c.ey = has_y ? (cur ^ py) & vpt : 0u;
-    c.ez = has_z ? (cur ^ pz) & vpt : 0u;
-    const uint32_t exn = ved_n ? ((nxt ^ (nxt >> 1)) & 1u) : 0u;
-    const uint32_t eyn = (has_y && vpt_n) ? ((nxt ^ pyn) & 1u) : 0u;
-    c.sx = sh1(c.ex, exn);
-    c.sy = sh1(c.ey, eyn);
-    return c;
-}
-
-// Fills the calling wave's LDS list with its active cells of entries
-// [r0, r0 + kCellCap) of the canonical order (lane | x << 6).
-__device__ __forceinline__ void fill_cells(uint16_t *list, uint32_t act, uint32_t nact,
-                                           uint32_t aex, uint32_t atot, uint32_t r0,
-                                           uint32_t lane) {
-    if (atot <= kCellCap) {
-        uint32_t i = aex;
-        uint32_t m = act;
-        while (m) {
-            const uint32_t x = (uint32_t)__builtin_ctz(m);
-            m &= m - 1;
-            list[i++] = (uint16_t)(lane | (x << 6));
-        }
-    } else if (nact && aex < r0 + kCellCap && aex + nact > r0) {
-        uint32_t m = act;
-        uint32_t i = aex;
-        while (m) {
-            const uint32_t x = (uint32_t)__builtin_ctz(m);
-            m &= m - 1;
-            if (i >= r0 && i < r0 + kCellCap) list[i - r0] = (uint16_t)(lane | (x << 6));
-            ++i;
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-}
-
-struct TriArgs {
-    const uint64_t *signs;  // sign buffer base
-    const uint32_t *base;   // block-local first vertex number of each half word
-    const uint32_t *twave;  // triangles of each group of 32 words
-    const uint64_t *bsum;
-    const uint64_t *tri_packed;
-    const SegResult *res;
     uint32_t *triangles;
     uint64_t tcap;
+    uint32_t lw;            // log2 of the words per wave: 3, 4 or 5
+    uint32_t nb;            // kSelf: blocks of the grid
+    uint64_t *ctl, *d_counts;  // kSelf: written by the first workgroup
 };
 
-// The triangle stage's LDS.
-struct TriShared {
-    static constexpr int kWaves = kTriThreads / 64;
-    uint64_t tri[256];
-    uint16_t list[kWaves][kCellCap];
-    uint32_t vid[kWaves][12 * 64];  // id k of lane l at k*64 + (l ^ k)
-    // triangle -> lane | its three edges (4 bits each) << 8
-    uint32_t own[kWaves][5 * 64];
+struct EmitWave {
+    uint32_t vid[12 * kIdStride];  // vertex number of edge e of cell l at e * kIdStride + l
+    uint32_t own[5 * 64 + 8];      // a step's triangles: byte offsets of their three numbers
+    uint16_t list[kCellCap];       // cells: owner lane * 4 | x << 8
+    uint16_t ring[kRing];          // edges: the cell's entry | axis
 };
 
-// Triangles of triangle block tb (half tb & 1 of count block tb >> 1).
-template <class Src>
-__device__ __forceinline__ void tri_block(const Src &src, const TriArgs &a, uint32_t tb,
-                                          TriShared &sh) {
-    static_assert(kTriThreads == 256, "one case-table entry per thread");
-    uint64_t *s_tri = sh.tri;
-    // the case table's entry is loaded first and stored to LDS after the
-    // sign loads below have returned: both share one round trip
-    const uint64_t tri_entry = a.tri_packed[threadIdx.x];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = tid & 1;
-    {
-        const uint32_t gb = tb >> 1, part = tb & 1;  // count block and its half
-        const uint32_t si = src.seg_of(gb);
-        // the block's bookkeeping, loaded with no branch on it so that its
-        // round trip is shared with the sign loads': the grid's overflow
-        // flag, the block's first triangle and its 8 group counts
-        const uint32_t ovf = a.res[si].ovf;
-        const uint64_t v_off = a.res[si].v_off;
-        const uint64_t tblock = a.bsum[2 * (uint64_t)gb + 1];
-        const uint4 ga = *(const uint4 *)(a.twave + kGroups * (uint64_t)gb);
-        const uint4 gc4 = *(const uint4 *)(a.twave + kGroups * (uint64_t)gb + 4);
-        const Seg s = src.get(si);
-        const Grid &g = s.g;
-        const uint32_t *signs = (const uint32_t *)(a.signs + s.sign_off);
-        const uint64_t k = (uint64_t)(gb - s.block_off) * kBlock + part * kTriWords + (tid >> 1);
-        const uint32_t *base = a.base + (uint64_t)s.block_off * kBlock * 2;  // by grid half word
-        const uint64_t *gbsum = a.bsum + 2 * (uint64_t)s.block_off;       // by grid block
-        // ---- per half word (owner lane): the sign half of row (y, z) and the
-        // crossing halves of the four rows (y..y+1, z..z+1) touching its
-        // cells; a cell's cube index and edge vertex numbers follow from these
-        // bits (sign of a neighbour corner = own sign ^ crossing of the edge
-        // between)
-        uint32_t wa = 0, act = 0;
-        uint32_t ex0 = 0, ey0 = 0, ez0 = 0, ex1 = 0, ey1 = 0, ez1 = 0;
-        uint32_t ex2 = 0, ey2 = 0, ez2 = 0, ex3 = 0, ey3 = 0, ez3 = 0;
-        uint32_t carry = 0;  // crossing bits of point 32 (next half): x0 y0 x1 y1 x2
-        uint32_t vb0 = 0, vb1 = 0, vb2 = 0, vb3 = 0;
-        if (k < g.words) {
-            const WordPos p = word_pos(k, g);
-            const int xh = 64 * p.w + 32 * (int)h;  // first point of the half
-            const uint32_t ved = below32((int64_t)g.nx - 1 - xh);
-            if (p.y + 1 < g.ny && p.z + 1 < g.nz && ved) {
-                const bool has_y2 = p.y + 2 < g.ny, has_z2 = p.z + 2 < g.nz;
-                const uint32_t W2 = 2u * (uint32_t)g.W, RW2 = (uint32_t)g.ny * W2;
-                const uint32_t i0 = 2u * (uint32_t)k + h;
-                const bool hn = h == 0 || p.w + 1 < g.W;  // the row has a next half
-                // every load of the half at once (one round trip); a half
-                // without active cells discards them
-                wa = signs[i0];
-                const uint32_t na = ldh(signs, i0 + 1, hn);
-                const uint32_t wb = signs[i0 + W2];
-                const uint32_t nb = ldh(signs, i0 + W2 + 1, hn);
-                const uint32_t wc = signs[i0 + RW2];
-                const uint32_t nc = ldh(signs, i0 + RW2 + 1, hn);
-                const uint32_t wd = signs[i0 + RW2 + W2];
-                const uint32_t nd = ldh(signs, i0 + RW2 + W2 + 1, hn);
-                const uint32_t we = ldh(signs, i0 + 2 * W2, has_y2),
-                               ne = ldh(signs, i0 + 2 * W2 + 1, has_y2 && hn);
-                const uint32_t wf = ldh(signs, i0 + 2 * W2 + RW2, has_y2);
-                const uint32_t wg = ldh(signs, i0 + 2 * RW2, has_z2);
-                const uint32_t wh = ldh(signs, i0 + 2 * RW2 + W2, has_z2);
-                // the first vertex ids (block-local, plus the first vertex
-                // of the block holding the row's word) are needed only by
-                // halves with active cells, but are loaded (and kept)
-                // unconditionally so that they share the sign loads' round trip
-                static_assert(kBlock == 256, "a word's block is its index >> 8");
-                const uint32_t kw = (uint32_t)k, Wd = (uint32_t)g.W, RWd = (uint32_t)g.ny * Wd;
-                vb0 = base[i0] + (uint32_t)(gbsum[2 * (kw >> 8)] - v_off);
-                vb1 = base[i0 + W2] + (uint32_t)(gbsum[2 * ((kw + Wd) >> 8)] - v_off);
-                vb2 = base[i0 + RW2] + (uint32_t)(gbsum[2 * ((kw + RWd) >> 8)] - v_off);
-                vb3 = base[i0 + RW2 + W2] + (uint32_t)(gbsum[2 * ((kw + RWd + Wd) >> 8)] - v_off);
-                const uint32_t sa = sh1(wa, na), sb = sh1(wb, nb), sc = sh1(wc, nc),
-                               sd = sh1(wd, nd);
-                act = ((wa ^ sa) | (wa ^ wb) | (wa ^ sb) | (wa ^ wc) | (wa ^ sc) | (wa ^ wd) |
-                       (wa ^ sd)) & ved;
-                if (act) {
-                    const uint32_t vpt = below32((int64_t)g.nx - xh);
-                    const bool vpt_n = xh + 32 < g.nx, ved_n = xh + 32 < g.nx - 1;
-                    const Cross32 c0 = row_cross32(wa, na, wb, nb, wc, true, true, ved, vpt, ved_n, vpt_n);
-                    const Cross32 c1 = row_cross32(wb, nb, we, ne, wd, has_y2, true, ved, vpt, ved_n, vpt_n);
-                    const Cross32 c2 = row_cross32(wc, nc, wd, nd, wg, true, has_z2, ved, vpt, ved_n, vpt_n);
-                    const Cross32 c3 = row_cross32(wd, nd, wf, 0u, wh, has_y2, has_z2, ved, vpt, ved_n, vpt_n);
-                    ex0 = c0.ex; ey0 = c0.ey; ez0 = c0.ez;
-                    ex1 = c1.ex; ey1 = c1.ey; ez1 = c1.ez;
-                    ex2 = c2.ex; ey2 = c2.ey; ez2 = c2.ez;
-                    ex3 = c3.ex; ey3 = c3.ey; ez3 = c3.ez;
-                    carry = (c0.sx >> 31) | ((c0.sy >> 31) << 1) | ((c1.sx >> 31) << 2) |
-                            ((c1.sy >> 31) << 3) | ((c2.sx >> 31) << 4);
-                }
-            }
-        }
-        s_tri[tid] = tri_entry;
-        __syncthreads();
-        // vertex numbers that do not fit 32 bits: the grid's triangles are
-        // not written
-        const uint64_t tcap = ovf ? 0ull : a.tcap;
-        // the wave's first triangle follows the part * 4 + wave groups before it
-        static_assert(kGroups == 8, "two uint4 loads carry a block's group counts");
-        const uint32_t ng = part * 4 + wave;
-        const uint32_t gcount[kGroups] = {ga.x, ga.y, ga.z, ga.w, gc4.x, gc4.y, gc4.z, gc4.w};
-        uint64_t tnext = tblock;
+template <bool kSelf>
+struct EmitShared {
+    EmitWave w[kEmitWaves];
+    uint64_t stride[3];  // bytes from a point to the next one along an axis
+    uint32_t tab[5 * 256];  // words 0 and 1 in pairs, 2 and 3 in pairs, 4
+    uint32_t pre[kSelf ? kSelfBlocks : 1];  // first vertex of each block
+    uint2 sum[kSelf ? kEmitWaves : 1];      // the sums, wave by wave
+    uint32_t first_tri;                     // first triangle of this block
+};
+
+// a wave's LDS accesses are in order: this only keeps the compiler from
+// moving them across
+__device__ __forceinline__ void wave_sync() { __builtin_amdgcn_wave_barrier(); }
+// keeps a lane's LDS stores in program order, unmerged
+__device__ __forceinline__ void in_order() { asm volatile("" ::: "memory"); }
+
+__device__ __forceinline__ uint32_t below32(int n) {
+    return n <= 0 ? 0u : (n >= 32 ? ~0u : (1u << n) - 1u);
+}
+__device__ __forceinline__ uint32_t load_u32(const void *base, uint32_t off) {
+    return *(const uint32_t *)((const char *)base + off);
+}
+
+// Records of 12 bytes by which p lies past a 128-byte line boundary, modulo
+// the 32 of three lines: 3 n = p / 4 mod 32, and 11 is the inverse of 3.
+__device__ __forceinline__ uint32_t past_line(const void *p) {
+    return (uint32_t)((uint64_t)p >> 2) * 11u & 31u;
+}
+// records [0, n) of a wave that fit below a capacity of `cap`, the wave's
+// record `skip` being number `at`
+__device__ __forceinline__ uint32_t record_limit(uint64_t cap, uint64_t at, uint32_t skip) {
+    return cap > at ? (uint32_t)min(cap - at, (uint64_t)0x40000000u) + skip : 0u;
+}
+
+// The whole mesh of a chunk of 8, 16 or 32 words by one wave.
+//
+// Bound: at 1024^3 (222 M vertices, 445 M triangles) it moves 11.1 GB, 2.1 ms
+// at the copy rate; the vector units are busy 60 % and LDS 50 % of the time.
+// One wave makes a chunk's vertices and triangles, so the signs are loaded and
+// the crossings derived once and the edges come out of the cell steps as a
+// ring, without a pass of their own (two kinds of workgroup before: 18 % of
+// the vector instructions were second copies of this set-up, 30 % the edge
+// lists).  Edge and triangle records leave 64 at a time on 128-byte line
+// boundaries: non-temporal stores of 12-byte records move 3.9 TB/s when every
+// store ends inside a line and 5.0 TB/s when only a wave's first and last do.
+// 1024^3: 3231 -> 2665 us, 512^3: 186 -> 172, 128^3: 25 -> 15, 40^3: 23 -> 10.
+//
+// Workgroups of four waves: they share the triangle table, and with eight a
+// wave that is done waits for more of the others before its LDS is free
+// (1024^3: 2860).  LDS (29 KB) and registers hold five workgroups per CU;
+// owner data in LDS instead of cross-lane reads costs two of them (3225).
+template <class Src, bool kSelf>
+__global__ void __launch_bounds__(64 * kEmitWaves)
+emit_kernel(Src src, EmitArgs a) {
+    __shared__ EmitShared<kSelf> sh;
+    constexpr uint32_t kThreads = 64 * kEmitWaves;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    // Workgroup b runs on XCD b % 8, and so would every eighth workgroup of a
+    // plane, the same rows in every plane: mixing the higher bits in spreads a
+    // part that fills some of the rows over all XCDs (512^3: 185 -> 175 us).
+    uint32_t bx = blockIdx.x;
+    if ((bx | 7u) < gridDim.x) bx ^= (bx >> 3 ^ bx >> 6 ^ bx >> 9 ^ bx >> 12 ^ bx >> 15) & 7u;
+    // a workgroup takes 4 << lw words of a block of 256
+    const uint32_t lw = a.lw, lparts = 6 - lw;
+    const uint32_t gb = bx >> lparts, part = bx & ((1u << lparts) - 1u);
+    const uint32_t w0 = (kEmitWaves * part + wave) << lw;  // the wave's first word in its block
+    static_assert(kEmitWaves == 4 && kBlock == 256, "64 >> lw workgroups per block");
+    uint64_t vblock, tblock;  // the block's first vertex and triangle
+    ulonglong2 q0 = make_ulonglong2(0, 0), q1 = q0;
+    if constexpr (kSelf) {
+        static_assert(kSelfBlocks == 2 * kThreads, "two blocks per thread");
+        if (2 * tid < a.nb) q0 = ((const ulonglong2 *)a.bsum)[2 * tid];
+        if (2 * tid + 1 < a.nb) q1 = ((const ulonglong2 *)a.bsum)[2 * tid + 1];
+    }
+    const uint32_t live = a.live[gb];
+    const uint32_t wg_groups = kEmitWaves << lw >> 3;  // groups of 8 words per workgroup
+    const bool wg_live = (live >> (part * wg_groups)) & ((1u << wg_groups) - 1u);
+    if (!wg_live && !(kSelf && gb == 0 && part == 0)) return;
+    const uint32_t si = src.seg_of(gb);
+    const Seg s = src.get(si);
+    const Grid &g = s.g;
+    // words of this wave: [k0, k0 + (1 << lw)); lane: one half word
+    const uint32_t k0 = (gb - s.block_off) * kBlock + w0;
+    const uint32_t h = lane & 1;
+    const uint32_t kw = k0 + (lane >> 1);
+    const bool mine = lane < (2u << lw) && kw < (uint32_t)g.words;
+    const uint32_t kk = mine ? kw : k0;
+    const bool wave_live = (live >> (w0 >> 3)) & ((1u << (1u << (lw - 3))) - 1u);
+    uint32_t wa, wb, wc, wd, we, wf, wg, wh, na, nb, nc, nd, ne;
+    uint32_t b1 = 0, b2 = 0, b3 = 0, vb1, vb2, vb3, todo = 0, cy = 0, off = 0, yz = 0, xh = 0, row0 = 0;
+    constexpr int kTab = 5 * 256 / kThreads;
+    static_assert(kTab * kThreads == 5 * 256, "the table is loaded whole");
+    uint32_t tb[kTab];
 #pragma unroll
-        for (uint32_t i = 0; i < kGroups; ++i) tnext += i < ng ? gcount[i] : 0u;
-        const uint32_t nact = (uint32_t)__popc(act);
-        const uint32_t aincl = wave_scan_incl(nact);
-        const uint32_t atot = readlane32(aincl, 63);
-        const uint32_t aex = aincl - nact;
-        uint16_t *list = sh.list[wave];
-        uint32_t *vid = sh.vid[wave];
-        uint32_t *own = sh.own[wave];
-        for (uint32_t r0 = 0; r0 < atot; r0 += kCellCap) {
-            fill_cells(list, act, nact, aex, atot, r0, lane);
-            const uint32_t n = min((uint32_t)kCellCap, atot - r0);
-            for (uint32_t e0 = 0; e0 < n; e0 += 64) {
-                const uint32_t e = e0 + lane;
-                const bool on = e < n;
-                const uint32_t ent = on ? list[e] : 0u;
-                const uint32_t j = ent & 63, x = ent >> 6;
-                // row by row: each row's edge ids go to LDS as soon as they
-                // are known, so only one row's gathered halves are live
-                const bool last = x == 31;
-                const uint32_t xn = last ? 0u : x + 1;
-                const uint32_t below = (1u << x) - 1u;
-                const uint32_t cy = gather32(carry, j);
-                const uint32_t a0 = bit32(gather32(wa, j), x);
-                uint32_t x0, y0, z0, x1, z1, x2, x3;
-                {  // row (y, z): x- and y-edges at x and x+1, z-edges at x and x+1
-                    const uint32_t gx = gather32(ex0, j), gy = gather32(ey0, j), gz = gather32(ez0, j);
-                    x0 = bit32(gx, x);
-                    y0 = bit32(gy, x);
-                    z0 = bit32(gz, x);
-                    const uint32_t sx = last ? (cy & 1u) : bit32(gx, xn);
-                    const uint32_t sy = last ? ((cy >> 1) & 1u) : bit32(gy, xn);
-                    const uint32_t p = gather32(vb0, j) + __popc(gx & below) + __popc(gy & below) +
-                                       __popc(gz & below);
-                    const uint32_t q = p + x0 + y0 + z0;  // first edge of point x+1
-                    vid[0 * 64 + (lane ^ 0)] = p;             // x-edge of (x,   y,   z)
-                    vid[3 * 64 + (lane ^ 3)] = p + x0;        // y-edge of (x,   y,   z)
-                    vid[8 * 64 + (lane ^ 8)] = p + x0 + y0;   // z-edge of (x,   y,   z)
-                    vid[1 * 64 + (lane ^ 1)] = q + sx;        // y-edge of (x+1, y,   z)
-                    vid[9 * 64 + (lane ^ 9)] = q + sx + sy;   // z-edge of (x+1, y,   z)
-                }
-                {  // row (y+1, z)
-                    const uint32_t gx = gather32(ex1, j), gy = gather32(ey1, j), gz = gather32(ez1, j);
-                    x1 = bit32(gx, x);
-                    const uint32_t y1 = bit32(gy, x);
-                    z1 = bit32(gz, x);
-                    const uint32_t sx = last ? ((cy >> 2) & 1u) : bit32(gx, xn);
-                    const uint32_t sy = last ? ((cy >> 3) & 1u) : bit32(gy, xn);
-                    const uint32_t p = gather32(vb1, j) + __popc(gx & below) + __popc(gy & below) +
-                                       __popc(gz & below);
-                    vid[2 * 64 + (lane ^ 2)] = p;                         // x-edge of (x,   y+1, z)
-                    vid[11 * 64 + (lane ^ 11)] = p + x1 + y1;             // z-edge of (x,   y+1, z)
-                    vid[10 * 64 + (lane ^ 10)] = p + x1 + y1 + z1 + sx + sy;  // z-edge of (x+1, y+1, z)
-                }
-                {  // row (y, z+1)
-                    const uint32_t gx = gather32(ex2, j), gy = gather32(ey2, j), gz = gather32(ez2, j);
-                    x2 = bit32(gx, x);
-                    const uint32_t y2 = bit32(gy, x), z2 = bit32(gz, x);
-                    const uint32_t sx = last ? ((cy >> 4) & 1u) : bit32(gx, xn);
-                    const uint32_t p = gather32(vb2, j) + __popc(gx & below) + __popc(gy & below) +
-                                       __popc(gz & below);
-                    vid[4 * 64 + (lane ^ 4)] = p;                    // x-edge of (x,   y,   z+1)
-                    vid[7 * 64 + (lane ^ 7)] = p + x2;               // y-edge of (x,   y,   z+1)
-                    vid[5 * 64 + (lane ^ 5)] = p + x2 + y2 + z2 + sx;  // y-edge of (x+1, y,   z+1)
-                }
-                {  // row (y+1, z+1)
-                    const uint32_t gx = gather32(ex3, j), gy = gather32(ey3, j), gz = gather32(ez3, j);
-                    x3 = bit32(gx, x);
-                    vid[6 * 64 + (lane ^ 6)] = gather32(vb3, j) + __popc(gx & below) +
-                                               __popc(gy & below) + __popc(gz & below);
-                }
-                // corners: 0 (x,y,z) 1 (x+1,y,z) 2 (x+1,y+1,z) 3 (x,y+1,z)
-                //          4 (x,y,z+1) 5 (x+1,y,z+1) 6 (x+1,y+1,z+1) 7 (x,y+1,z+1)
-                const uint32_t k0 = a0, k1 = a0 ^ x0, k3 = a0 ^ y0, k2 = k3 ^ x1;
-                const uint32_t k4 = a0 ^ z0, k5 = k4 ^ x2, k7 = k3 ^ z1, k6 = k7 ^ x3;
-                const uint32_t cube = k0 | (k1 << 1) | (k2 << 2) | (k3 << 3) | (k4 << 4) |
-                                      (k5 << 5) | (k6 << 6) | (k7 << 7);
-                const uint64_t packed = s_tri[cube];
-                const uint32_t nt = on ? (uint32_t)(packed >> 60) : 0u;
-                const uint32_t tincl = wave_scan_incl(nt);
-                const uint32_t tex = tincl - nt, ttot = readlane32(tincl, 63);
-                if (on) {
-                    uint64_t rest = packed;
-                    for (uint32_t jt = 0; jt < nt; ++jt, rest >>= 12)
-                        own[tex + jt] = lane | (((uint32_t)rest & 0xfffu) << 8);
-                }
-                __builtin_amdgcn_wave_barrier();
-                // the wave's triangles, one per lane: consecutive lanes store
-                // consecutive 12-byte records
-                for (uint32_t te = lane; te < ttot; te += 64) {
-                    const uint32_t o = own[te], l = o & 63u;
-                    const uint64_t t = tnext + te;
-                    if (t < tcap) {
-                        const uint32_t e0v = (o >> 8) & 15u;
-                        const uint32_t e1v = (o >> 12) & 15u;
-                        const uint32_t e2v = (o >> 16) & 15u;
-                        const uint32_t v0 = vid[e0v * 64 + (l ^ e0v)];
-                        const uint32_t v1 = vid[e1v * 64 + (l ^ e1v)];
-                        const uint32_t v2 = vid[e2v * 64 + (l ^ e2v)];
-                        store_nt(a.triangles + 3 * t, T3{v0, v1, v2});
-                    }
-                }
-                tnext += ttot;
-                __builtin_amdgcn_wave_barrier();
+    for (int i = 0; i < kTab; ++i) tb[i] = a.table[tid + i * kThreads];
+    uint2 first = make_uint2(0, 0);
+    if (wave_live) {
+        const WordPos p = word_pos(kk, g);
+        row0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(p.z * g.ny + p.y));
+        xh = 64u * (uint32_t)p.w + 32u * h;
+        off = ((uint32_t)(p.z * g.ny + p.y) - row0) * (uint32_t)g.nx + xh;
+        yz = (uint32_t)p.y | (uint32_t)p.z << 16;
+        const bool has_y = p.y + 1 < g.ny, has_z = p.z + 1 < g.nz;
+        // a row that does not exist stands for its own predecessor (no
+        // crossing between them), so no load needs a mask
+        const uint32_t W8 = 8u * (uint32_t)g.W, RW8 = (uint32_t)g.ny * W8;
+        const uint32_t dy = has_y ? W8 : 0u, dz = has_z ? RW8 : 0u;
+        const uint32_t dy2 = p.y + 2 < g.ny ? W8 : 0u, dz2 = p.z + 2 < g.nz ? RW8 : 0u;
+        const uint32_t dn = h == 0 || p.w + 1 < g.W ? 4u : 0u;  // the row's next half
+        const uint64_t *sg = a.signs + s.sign_off + k0;
+        const uint32_t oa = 8u * (kk - k0) + 4u * h;
+        const uint32_t ob = oa + dy, oc = oa + dz, od = ob + dz, oe = ob + dy2;
+        wa = load_u32(sg, oa);
+        wb = load_u32(sg, ob);
+        wc = load_u32(sg, oc);
+        wd = load_u32(sg, od);
+        we = load_u32(sg, oe);
+        wf = load_u32(sg, oe + dz);
+        wg = load_u32(sg, oc + dz2);
+        wh = load_u32(sg, od + dz2);
+        na = load_u32(sg, oa + dn);
+        nb = load_u32(sg, ob + dn);
+        nc = load_u32(sg, oc + dn);
+        nd = load_u32(sg, od + dn);
+        ne = load_u32(sg, oe + dn);
+        // first vertex of the half within its block, and of the block
+        const uint2 *bg = a.base + (uint64_t)s.block_off * kBlock + k0;
+        first = bg[0];
+        vb1 = *(const uint16_t *)((const char *)bg + (ob - 2u * h));
+        vb2 = *(const uint16_t *)((const char *)bg + (oc - 2u * h));
+        vb3 = *(const uint16_t *)((const char *)bg + (od - 2u * h));
+        b1 = (k0 + (ob >> 3)) >> 8;
+        b2 = (k0 + (oc >> 3)) >> 8;
+        b3 = (k0 + (od >> 3)) >> 8;
+        if constexpr (!kSelf) {
+            const uint64_t *gs = a.bsum + 2 * (uint64_t)s.block_off;
+            const uint32_t v_off = (uint32_t)a.res[si].v_off;
+            vb1 += (uint32_t)gs[2 * (uint64_t)b1] - v_off;
+            vb2 += (uint32_t)gs[2 * (uint64_t)b2] - v_off;
+            vb3 += (uint32_t)gs[2 * (uint64_t)b3] - v_off;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // the sign past the row's last point repeats it (no crossing there)
+        const int nv = g.nx - (int)xh;  // points from this half on
+        const uint32_t mw = (uint32_t)nv < 32u ? 1u << nv : 0u;
+        const uint32_t mn = nv == 32 ? 1u : (nv == 33 ? 2u : 0u);
+        na = (na & ~mn) | (__builtin_amdgcn_alignbit(na, wa, 31) & mn);
+        nb = (nb & ~mn) | (__builtin_amdgcn_alignbit(nb, wb, 31) & mn);
+        nc = (nc & ~mn) | (__builtin_amdgcn_alignbit(nc, wc, 31) & mn);
+        wa = (wa & ~mw) | ((wa + wa) & mw);
+        wb = (wb & ~mw) | ((wb + wb) & mw);
+        wc = (wc & ~mw) | ((wc + wc) & mw);
+        const uint32_t sa = __builtin_amdgcn_alignbit(na, wa, 1);
+        const uint32_t sb = __builtin_amdgcn_alignbit(nb, wb, 1);
+        const uint32_t sc = __builtin_amdgcn_alignbit(nc, wc, 1);
+        const uint32_t sd = __builtin_amdgcn_alignbit(nd, wd, 1);
+        const uint32_t own = (wa ^ sa) | (wa ^ wb) | (wa ^ wc);  // points with an edge
+        const uint32_t any = wa | sa | wb | sb | wc | sc | wd | sd;
+        const uint32_t all = wa & sa & wb & sb & wc & sc & wd & sd;
+        const uint32_t cells = has_y && has_z ? below32(nv - 1) : 0u;
+        todo = mine ? (own & below32(nv)) | (any & ~all & cells) : 0u;
+        cy = (na & 3u) | (nb & 3u) << 2 | (nc & 3u) << 4 | (nd & 1u) << 6 | (ne & 1u) << 7 |
+             (uint32_t)__popc(cells) << 16;
+    }
+    if constexpr (kSelf) {
+        // block sums -> first vertex of every block, this block's first
+        // triangle; the first block's workgroup writes the totals (512 blocks
+        // hold at most 512 x 81920 triangles: 32 bits)
+        const uint32_t qv = (uint32_t)(q0.x + q1.x), qt = (uint32_t)(q0.y + q1.y);
+        const uint32_t iv = wave_scan_incl(qv), it = wave_scan_incl(qt);
+        if (lane == 63) sh.sum[wave] = make_uint2(iv, it);
+        __syncthreads();
+        uint32_t v = iv - qv, t = it - qt;
+        for (uint32_t i = 0; i < kEmitWaves; ++i) {
+            v += i < wave ? sh.sum[i].x : 0u;
+            t += i < wave ? sh.sum[i].y : 0u;
+        }
+        sh.pre[2 * tid] = v;
+        sh.pre[2 * tid + 1] = v + (uint32_t)q0.x;
+        if (tid == gb >> 1) sh.first_tri = t + (gb & 1 ? (uint32_t)q0.y : 0u);
+        if (gb == 0 && part == 0 && tid == kThreads - 1) {
+            a.ctl[CTL_NV] = v + qv;
+            a.ctl[CTL_NT] = t + qt;
+            a.ctl[CTL_OVF] = 0;
+            if (a.d_counts) {
+                a.d_counts[0] = v + qv;
+                a.d_counts[1] = t + qt;
             }
         }
+        if (!wg_live) return;
+        __syncthreads();
+        if (wave_live) {
+            vb1 += sh.pre[b1];
+            vb2 += sh.pre[b2];
+            vb3 += sh.pre[b3];
+        }
+        vblock = sh.pre[gb];
+        tblock = sh.first_tri;
+    } else {
+        vblock = a.bsum[2 * (uint64_t)gb];
+        tblock = a.bsum[2 * (uint64_t)gb + 1];
+    }
+#pragma unroll
+    for (int i = 0; i < kTab; ++i) sh.tab[tid + i * kThreads] = tb[i];
+    if (tid < 3)
+        sh.stride[tid] = 4 * (tid == 0 ? 1ull : (uint64_t)g.nx * (tid == 2 ? (uint32_t)g.ny : 1u));
+    __syncthreads();
+    if (!wave_live) return;
+    uint64_t v_off = 0;
+    if constexpr (!kSelf) {
+        // vertex numbers that do not fit 32 bits: nothing of the grid is written
+        if (a.res[si].ovf) return;
+        v_off = a.res[si].v_off;
+    }
+    first.x = (uint32_t)__builtin_amdgcn_readfirstlane((int)first.x);
+    first.y = (uint32_t)__builtin_amdgcn_readfirstlane((int)first.y);
+    const uint64_t vout = vblock + (first.x & 0xffffu);  // the wave's first vertex
+    const uint64_t tout = tblock + first.y;              // and triangle
+    // Vertices and triangles are stored 64 at a time on line boundaries: the
+    // wave's records are counted from the boundary at or before its first
+    // one, `vskip` and `tskip` records earlier.
+    const uint32_t vskip = past_line(a.vertices + 3 * vout);
+    const uint32_t tskip = past_line(a.triangles + 3 * tout);
+    char *const vp = (char *)(a.vertices + 3 * vout) - 12 * vskip;
+    char *tp = (char *)(a.triangles + 3 * tout) - 12 * tskip;
+    const uint32_t vlimit = record_limit(a.vcap, vout, vskip);
+    uint32_t tlimit = record_limit(a.tcap, tout, tskip);
+    const uint32_t vid0 = (uint32_t)(vout - v_off) - vskip;  // number of record 0
+    uint32_t vnext = vskip, vdone = 0;                       // vertices listed, fetched
+    const float *field = a.field + s.field_off + (uint64_t)row0 * (uint32_t)g.nx;
+    EmitWave &w = sh.w[wave];
+    char *const vid = (char *)w.vid + 4 * lane;
+
+    // in VGPRs: an instruction with a scalar operand takes twice as long
+    Frame fr = {s.iso, s.ox, s.oy, s.oz, s.sx, s.sy, s.sz};
+    asm volatile("" : "+v"(fr.iso), "+v"(fr.ox), "+v"(fr.oy), "+v"(fr.oz));
+    asm volatile("" : "+v"(fr.sx), "+v"(fr.sy), "+v"(fr.sz));
+    uint32_t lane12 = 12 * lane;
+    asm volatile("" : "+v"(lane12));
+
+    // 64 edges from record `from` on (some listed): ring entries, owner data
+    // and field values; lanes without a listed edge repeat the nearest one
+    struct Flight {
+        uint32_t en, x, yz;
+        float f0, f1;
+    };
+    const auto fetch = [&](uint32_t from) {
+        Flight t;
+        t.en = w.ring[max(min(from + lane, vnext - 1), vskip) % kRing];
+        const int jj = (int)(t.en & 0xfcu);
+        const uint64_t step = sh.stride[t.en & 3u];
+        const uint32_t o = (uint32_t)__builtin_amdgcn_ds_bpermute(jj, (int)off) + (t.en >> 8);
+        t.yz = (uint32_t)__builtin_amdgcn_ds_bpermute(jj, (int)yz);
+        t.x = (uint32_t)__builtin_amdgcn_ds_bpermute(jj, (int)xh) + (t.en >> 8);
+        const char *p = (const char *)(field + o);
+        t.f0 = *(const float *)p;
+        t.f1 = *(const float *)(p + step);
+        return t;
+    };
+    const auto write = [&](const Flight &t, uint32_t from, uint32_t to) {
+        const V3 v = edge_vertex(fr, (float)t.x, (float)(t.yz & 0xffffu), (float)(t.yz >> 16),
+                                 t.en & 3u, t.f0, t.f1);
+        const uint32_t i = from + lane;
+        if (i >= vskip && i < min(to, vlimit)) store_nt((float *)(vp + (12 * from + lane12)), v);
+    };
+
+    // the cells (and points with an edge but no cell) in canonical order
+    const uint32_t ntodo = (uint32_t)__popc(todo);
+    const uint32_t incl = wave_scan_incl(ntodo);
+    const uint32_t total = readlane32(incl, 63);
+    uint32_t next = incl - ntodo;
+    // triangles left over by the last step: records [0, kept) in the lanes
+    T3 rec = {0, 0, 0};
+    uint32_t kept = tskip, tlow = tskip;
+
+    for (uint32_t e0 = 0; e0 < total; e0 += 64) {
+        if (e0 % kCellCap == 0) {
+            uint16_t *to = w.list + (next - e0);
+            for (; todo && next < e0 + kCellCap; todo &= todo - 1, ++next)
+                *to++ = (uint16_t)(4 * lane | (uint32_t)__builtin_ctz(todo) << 8);
+            wave_sync();
+        }
+        const bool on = e0 + lane < total;
+        const uint32_t ent = w.list[min(e0 + lane, total - 1) % kCellCap];
+        const bool ready = vnext - vdone >= 64;
+        Flight fl = {0, 0, 0, 0.f, 0.f};
+        if (ready) fl = fetch(vdone);
+        const int j = (int)(ent & 0xfcu);
+        const uint32_t x = ent >> 8;
+        const auto at = [&](uint32_t v) {
+            return (uint32_t)__builtin_amdgcn_ds_bpermute(j, (int)v);
+        };
+        const uint32_t c = at(cy);
+        const uint32_t ga = at(wa), gB = at(wb), gc_ = at(wc), gd = at(wd);
+        const uint32_t ge = at(we), gf = at(wf), gg = at(wg), gh = at(wh);
+        const uint32_t p1 = at(vb1), p2 = at(vb2), p3 = at(vb3);
+        // signs at x, x+1 (and x+2) of the four rows, at x (and x+1) past them
+        const uint32_t A = __builtin_amdgcn_alignbit(c, ga, x);
+        const uint32_t B = __builtin_amdgcn_alignbit(c >> 2, gB, x);
+        const uint32_t C = __builtin_amdgcn_alignbit(c >> 4, gc_, x);
+        const uint32_t D = __builtin_amdgcn_alignbit(c >> 6, gd, x);
+        const uint32_t E = __builtin_amdgcn_alignbit(c >> 7, ge, x);
+        const uint32_t G = gg >> x;
+        const uint32_t corners =
+            (((D << 2 | (C & 3u)) << 2 | (B & 3u)) << 2 | (A & 3u)) & 0xffu;
+        const bool cell = on && x < c >> 16;
+        const uint2 t01 = *(const uint2 *)(sh.tab + 2 * corners);
+        const uint32_t nt = cell ? (t01.x & 3u) | (t01.y & 3u) << 2 : 0u;
+        // row (y, z): edges of points x and x+1
+        const uint32_t xa = A ^ A >> 1, ya = A ^ B, za = A ^ C;
+        const uint32_t x0 = on ? xa & 1u : 0u, y0 = on ? ya & 1u : 0u, z0 = on ? za & 1u : 0u;
+        const uint32_t c0 = x0 + y0 + z0;
+        const uint32_t mine2 = c0 | nt << 16;
+        const uint32_t inc2 = wave_scan_incl(mine2), tot2 = readlane32(inc2, 63);
+        const uint32_t ex2 = inc2 - mine2;
+        const uint32_t ttot = tot2 >> 16;
+        uint32_t tpos = ex2 >> 16;
+        const uint32_t rel = vnext + (ex2 & 0xffffu);
+        const auto id = [&](int e, uint32_t v) { *(uint32_t *)(vid + 4 * kIdStride * e) = v; };
+        {
+            const uint32_t p = vid0 + rel, px = p + x0, py = px + y0, q = py + z0;
+            const uint32_t qx = q + (xa >> 1 & 1u);
+            id(0, p);
+            id(3, px);
+            id(8, py);
+            id(1, qx);
+            id(9, qx + (ya >> 1 & 1u));
+            if (c0) {
+                // its edges in order; a lane writes three entries, the
+                // last first, and what is not its own is overwritten by
+                // the lane that it belongs to
+                w.ring[(rel + 2) % kRing] = (uint16_t)(ent + 2);
+                in_order();
+                w.ring[(rel + 1) % kRing] = (uint16_t)(ent + 2 - (x0 & y0));
+                in_order();
+                w.ring[rel % kRing] = (uint16_t)(ent + ((2 - y0) & (x0 - 1)));
+            }
+        }
+        const uint32_t low = (1u << x) - 1u;  // points before x in the half
+        {                                     // row (y+1, z)
+            const uint32_t xb = B ^ B >> 1, yb = B ^ E, zb = B ^ D;
+            const uint32_t s_b = __builtin_amdgcn_alignbit(c >> 2, gB, 1);
+            const uint32_t p = p1 + __popc((gB ^ s_b) & low) + __popc((gB ^ ge) & low) +
+                               __popc((gB ^ gd) & low);
+            const uint32_t q = p + (xb & 1u) + (yb & 1u);
+            id(2, p);
+            id(11, q);
+            id(10, q + (zb & 1u) + (xb >> 1 & 1u) + (yb >> 1 & 1u));
+        }
+        {  // row (y, z+1)
+            const uint32_t xc = C ^ C >> 1, yc = C ^ D, zc = C ^ G;
+            const uint32_t s_c = __builtin_amdgcn_alignbit(c >> 4, gc_, 1);
+            const uint32_t p = p2 + __popc((gc_ ^ s_c) & low) + __popc((gc_ ^ gd) & low) +
+                               __popc((gc_ ^ gg) & low);
+            const uint32_t q = p + (xc & 1u);
+            id(4, p);
+            id(7, q);
+            id(5, q + (yc & 1u) + (zc & 1u) + (xc >> 1 & 1u));
+        }
+        {  // row (y+1, z+1)
+            const uint32_t s_d = __builtin_amdgcn_alignbit(c >> 6, gd, 1);
+            id(6, p3 + __popc((gd ^ s_d) & low) + __popc((gd ^ gf) & low) +
+                      __popc((gd ^ gh) & low));
+        }
+        // the step's triangles in order, the same way
+        const uint32_t me = lane * 0x00401004u;
+        if (nt) {
+            uint32_t *own = w.own + tpos;
+            if (__any(nt > 2)) {
+                const uint2 t23 = *(const uint2 *)(sh.tab + 512 + 2 * corners);
+                if (__any(nt > 4)) own[4] = sh.tab[1024 + corners] + me;
+                in_order();
+                own[3] = t23.y + me;
+                in_order();
+                own[2] = t23.x + me;
+                in_order();
+            }
+            own[1] = t01.y + me;
+            in_order();
+            own[0] = t01.x + me;
+        }
+        vnext += tot2 & 0xffffu;
+        wave_sync();
+        // the edges whose loads were issued at the top of the step, before
+        // the triangles' stores (a wait for loads waits for stores as well)
+        if (ready) {
+            write(fl, vdone, vdone + 64);
+            vdone += 64;
+        }
+        // triangles: kept ones and this step's, 64 records per store
+        const uint32_t avail = kept + ttot;
+        const char *ids = (const char *)w.vid;
+        for (uint32_t at = 0;; at += 64) {
+            const uint32_t i = at + lane;
+            if (i >= kept && i < avail) {
+                const uint32_t q = w.own[i - kept];
+                rec.a = *(const uint32_t *)(ids + (q & 0xffcu));
+                rec.b = *(const uint32_t *)(ids + (q >> 10 & 0xffcu));
+                rec.c = *(const uint32_t *)(ids + (q >> 20 & 0xffcu));
+            }
+            if (at + 64 > avail) break;
+            if (lane >= tlow && lane < tlimit) store_nt((uint32_t *)(tp + lane12), rec);
+            tp += 768;
+            tlimit -= min(tlimit, 64u);
+            tlow = 0;
+        }
+        kept = avail % 64;
+        while (vnext - vdone >= 128) {
+            write(fetch(vdone), vdone, vdone + 64);
+            vdone += 64;
+        }
+        wave_sync();
+    }
+    if (lane >= tlow && lane < min(kept, tlimit)) store_nt((uint32_t *)(tp + lane12), rec);
+    // at most 127 edges are left: both fetches before the first store
+    if (vnext - vdone > 64) {
+        const Flight f = fetch(vdone), l = fetch(vdone + 64);
+        write(f, vdone, vnext);
+        write(l, vdone + 64, vnext);
+    } else if (max(vdone, vskip) < vnext) {
+        write(fetch(vdone), vdone, vnext);
     }
 }
 
-// The vertex and triangle stages in one launch: they depend only on the count
-// stage and the block scan, so their workgroups are interleaved (workgroup w:
-// w % 3 == 0 runs count block w / 3's vertices, the other two its two
-// triangle halves) and run side by side on every CU; the stages wait on
-// different things (field loads, LDS gathers), so each hides the other's
-// latency.
-union EmitShared {
-    VertShared v;
-    TriShared t;
-};
+}  // namespace
 
-template <class Src>
-__global__ void __launch_bounds__(kBlock) emit_kernel(Src src, VertArgs va, TriArgs ta) {
-    static_assert(kTriThreads == kBlock, "both stages run 256-thread workgroups");
-    __shared__ EmitShared sh;
-    const uint32_t w = blockIdx.x, gb = w / 3, r = w - 3 * gb;
-    if (r == 0)
-        vert_block(src, va, gb, sh.v);
-    else
-        tri_block(src, ta, 2 * gb + (r - 1), sh.t);
+namespace {
+// Words per wave of the emission for a launch of nb blocks, as a logarithm.
+// The chip holds 5120 waves of it: a launch gets that many, in shorter chunks
+// (a wave works through its cells 64 at a time), before the chunks grow to 32
+// words, which costs least per cell.
+// 128 blocks (128^3): 16.1 us in chunks of 8 words, 17.3 of 16; 422 blocks:
+// 37.6, 35.6, 35.6 (32 words); 1.7 k blocks (16 served grids): 119.5 of 16, 126 of 32.
+uint32_t words_per_wave_log2(uint64_t nb) { return nb >= 4096 ? 5 : (nb >= 256 ? 4 : 3); }
+
+template <class Src, bool kSelf>
+int launch_emit(const Src &src, const EmitArgs &a, uint64_t nb, hipStream_t stream) {
+    const uint64_t wgs = nb << (6 - a.lw);
+    GC_ARG(wgs <= 0xffffffffull, "grid too large");
+    hipLaunchKernelGGL((emit_kernel<Src, kSelf>), dim3((unsigned)wgs), dim3(64 * kEmitWaves), 0,
+                       stream, src, a);
+    GC_CHECK_LAUNCH();
+    return GPUCAD_OK;
 }
-
 }  // namespace
 
 // Enqueues the whole one-grid extraction on `stream` given a workspace.
@@ -985,54 +958,49 @@ int enqueue_extract(const gc_extract_args *a, hipStream_t stream) {
         GC_CHECK_LAUNCH();
         signs = sw;
     }
-    uint32_t *base = (uint32_t *)(ws + L.base_off);
-    uint32_t *twave = (uint32_t *)(ws + L.twave_off);
+    uint2 *base = (uint2 *)(ws + L.base_off);
+    uint32_t *live = (uint32_t *)(ws + L.live_off);
     uint64_t *bsum = (uint64_t *)(ws + L.bsum_off);
     uint64_t *ctl = (uint64_t *)(ws + L.ctl_off);
     SegResult *res = (SegResult *)(ws + L.res_off);
     hipLaunchKernelGGL(count_kernel<OneGrid>, dim3((unsigned)L.nb), dim3(kBlock), 0, stream, one,
-                       CountArgs{signs, twave, bsum, base});
+                       CountArgs{signs, live, bsum, base});
     GC_CHECK_LAUNCH();
-    hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(1024), 0, stream, bsum, L.nb, ctl,
-                       a->d_counts, (const Seg *)nullptr, 1u, res);
-    GC_CHECK_LAUNCH();
-    const VertArgs va = {a->field, signs, bsum, res, a->vertices,
-                         a->vertices ? a->vert_capacity : 0};
-    const TriArgs ta = {signs, base, twave, bsum, tabs->tri_packed, res, a->triangles,
-                        a->triangles ? a->tri_capacity : 0};
-    GC_ARG(L.nb <= 0xffffffffull / 3, "grid too large");
+    const bool self = L.nb <= (uint64_t)kSelfBlocks;
+    if (!self) {
+        hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(1024), 0, stream, bsum, L.nb, ctl,
+                           a->d_counts, (const Seg *)nullptr, 1u, res);
+        GC_CHECK_LAUNCH();
+    }
+    const uint32_t lw = words_per_wave_log2(L.nb);
+    const EmitArgs ea = {a->field, signs, base, live, bsum, res, tabs->emit, a->vertices,
+                         a->vertices ? a->vert_capacity : 0, a->triangles,
+                         a->triangles ? a->tri_capacity : 0, lw, (uint32_t)L.nb, ctl, a->d_counts};
     if (a->emit_event) GC_HIP(hipEventRecord((hipEvent_t)a->emit_event, stream));
-    hipLaunchKernelGGL(emit_kernel<OneGrid>, dim3(3 * (unsigned)L.nb), dim3(kBlock), 0, stream,
-                       one, va, ta);
-    GC_CHECK_LAUNCH();
-    return GPUCAD_OK;
+    return self ? launch_emit<OneGrid, true>(one, ea, L.nb, stream)
+                : launch_emit<OneGrid, false>(one, ea, L.nb, stream);
 }
 
 int enqueue_extract_batch(const BatchExtract &b, int phases, hipStream_t stream) {
     GC_ARG(b.nseg > 0 && b.nb > 0 && b.segs && b.blk2seg, "empty batch");
-    GC_ARG(b.nb <= 0xffffffffu / 3, "batch too large");
+    const uint32_t lw = words_per_wave_log2(b.nb);
     const DeviceTables *tabs = nullptr;
     int st = device_tables(&tabs);
     if (st) return st;
     const ManyGrids src = {b.segs, b.blk2seg};
-    // one workgroup per block (two per block for the triangle stage), as for
-    // one grid
     if (phases & EXTRACT_COUNT) {
         hipLaunchKernelGGL(count_kernel<ManyGrids>, dim3(b.nb), dim3(kBlock), 0, stream, src,
-                           CountArgs{b.signs, b.twave, b.bsum, b.base});
+                           CountArgs{b.signs, b.live, b.bsum, (uint2 *)b.base});
         GC_CHECK_LAUNCH();
         hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(1024), 0, stream, b.bsum,
                            (uint64_t)b.nb, b.ctl, (uint64_t *)nullptr, b.segs, b.nseg, b.res);
         GC_CHECK_LAUNCH();
     }
     if (phases & EXTRACT_EMIT) {
-        const VertArgs va = {b.fields, b.signs, b.bsum, b.res, b.vertices,
-                             b.vertices ? b.vcap : 0};
-        const TriArgs ta = {b.signs, b.base, b.twave, b.bsum, tabs->tri_packed, b.res,
-                            b.triangles, b.triangles ? b.tcap : 0};
-        hipLaunchKernelGGL(emit_kernel<ManyGrids>, dim3(3 * b.nb), dim3(kBlock), 0, stream, src,
-                           va, ta);
-        GC_CHECK_LAUNCH();
+        const EmitArgs ea = {b.fields, b.signs, (const uint2 *)b.base, b.live, b.bsum, b.res,
+                             tabs->emit, b.vertices, b.vertices ? b.vcap : 0, b.triangles,
+                             b.triangles ? b.tcap : 0, lw, b.nb, nullptr, nullptr};
+        if ((st = launch_emit<ManyGrids, false>(src, ea, b.nb, stream))) return st;
     }
     return GPUCAD_OK;
 }

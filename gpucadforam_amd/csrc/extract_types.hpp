@@ -11,19 +11,22 @@
 namespace gc {
 
 constexpr int kBlock = 256;  // words per extraction block (4 waves)
-constexpr int kGroups = 8;   // triangle-count groups (32 words each) per block
-// per block: first vertex number of each 32-point half word (uint32), and the
-// triangle count of each group (uint32)
-constexpr uint64_t kBaseBytesPerBlock = (uint64_t)kBlock * 2 * 4;
-constexpr uint64_t kTwaveBytesPerBlock = (uint64_t)kGroups * 4;
+// per block: the block-local first vertices and first triangle of each word
+// (8 bytes), and a bit per 8 words that have something to emit (32 bits)
+constexpr uint64_t kBaseBytesPerBlock = (uint64_t)kBlock * 8;
+constexpr uint64_t kLiveBytesPerBlock = 4;
 
-// n / d for n < 2^32 through a double reciprocal and one correction step
+// n / d for n < 2^32: the high half of n * m, m = floor(2^32 / d), is n / d or
+// one less (the error n * (2^32 mod d) / (d * 2^32) is below n / 2^32 < 1), so
+// one comparison of the remainder corrects it.  d = 1: m = 2^32 - 1, which
+// gives n - 1 for n > 0.
 struct FastDiv {
-    uint32_t d;
-    double inv;
+    uint32_t d, m;
 };
 
-inline FastDiv make_div(uint32_t d) { return FastDiv{d, 1.0 / (double)d}; }
+inline FastDiv make_div(uint32_t d) {
+    return FastDiv{d, d == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / d)};
+}
 
 struct Grid {
     int nx, ny, nz, W;  // W = sign words per row
@@ -75,7 +78,7 @@ struct BatchExtract {
     const Seg *segs;           // device, nseg
     const uint32_t *blk2seg;   // device, nb: grid of each global block
     uint32_t nseg, nb;
-    uint32_t *base, *twave;    // nb * kBlock * 2, nb * kGroups
+    uint32_t *base, *live;     // nb * kBlock * 2, nb
     uint64_t *bsum;            // nb * 2
     uint64_t *ctl;             // 8 x uint64: totals, any overflow
     SegResult *res;            // device, nseg

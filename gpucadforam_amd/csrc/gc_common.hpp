@@ -38,7 +38,7 @@ void clear_error();
 
 // Device-resident copies of the marching-cubes tables (one set per device).
 struct DeviceTables {
-    uint64_t *tri_packed = nullptr;  // 256 x uint64: 15 edge nibbles + count in nibble 15
+    uint32_t *emit = nullptr;        // 5 x 256 (host_emit_table)
     uint8_t *num_verts = nullptr;    // 256
     uint8_t *tri_table = nullptr;    // 256*16 (255 terminated)
 };
@@ -50,7 +50,8 @@ int device_tables(const DeviceTables **out);
 const uint8_t *host_tri_table();     // 256*16
 const uint8_t *host_num_verts();     // 256
 const uint16_t *host_edge_mask();    // 256
-const uint64_t *host_tri_packed();   // 256
+constexpr int kEmitStride = 65;      // words from one edge's vertex numbers to the next's
+const uint32_t *host_emit_table();   // 5 x 256: triangles as the emission reads them
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 

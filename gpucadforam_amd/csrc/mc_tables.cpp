@@ -63,7 +63,7 @@ struct HostTables {
     uint8_t tri[256 * 16];
     uint8_t nverts[256];
     uint16_t emask[256];
-    uint64_t packed[256];
+    uint32_t emit[5 * 256];
 };
 
 HostTables g_tables;
@@ -76,22 +76,36 @@ void decode() {
     for (int c = 0; c < 256; ++c) {
         const char *row = kTriRows[c];
         int n = (int)std::strlen(row);
-        uint64_t packed = 0;
         for (int j = 0; j < 16; ++j) g_tables.tri[c * 16 + j] = 255;
         for (int j = 0; j < n; ++j) {
             int e = hexval(row[j]);
             g_tables.tri[c * 16 + j] = (uint8_t)e;
-            packed |= (uint64_t)e << (4 * j);
         }
-        packed |= (uint64_t)(n / 3) << 60;
         g_tables.nverts[c] = (uint8_t)n;
-        g_tables.packed[c] = packed;
         uint16_t m = 0;
         for (int e = 0; e < 12; ++e) {
             int a = (c >> kEdge[e][0]) & 1, b = (c >> kEdge[e][1]) & 1;
             if (a != b) m |= (uint16_t)(1u << e);
         }
         g_tables.emask[c] = m;
+    }
+    // The emission indexes cases by sign pairs, bit 2r + i: the sign at x + i
+    // of row r (rows (y,z) (y+1,z) (y,z+1) (y+1,z+1)), corners
+    // 0 1, 3 2, 4 5, 7 6.  Word q of a case holds the byte offsets of
+    // triangle q's three vertex numbers (edge e's row of kEmitStride words)
+    // in bits 2..11, 12..21 and 22..31; the two low bits of words 0 and 1 hold
+    // the number of triangles.
+    const int corner[8] = {0, 1, 3, 2, 4, 5, 7, 6};
+    for (int i = 0; i < 256; ++i) {
+        int c = 0;
+        for (int b = 0; b < 8; ++b) c |= ((i >> b) & 1) << corner[b];
+        const uint32_t nt = g_tables.nverts[c] / 3;
+        for (uint32_t q = 0; q < 5; ++q) {
+            uint32_t w = q == 0 ? nt & 3 : (q == 1 ? nt >> 2 : 0);
+            for (int v = 0; q < nt && v < 3; ++v)
+                w |= (uint32_t)(g_tables.tri[c * 16 + 3 * q + v] * kEmitStride) << (2 + 10 * v);
+            g_tables.emit[q < 4 ? 512 * (q / 2) + 2 * i + q % 2 : 1024 + i] = w;
+        }
     }
 }
 
@@ -105,7 +119,7 @@ const HostTables &tables() {
 const uint8_t *host_tri_table() { return tables().tri; }
 const uint8_t *host_num_verts() { return tables().nverts; }
 const uint16_t *host_edge_mask() { return tables().emask; }
-const uint64_t *host_tri_packed() { return tables().packed; }
+const uint32_t *host_emit_table() { return tables().emit; }
 
 }  // namespace gc
 

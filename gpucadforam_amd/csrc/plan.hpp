@@ -34,7 +34,7 @@ struct DevPlan {
     Seg *segs = nullptr;
     uint32_t *blk2seg = nullptr;
     SegResult *res = nullptr;
-    uint32_t *base = nullptr, *twave = nullptr;
+    uint32_t *base = nullptr, *live = nullptr;
     uint64_t *bsum = nullptr, *ctl = nullptr;
 };
 

@@ -116,7 +116,7 @@ uint64_t work_bytes(const gc_lattice_params &p, const Shape &sh) {
     b += round_up(brick_count(p, sh.bx, sh.lz) * 8, kGranule);
     b += round_up(nb * 4, kGranule);                    // blk2seg
     b += round_up(nb * kBaseBytesPerBlock, kGranule);   // base
-    b += round_up(nb * kTwaveBytesPerBlock, kGranule);  // twave
+    b += round_up(nb * kLiveBytesPerBlock, kGranule);   // live
     b += round_up(nb * 16, kGranule);                   // bsum
     b += round_up(round_up(words, 32) * 8, kGranule);   // sign words
     return b;
@@ -304,7 +304,7 @@ struct Server {
         const uint64_t o_b2s = take(nb * 4);
         const uint64_t o_res = take(n * sizeof(SegResult));
         const uint64_t o_base = take(nb * kBaseBytesPerBlock);
-        const uint64_t o_twave = take(nb * kTwaveBytesPerBlock);
+        const uint64_t o_live = take(nb * kLiveBytesPerBlock);
         const uint64_t o_bsum = take(nb * 16);
         const uint64_t o_ctl = take(64);
         if (at > g.work_off + g.work_size)
@@ -315,7 +315,7 @@ struct Server {
         g.d.blk2seg = (uint32_t *)(A + o_b2s);
         g.d.res = (SegResult *)(A + o_res);
         g.d.base = (uint32_t *)(A + o_base);
-        g.d.twave = (uint32_t *)(A + o_twave);
+        g.d.live = (uint32_t *)(A + o_live);
         g.d.bsum = (uint64_t *)(A + o_bsum);
         g.d.ctl = (uint64_t *)(A + o_ctl);
         g.fields = (float *)A;
