@@ -166,6 +166,10 @@ struct ManyGrids {
 // ---------------------------------------------------------------------------
 // signs
 // ---------------------------------------------------------------------------
+// A wave makes the words of 64 points of kSignZ rows, one above the other in
+// z.  Bound by the field's bytes; the rows' loads are all under way before
+// the first comparison (one load, one wait and one 8-byte store per row
+// before: 203 x 149 x 181, 22 MB, 12.6 us; 8.0 now).
 constexpr int kSignZ = 8;
 
 __global__ void __launch_bounds__(256)
@@ -178,11 +182,19 @@ signs_kernel(const float *__restrict__ field, uint64_t *__restrict__ signs, int 
     if (y >= ny) return;
     const bool xin = x < nx;
     const uint64_t plane = (uint64_t)nx * ny;
-    for (int z = z0; z < min(z0 + kSignZ, nz); ++z) {
-        float f = xin ? field[(uint64_t)z * plane + (uint64_t)y * nx + x] : 0.f;
-        uint64_t m = __ballot(xin && f < iso);
-        if (lane == 0) signs[((uint64_t)z * ny + y) * W + blockIdx.x] = m;
+    const float *p = field + (uint64_t)z0 * plane + (uint64_t)y * nx + (xin ? x : nx - 1);
+    const int n = min(kSignZ, nz - z0);
+    float f[kSignZ];
+#pragma unroll
+    for (int i = 0; i < kSignZ; ++i) f[i] = p[(uint64_t)min(i, n - 1) * plane];
+    __builtin_amdgcn_sched_barrier(0);
+    uint64_t mine = 0;
+#pragma unroll
+    for (int i = 0; i < kSignZ; ++i) {
+        const uint64_t m = __ballot(xin && f[i] < iso);
+        mine = lane == (uint32_t)i ? m : mine;
     }
+    if (lane < (uint32_t)n) signs[((uint64_t)(z0 + lane) * ny + y) * W + blockIdx.x] = mine;
 }
 
 // ---------------------------------------------------------------------------
