@@ -798,6 +798,12 @@ typedef float F4nt __attribute__((ext_vector_type(4)));
 // its waves share its L2.  Field two is read only by a wave with a corner
 // whose indicator is 2 (no other corner takes vertexInterp3_new's second
 // branch).
+//
+// Bound by the 32 bytes written per vertex: 240^3, 3.2 M active voxels, 22.6 M
+// vertices, 724 MB, 196 us with stores that begin inside a 128-byte line and
+// each batch's corners asked for behind the last one's stores; 177 us with
+// stores on line boundaries, 169 (4.3 TB/s) with the corners ahead of the
+// stores as well.  The vector units are busy half the time.
 template <int MODE>
 __global__ void __launch_bounds__(64) generate_kernel(GenArgs a) {
     __shared__ float3 vl[12][65];  // (stride 65: the edges of one voxel in different banks)
@@ -819,7 +825,10 @@ __global__ void __launch_bounds__(64) generate_kernel(GenArgs a) {
         bat_end = min(nbat, x * per + per);
         bat_step = gridDim.x >> 3;
     }
-    // each batch's voxel ids and vertex offsets are read one batch ahead
+    // Each batch's voxel ids and vertex offsets are read two batches ahead, its
+    // corners one: they are there before the batch in between writes its
+    // vertices, since a wait for a load waits for the stores before it too.
+    const uint32_t gx = a.g.size.x, gxy = a.g.size.x * a.g.size.y;
     uint32_t next_voxel = 0, next_vbase = 0;
     auto fetch = [&](uint32_t b) {
         const uint64_t j = (uint64_t)b * 64u + lane;
@@ -828,14 +837,37 @@ __global__ void __launch_bounds__(64) generate_kernel(GenArgs a) {
             next_vbase = a.vbase ? a.vbase[j] : a.scan[next_voxel];
         }
     };
+    float fid[8], f1[8];
+    uint32_t lin = 0;
+    uint3 gp = make_uint3(0, 0, 0);
+    auto load_corners = [&](uint32_t voxel, uint3 &p, uint32_t &at, float (&c)[8], float (&c1)[8]) {
+        p = calc_grid_pos(voxel, a.g.shift, a.g.mask);
+        at = p.z * gxy + p.y * gx + p.x;
+        corners_inside(a.vol, at, gx, gxy, c);
+        if (MODE != GEN_STD) corners_inside(a.vol1, at, gx, gxy, c1);
+    };
+    auto is_on = [&](uint32_t b) { return b < bat_end && (uint64_t)b * 64u + lane < active; };
+    if (bat >= bat_end) return;
     fetch(bat);
+    uint32_t vbase = next_vbase, cube = 0, nv = 0;
+    uint4 row = make_uint4(0, 0, 0, 0);
+    if (is_on(bat)) {
+        load_corners(next_voxel, gp, lin, fid, f1);
+        cube = cube_of(fid, a.iso);
+        nv = a.nverts[cube];
+        row = *(const uint4 *)(a.tri + cube * 16);
+    }
+    fetch(bat + bat_step);
     for (; bat < bat_end; bat += bat_step) {
-        const uint64_t i = (uint64_t)bat * 64u + lane;
-        const uint32_t voxel = next_voxel;
-        uint32_t cube = 0, nv = 0, vbase = next_vbase;
-        fetch(bat + bat_step);
-        if (i < active) {
-            const uint3 gp = calc_grid_pos(voxel, a.g.shift, a.g.mask);
+        // the next batch's corners, the ids of the one after
+        const bool more = is_on(bat + bat_step);
+        float nid[8] = {}, n1[8] = {};
+        uint3 ngp = gp;
+        uint32_t nlin = lin;
+        const uint32_t nvbase = next_vbase;
+        if (more) load_corners(next_voxel, ngp, nlin, nid, n1);
+        fetch(bat + 2 * bat_step);
+        if (is_on(bat)) {
             float3 p;
             p.x = ((float)gp.x - a.g.center.x) * a.g.vs.x;
             p.y = ((float)gp.y - a.g.center.y) * a.g.vs.y;
@@ -850,40 +882,30 @@ __global__ void __launch_bounds__(64) generate_kernel(GenArgs a) {
             v[5] = make_float3(p.x + vs.x, p.y + 0.f, p.z + vs.z);
             v[6] = make_float3(p.x + vs.x, p.y + vs.y, p.z + vs.z);
             v[7] = make_float3(p.x + 0.f, p.y + vs.y, p.z + vs.z);
-            const uint32_t gx = a.g.size.x, gxy = a.g.size.x * a.g.size.y;
-            const uint32_t lin = gp.z * gxy + gp.y * gx + gp.x;
-            float fid[8];
-            corners_inside(a.vol, lin, gx, gxy, fid);
-            cube = cube_of(fid, a.iso);
-            nv = a.nverts[cube];
             if (MODE == GEN_STD) {
                 // an active voxel has nv > 0 (src/MarchingCubes_kernel.cu:3103)
 #pragma unroll
                 for (int e = 0; e < 12; ++e)
                     vl[e][lane] = interp4(a.iso, v[c_edge_a[e]], v[c_edge_b[e]],
                                           fid[c_edge_a[e]], fid[c_edge_b[e]]);
+            } else if (MODE == GEN_BAND2) {
+                bool two = false;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) two |= fid[k] == 2.f;
+                float f2[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                if (__any(two)) corners_inside(a.vol2, lin, gx, gxy, f2);
+#pragma unroll
+                for (int e = 0; e < 12; ++e) {
+                    int ca = c_edge_a[e], cb = c_edge_b[e];
+                    vl[e][lane] = interp3(a.lo1, a.hi1, v[ca], v[cb], f1[ca], f1[cb], f2[ca],
+                                          f2[cb], a.lo2, a.hi2, fid[ca], fid[cb]);
+                }
             } else {
-                float f1[8];
-                corners_inside(a.vol1, lin, gx, gxy, f1);
-                if (MODE == GEN_BAND2) {
-                    bool two = false;
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) two |= fid[k] == 2.f;
-                    float f2[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                    if (__any(two)) corners_inside(a.vol2, lin, gx, gxy, f2);
-#pragma unroll
-                    for (int e = 0; e < 12; ++e) {
-                        int ca = c_edge_a[e], cb = c_edge_b[e];
-                        vl[e][lane] = interp3(a.lo1, a.hi1, v[ca], v[cb], f1[ca], f1[cb], f2[ca],
-                                              f2[cb], a.lo2, a.hi2, fid[ca], fid[cb]);
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 12; ++e) {
-                        int ca = c_edge_a[e], cb = c_edge_b[e];
-                        vl[e][lane] =
-                            interp2(a.lo1, a.hi1, v[ca], v[cb], f1[ca], f1[cb], fid[ca], fid[cb]);
-                    }
+                for (int e = 0; e < 12; ++e) {
+                    int ca = c_edge_a[e], cb = c_edge_b[e];
+                    vl[e][lane] =
+                        interp2(a.lo1, a.hi1, v[ca], v[cb], f1[ca], f1[cb], fid[ca], fid[cb]);
                 }
             }
         }
@@ -892,17 +914,36 @@ __global__ void __launch_bounds__(64) generate_kernel(GenArgs a) {
         const uint32_t total = __shfl(incl, 63, 64);
         s_first[lane] = first;
         s_base[lane] = vbase;
-        s_tri[lane] = *(const uint4 *)(a.tri + cube * 16);
+        s_tri[lane] = row;
         for (uint32_t j = 0; j < nv; ++j) owner[first + j] = (uint8_t)lane;
         __syncthreads();
-        for (uint32_t k = lane; k < total; k += 64) {
+        // the next batch's corners arrive and its table rows are asked for
+        cube = 0;
+        nv = 0;
+        vbase = nvbase;
+        gp = ngp;
+        lin = nlin;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            fid[k] = nid[k];
+            f1[k] = n1[k];
+            asm volatile("" : "+v"(fid[k]), "+v"(f1[k]));
+        }
+        if (more) {
+            cube = cube_of(fid, a.iso);
+            nv = a.nverts[cube];
+            row = *(const uint4 *)(a.tri + cube * 16);
+        }
+        // (stores start on a line boundary: 8 vertices of 16 bytes)
+        for (uint32_t k = lane - (s_base[0] & 7u); (int)k < (int)total; k += 64) {
+            if ((int)k < 0) continue;
             const uint32_t o = owner[k];
             const uint32_t j = k - s_first[o];
             const uint32_t t0 = j - j % 3u;  // the triangle's first vertex
-            const uint8_t *row = (const uint8_t *)&s_tri[o];
-            const float3 a0 = vl[row[t0]][o];
-            const float3 a1 = vl[row[t0 + 1]][o];
-            const float3 a2 = vl[row[t0 + 2]][o];
+            const uint8_t *edge = (const uint8_t *)&s_tri[o];
+            const float3 a0 = vl[edge[t0]][o];
+            const float3 a1 = vl[edge[t0 + 1]][o];
+            const float3 a2 = vl[edge[t0 + 2]][o];
             const float3 e0 = make_float3(a1.x - a0.x, a1.y - a0.y, a1.z - a0.z);
             const float3 e1 = make_float3(a2.x - a0.x, a2.y - a0.y, a2.z - a0.z);
             const float3 n = cross3(e0, e1);
