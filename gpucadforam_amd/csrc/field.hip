@@ -149,10 +149,75 @@ Rows euler_rows(gc_float3 a) {
     return r;
 }
 
+// Points are taken in runs of kRunPoints per workgroup: kRun per thread, 256
+// apart.  The run's first point is decoded once (in 32 bits where they hold
+// it), a thread's first from it, and the rest by steps with one carry per
+// axis.
+constexpr int kRun = 8;
+constexpr uint32_t kRunPoints = 256 * kRun;
+
+struct PointSteps {
+    uint32_t nx, ny;
+    uint32_t dx, dy, dz;  // `step` points as steps along x, y, z
+};
+
+PointSteps point_steps(int nx, int ny, uint32_t step) {
+    PointSteps s;
+    const uint64_t plane = (uint64_t)nx * ny;
+    s.nx = (uint32_t)nx;
+    s.ny = (uint32_t)ny;
+    s.dz = (uint32_t)(step / plane);
+    s.dy = (uint32_t)(step % plane / (uint64_t)nx);
+    s.dx = (uint32_t)(step % plane % (uint64_t)nx);
+    return s;
+}
+
+struct Point {
+    uint32_t x, y, z;
+    // point `first` + `ahead` (first: the same in every lane)
+    __device__ __forceinline__ Point(const PointSteps &s, uint64_t first, uint32_t ahead) {
+        const uint64_t plane = (uint64_t)s.nx * s.ny;
+        if (((first | plane) >> 32) == 0) {
+            z = (uint32_t)first / (uint32_t)plane;
+            const uint32_t rem = (uint32_t)first - z * (uint32_t)plane;
+            y = rem / s.nx;
+            x = rem - y * s.nx;
+        } else {
+            const uint64_t zb = first / plane, rem = first - zb * plane, yb = rem / s.nx;
+            z = (uint32_t)zb;
+            y = (uint32_t)yb;
+            x = (uint32_t)(rem - yb * s.nx);
+        }
+        // x, y < 2^31 and `ahead` is small: no sum wraps
+        x += ahead;
+        const uint32_t rows = x / s.nx;
+        x -= rows * s.nx;
+        y += rows;
+        const uint32_t planes = y / s.ny;
+        y -= planes * s.ny;
+        z += planes;
+    }
+    __device__ __forceinline__ void advance(const PointSteps &s, uint32_t dx, uint32_t dy,
+                                            uint32_t dz) {
+        x += dx;
+        y += dy;
+        z += dz;
+        if (x >= s.nx) {
+            x -= s.nx;
+            ++y;
+        }
+        if (y >= s.ny) {
+            y -= s.ny;
+            ++z;
+        }
+    }
+};
+
 struct Grid3 {
     int nx, ny, nz;
     float dx, dy, dz;
     float mx, my, mz;  // (N-1)/2.0
+    PointSteps s;
 };
 
 Grid3 make_grid(int nx, int ny, int nz, float dx, float dy, float dz) {
@@ -162,19 +227,26 @@ Grid3 make_grid(int nx, int ny, int nz, float dx, float dy, float dz) {
     g.mx = (float)((nx - 1) / 2.0);
     g.my = (float)((ny - 1) / 2.0);
     g.mz = (float)((nz - 1) / 2.0);
+    g.s = point_steps(nx, ny, 256);
     return g;
 }
 
-__device__ __forceinline__ bool grid_point(const Grid3 &g, uint64_t &i, int &xx, int &yy, int &zz) {
-    i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    uint64_t n = (uint64_t)g.nx * g.ny * g.nz;
-    if (i >= n) return false;
-    uint64_t plane = (uint64_t)g.nx * g.ny;
-    zz = (int)(i / plane);
-    uint64_t rem = i - (uint64_t)zz * plane;
-    yy = (int)(rem / g.nx);
-    xx = (int)(rem - (uint64_t)yy * g.nx);
-    return true;
+// fn(i, x, y, z) for the points of this thread.  A primitive is bound by the
+// 4 bytes that it writes per point once the point's coordinates cost little:
+// cuboid on 211 x 193 x 229 25.2 us with a 64-bit division per point and axis,
+// 18.0 so.
+template <class F>
+__device__ __forceinline__ void for_points(const Grid3 &g, F fn) {
+    const uint64_t n = (uint64_t)g.nx * g.ny * g.nz, first = (uint64_t)blockIdx.x * kRunPoints;
+    Point p(g.s, first, threadIdx.x);
+    uint64_t i = first + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) {
+        if (i >= n) return;
+        fn(i, (int)p.x, (int)p.y, (int)p.z);
+        p.advance(g.s, g.s.dx, g.s.dy, g.s.dz);
+        i += 256;
+    }
 }
 
 __device__ __forceinline__ float3 centred(const Grid3 &g, int xx, int yy, int zz, float3 c) {
@@ -187,127 +259,127 @@ __device__ __forceinline__ float dot_rows(float3 v, float3 r) {
 }
 
 __global__ void sphere_kernel(Grid3 g, float *out, float3 c, float radius, float thick, int shell) {
-    uint64_t i; int xx, yy, zz;
-    if (!grid_point(g, i, xx, yy, zz)) return;
-    float3 v = centred(g, xx, yy, zz, c);
-    float t_diff = (float)(thick / 2.0);
-    float r2 = v.x * v.x + v.y * v.y + v.z * v.z;
-    if (shell) {
-        float ri = radius - t_diff, ro = radius + t_diff;
-        float f1 = r2 - ri * ri;
-        float f2 = r2 - ro * ro;
-        out[i] = (float)fmax((double)f1 * -1.0, (double)f2);
-    } else {
-        out[i] = r2 - radius * radius;
-    }
+    for_points(g, [&](uint64_t i, int xx, int yy, int zz) {
+        float3 v = centred(g, xx, yy, zz, c);
+        float t_diff = (float)(thick / 2.0);
+        float r2 = v.x * v.x + v.y * v.y + v.z * v.z;
+        if (shell) {
+            float ri = radius - t_diff, ro = radius + t_diff;
+            float f1 = r2 - ri * ri;
+            float f2 = r2 - ro * ro;
+            out[i] = (float)fmax((double)f1 * -1.0, (double)f2);
+        } else {
+            out[i] = r2 - radius * radius;
+        }
+    });
 }
 
 __global__ void cuboid_kernel(Grid3 g, float *out, float3 c, Rows R, float xw, float yw, float zw) {
-    uint64_t i; int xx, yy, zz;
-    if (!grid_point(g, i, xx, yy, zz)) return;
-    float3 v = centred(g, xx, yy, zz, c);
-    float f1 = fabsf(dot_rows(v, R.x)) - xw;
-    float f2 = fabsf(dot_rows(v, R.y)) - yw;
-    float f3 = fabsf(dot_rows(v, R.z)) - zw;
-    out[i] = fmaxf(fmaxf(f1, f2), f3);
+    for_points(g, [&](uint64_t i, int xx, int yy, int zz) {
+        float3 v = centred(g, xx, yy, zz, c);
+        float f1 = fabsf(dot_rows(v, R.x)) - xw;
+        float f2 = fabsf(dot_rows(v, R.y)) - yw;
+        float f3 = fabsf(dot_rows(v, R.z)) - zw;
+        out[i] = fmaxf(fmaxf(f1, f2), f3);
+    });
 }
 
 __global__ void cuboid_shell_kernel(Grid3 g, float *out, float3 c, Rows R, float xw, float yw,
                                     float zw, float thick) {
-    uint64_t i; int xx, yy, zz;
-    if (!grid_point(g, i, xx, yy, zz)) return;
-    float3 v = centred(g, xx, yy, zz, c);
-    float f1 = dot_rows(v, R.x);
-    float f11 = fabsf(f1) - xw;
-    float f12 = fabsf(f1) - (xw - thick);
-    float f2 = dot_rows(v, R.y);
-    float f21 = fabsf(f2) - yw;
-    float f22 = fabsf(f2) - (yw - thick);
-    float f3 = fabsf(dot_rows(v, R.z)) - zw;
-    double inner = (double)fmaxf(f12, f22) * -1.0;
-    out[i] = (float)fmax(fmax((double)fmaxf(f11, f21), inner), (double)f3);
+    for_points(g, [&](uint64_t i, int xx, int yy, int zz) {
+        float3 v = centred(g, xx, yy, zz, c);
+        float f1 = dot_rows(v, R.x);
+        float f11 = fabsf(f1) - xw;
+        float f12 = fabsf(f1) - (xw - thick);
+        float f2 = dot_rows(v, R.y);
+        float f21 = fabsf(f2) - yw;
+        float f22 = fabsf(f2) - (yw - thick);
+        float f3 = fabsf(dot_rows(v, R.z)) - zw;
+        double inner = (double)fmaxf(f12, f22) * -1.0;
+        out[i] = (float)fmax(fmax((double)fmaxf(f11, f21), inner), (double)f3);
+    });
 }
 
 __global__ void pyramid_kernel(Grid3 g, float *out, float3 c, Rows R, float xwb, float xwt,
                                float yh, float zwb, float zwt) {
-    uint64_t i; int xx, yy, zz;
-    if (!grid_point(g, i, xx, yy, zz)) return;
-    float3 v = centred(g, xx, yy, zz, c);
-    float f1 = dot_rows(v, R.x);
-    float f2 = dot_rows(v, R.y);
-    float f3 = dot_rows(v, R.z);
-    float ratio = (yh - f2) / yh;
-    float xw = ratio * (xwb - xwt) + xwt;
-    f1 = fabsf(f1) - xw;
-    f2 = fabsf(f2 - yh / 2) - yh / 2;
-    float zw = ratio * (zwb - zwt) + zwt;
-    f3 = fabsf(f3) - zw;
-    out[i] = fmaxf(fmaxf(f1, f2), f3);
+    for_points(g, [&](uint64_t i, int xx, int yy, int zz) {
+        float3 v = centred(g, xx, yy, zz, c);
+        float f1 = dot_rows(v, R.x);
+        float f2 = dot_rows(v, R.y);
+        float f3 = dot_rows(v, R.z);
+        float ratio = (yh - f2) / yh;
+        float xw = ratio * (xwb - xwt) + xwt;
+        f1 = fabsf(f1) - xw;
+        f2 = fabsf(f2 - yh / 2) - yh / 2;
+        float zw = ratio * (zwb - zwt) + zwt;
+        f3 = fabsf(f3) - zw;
+        out[i] = fmaxf(fmaxf(f1, f2), f3);
+    });
 }
 
 __global__ void torus_kernel(Grid3 g, float *out, float3 c, Rows R, float tr, float cr) {
-    uint64_t i; int xx, yy, zz;
-    if (!grid_point(g, i, xx, yy, zz)) return;
-    float3 v = centred(g, xx, yy, zz, c);
-    float vx = dot_rows(v, R.x), vy = dot_rows(v, R.y), vz = dot_rows(v, R.z);
-    float side = tr - __builtin_sqrtf(vx * vx + vy * vy);
-    out[i] = vz * vz - cr * cr + side * side;
+    for_points(g, [&](uint64_t i, int xx, int yy, int zz) {
+        float3 v = centred(g, xx, yy, zz, c);
+        float vx = dot_rows(v, R.x), vy = dot_rows(v, R.y), vz = dot_rows(v, R.z);
+        float side = tr - __builtin_sqrtf(vx * vx + vy * vy);
+        out[i] = vz * vz - cr * cr + side * side;
+    });
 }
 
 __global__ void cone_kernel(Grid3 g, float *out, float3 c, Rows R, float br, float h) {
-    uint64_t i; int xx, yy, zz;
-    if (!grid_point(g, i, xx, yy, zz)) return;
-    float3 v = centred(g, xx, yy, zz, c);
-    float q = h / br;
-    float f2 = q * q;
-    float vx = dot_rows(v, R.x), vy = dot_rows(v, R.y), vz = dot_rows(v, R.z);
-    float gg = (float)((double)vy - (double)h / 2.0);
-    float hh = (float)fmax(((double)gg - (double)h / 2.0) * 100.0,
-                           ((double)gg + (double)h / 2.0) * 100.0 * -1.0);
-    float d = vy - h;
-    float f1 = ((vx * vx + vz * vz) * f2) - d * d;
-    out[i] = fmaxf(f1, hh);
+    for_points(g, [&](uint64_t i, int xx, int yy, int zz) {
+        float3 v = centred(g, xx, yy, zz, c);
+        float q = h / br;
+        float f2 = q * q;
+        float vx = dot_rows(v, R.x), vy = dot_rows(v, R.y), vz = dot_rows(v, R.z);
+        float gg = (float)((double)vy - (double)h / 2.0);
+        float hh = (float)fmax(((double)gg - (double)h / 2.0) * 100.0,
+                               ((double)gg + (double)h / 2.0) * 100.0 * -1.0);
+        float d = vy - h;
+        float f1 = ((vx * vx + vz * vz) * f2) - d * d;
+        out[i] = fmaxf(f1, hh);
+    });
 }
 
 __global__ void cone_frustum_kernel(Grid3 g, float *out, float3 c, Rows R, float tr, float br,
                                     float h) {
-    uint64_t i; int xx, yy, zz;
-    if (!grid_point(g, i, xx, yy, zz)) return;
-    float3 v = centred(g, xx, yy, zz, c);
-    float vx = dot_rows(v, R.x), vy = dot_rows(v, R.y), vz = dot_rows(v, R.z);
-    float r_diff = ((h - vy) / h) * (br - tr);
-    float gg = (float)((double)vy - (double)h / 2.0);
-    float hh = (float)fmax(((double)gg - (double)h / 2.0) * 100.0,
-                           ((double)gg + (double)h / 2.0) * 100.0 * -1.0);
-    double rr = (double)(r_diff + tr);
-    float f1 = (float)((double)(vx * vx + vz * vz) - rr * rr);
-    out[i] = fmaxf(f1, hh);
+    for_points(g, [&](uint64_t i, int xx, int yy, int zz) {
+        float3 v = centred(g, xx, yy, zz, c);
+        float vx = dot_rows(v, R.x), vy = dot_rows(v, R.y), vz = dot_rows(v, R.z);
+        float r_diff = ((h - vy) / h) * (br - tr);
+        float gg = (float)((double)vy - (double)h / 2.0);
+        float hh = (float)fmax(((double)gg - (double)h / 2.0) * 100.0,
+                               ((double)gg + (double)h / 2.0) * 100.0 * -1.0);
+        double rr = (double)(r_diff + tr);
+        float f1 = (float)((double)(vx * vx + vz * vz) - rr * rr);
+        out[i] = fmaxf(f1, hh);
+    });
 }
 
 __global__ void line_kernel(Grid3 g, float *out, float3 c, float3 axis, float radius, float t_diff,
                             float t_diff_ax, int cyl) {
-    uint64_t i; int xx, yy, zz;
-    if (!grid_point(g, i, xx, yy, zz)) return;
-    float x1 = ((float)xx - g.mx) * g.dx;
-    float y1 = ((float)yy - g.my) * g.dy;
-    float z1 = ((float)zz - g.mz) * g.dz;
-    float3 end = make_float3(axis.x + c.x, axis.y + c.y, axis.z + c.z);
-    float3 w1 = make_float3(x1 - c.x, y1 - c.y, z1 - c.z);
-    float3 w2 = make_float3(x1 - end.x, y1 - end.y, z1 - end.z);
-    float3 w3 = make_float3(end.x - c.x, end.y - c.y, end.z - c.z);
-    float3 d = make_float3(w1.y * w2.z - w1.z * w2.y, w1.z * w2.x - w1.x * w2.z,
-                           w1.x * w2.y - w1.y * w2.x);
-    float e = __builtin_sqrtf(d.x * d.x + d.y * d.y + d.z * d.z);
-    float dis = __builtin_sqrtf(w3.x * w3.x + w3.y * w3.y + w3.z * w3.z);
-    float f = e / dis;
-    float gg = (x1 - c.x) * axis.x + (y1 - c.y) * axis.y + (z1 - c.z) * axis.z;
-    float f1 = fmaxf(gg - t_diff_ax, (gg + t_diff_ax) * -1.0f);
-    float f2;
-    if (cyl)
-        f2 = fmaxf(f - (radius + t_diff), (f - (radius - t_diff)) * -1.0f);
-    else
-        f2 = f - radius;
-    out[i] = fmaxf(f1, f2);
+    for_points(g, [&](uint64_t i, int xx, int yy, int zz) {
+        float x1 = ((float)xx - g.mx) * g.dx;
+        float y1 = ((float)yy - g.my) * g.dy;
+        float z1 = ((float)zz - g.mz) * g.dz;
+        float3 end = make_float3(axis.x + c.x, axis.y + c.y, axis.z + c.z);
+        float3 w1 = make_float3(x1 - c.x, y1 - c.y, z1 - c.z);
+        float3 w2 = make_float3(x1 - end.x, y1 - end.y, z1 - end.z);
+        float3 w3 = make_float3(end.x - c.x, end.y - c.y, end.z - c.z);
+        float3 d = make_float3(w1.y * w2.z - w1.z * w2.y, w1.z * w2.x - w1.x * w2.z,
+                               w1.x * w2.y - w1.y * w2.x);
+        float e = __builtin_sqrtf(d.x * d.x + d.y * d.y + d.z * d.z);
+        float dis = __builtin_sqrtf(w3.x * w3.x + w3.y * w3.y + w3.z * w3.z);
+        float f = e / dis;
+        float gg = (x1 - c.x) * axis.x + (y1 - c.y) * axis.y + (z1 - c.z) * axis.z;
+        float f1 = fmaxf(gg - t_diff_ax, (gg + t_diff_ax) * -1.0f);
+        float f2;
+        if (cyl)
+            f2 = fmaxf(f - (radius + t_diff), (f - (radius - t_diff)) * -1.0f);
+        else
+            f2 = f - radius;
+        out[i] = fmaxf(f1, f2);
+    });
 }
 
 // Fft_lattice::create_lattice unit-cell forms (src/lattice_files/Fft_lattice.cu:12-66).
@@ -348,68 +420,115 @@ __global__ void unit_lattice_kernel(float *out, uint32_t nx, uint32_t ny, uint32
 }
 
 // ---- normalise_four: min/max (seeded with 0) then band indicator
-__global__ void minmax_partial_kernel(const float *in, uint64_t n, float2 *partial) {
-    __shared__ float smin[256], smax[256];
-    float lo = 0.f, hi = 0.f;  // the reference's second pass seeds with 0
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x) {
-        float v = in[i];
-        lo = fminf(lo, v);
-        hi = fmaxf(hi, v);
+// A workgroup's min and max into thread 0 (lo, hi: the thread's own).
+__device__ __forceinline__ void block_minmax(float &lo, float &hi) {
+    __shared__ float smin[4], smax[4];
+    for (int d = 32; d > 0; d >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, d, 64));
+        hi = fmaxf(hi, __shfl_xor(hi, d, 64));
     }
-    smin[threadIdx.x] = lo;
-    smax[threadIdx.x] = hi;
+    if ((threadIdx.x & 63) == 0) {
+        smin[threadIdx.x >> 6] = lo;
+        smax[threadIdx.x >> 6] = hi;
+    }
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            smin[threadIdx.x] = fminf(smin[threadIdx.x], smin[threadIdx.x + s]);
-            smax[threadIdx.x] = fmaxf(smax[threadIdx.x], smax[threadIdx.x + s]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = make_float2(smin[0], smax[0]);
+    lo = fminf(fminf(smin[0], smin[1]), fminf(smin[2], smin[3]));
+    hi = fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3]));
 }
 
-__global__ void minmax_final_kernel(float2 *partial, int nparts) {
-    __shared__ float smin[256], smax[256];
+// Bound by the bytes read, with eight loads per thread under way (one load
+// per iteration before: 240^3 19.5 us, now 11.2).
+__global__ void __launch_bounds__(256) minmax_partial_kernel(const float *in, uint64_t n,
+                                                             float2 *partial) {
+    float lo = 0.f, hi = 0.f;  // the reference's second pass seeds with 0
+    const uint64_t stride = (uint64_t)gridDim.x * 256;
+    uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    for (; i + 7 * stride < n; i += 8 * stride) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = in[i + k * stride];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            lo = fminf(lo, v[k]);
+            hi = fmaxf(hi, v[k]);
+        }
+    }
+    for (; i < n; i += stride) {
+        lo = fminf(lo, in[i]);
+        hi = fmaxf(hi, in[i]);
+    }
+    block_minmax(lo, hi);
+    if (threadIdx.x == 0) partial[blockIdx.x] = make_float2(lo, hi);
+}
+
+__global__ void __launch_bounds__(256) minmax_final_kernel(float2 *partial, int nparts) {
     float lo = 0.f, hi = 0.f;
-    for (int i = threadIdx.x; i < nparts; i += blockDim.x) {
+    for (int i = threadIdx.x; i < nparts; i += 256) {
         lo = fminf(lo, partial[i].x);
         hi = fmaxf(hi, partial[i].y);
     }
-    smin[threadIdx.x] = lo;
-    smax[threadIdx.x] = hi;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            smin[threadIdx.x] = fminf(smin[threadIdx.x], smin[threadIdx.x + s]);
-            smax[threadIdx.x] = fmaxf(smax[threadIdx.x], smax[threadIdx.x + s]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[0] = make_float2(smin[0], smax[0]);
+    block_minmax(lo, hi);
+    if (threadIdx.x == 0) partial[0] = make_float2(lo, hi);
 }
 
-__global__ void band_kernel(const float *in, float *indicator, float *normalised, const float2 *ab,
-                            int nx, int ny, int nz, float iso1, float iso2) {
-    uint64_t tx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    uint64_t size = (uint64_t)nx * ny * nz;
-    if (tx >= size) return;
-    float a = ab->x, b = ab->y;
-    int xx = (int)(tx % (uint64_t)nx);
-    int yy = (int)((tx % ((uint64_t)nx * ny)) / (uint64_t)nx);
-    int zz = (int)(tx / ((uint64_t)nx * ny));
-    float k = in[tx];
-    k = (k - a) / (b - a);
-    float m;
-    if (xx == 0 || xx == nx - 1 || yy == 0 || yy == ny - 1 || zz == 0 || zz == nz - 1) {
-        m = 0.f;
-        k = 0.f;
-    } else {
-        m = (k >= iso1 && k <= iso2) ? 1.f : 0.f;
+// Points in fours, kBandFours per thread; VEC: the three arrays are 16-byte
+// aligned.  Bound by the 12 bytes per point: 240^3 40.5 us with 64-bit
+// divisions per point, 26.4 so.
+constexpr int kBandFours = 4;
+constexpr uint32_t kBandPoints = 1024 * kBandFours;
+
+template <bool VEC>
+__global__ void __launch_bounds__(256) band_kernel(const float *in, float *indicator,
+                                                   float *normalised, const float2 *ab,
+                                                   PointSteps s, uint32_t nz, float iso1,
+                                                   float iso2) {
+    const uint64_t size = (uint64_t)s.nx * s.ny * nz;
+    const uint64_t first = (uint64_t)blockIdx.x * kBandPoints;
+    const float a = ab->x, b = ab->y;
+    Point p(s, first, 4 * threadIdx.x);
+    uint64_t i = first + 4 * threadIdx.x;
+    float v[kBandFours][4];
+#pragma unroll
+    for (int k = 0; k < kBandFours; ++k) {
+        const uint64_t j = i + 1024 * k;
+        if (VEC && j + 3 < size) {
+            const float4 q = *(const float4 *)(in + j);
+            v[k][0] = q.x;
+            v[k][1] = q.y;
+            v[k][2] = q.z;
+            v[k][3] = q.w;
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[k][c] = j + c < size ? in[j + c] : 0.f;
+        }
     }
-    indicator[tx] = m;
-    normalised[tx] = k;
+#pragma unroll
+    for (int k = 0; k < kBandFours; ++k) {
+        const uint64_t j = i + 1024 * k;
+        float m[4], t[4];
+        Point q = p;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const bool face = q.x == 0 || q.x == s.nx - 1 || q.y == 0 || q.y == s.ny - 1 ||
+                              q.z == 0 || q.z == nz - 1;
+            const float f = (v[k][c] - a) / (b - a);
+            m[c] = !face && f >= iso1 && f <= iso2 ? 1.f : 0.f;
+            t[c] = face ? 0.f : f;
+            q.advance(s, 1, 0, 0);
+        }
+        p.advance(s, s.dx, s.dy, s.dz);
+        if (VEC && j + 3 < size) {
+            *(float4 *)(indicator + j) = make_float4(m[0], m[1], m[2], m[3]);
+            *(float4 *)(normalised + j) = make_float4(t[0], t[1], t[2], t[3]);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (j + c < size) {
+                    indicator[j + c] = m[c];
+                    normalised[j + c] = t[c];
+                }
+        }
+    }
 }
 
 __global__ void primitive_dynamic_kernel(const float *active, float *iso, uint64_t n) {
@@ -423,11 +542,11 @@ __global__ void primitive_fixed_kernel(const int4 *fixed, float *iso, uint64_t n
     if (i < n && fixed[i].x > -1) iso[i] = FLT_MAX;
 }
 
-int point_launch(int nx, int ny, int nz, dim3 *grid) {
+int point_launch(int nx, int ny, int nz, dim3 *grid, uint32_t per_block = 256) {
     GC_ARG(nx >= 1 && ny >= 1 && nz >= 1, "grid sizes must be positive");
     uint64_t n = (uint64_t)nx * ny * nz;
-    uint64_t blocks = (n + 255) / 256;
-    GC_ARG(blocks <= 0x7fffffffull, "grid too large");
+    GC_ARG((n + 255) / 256 <= 0x7fffffffull, "grid too large");
+    uint64_t blocks = (n + per_block - 1) / per_block;
     *grid = dim3((unsigned)blocks);
     return GPUCAD_OK;
 }
@@ -489,7 +608,7 @@ int gpucad_create_lattice(float *d, uint32_t nx, uint32_t ny, uint32_t nz, uint3
     GC_ARG(ptr, "output is NULL");                              \
     dim3 grid;                                                  \
     {                                                           \
-        int st_ = point_launch(nx, ny, nz, &grid);              \
+        int st_ = point_launch(nx, ny, nz, &grid, kRunPoints);  \
         if (st_) return st_;                                    \
     }                                                           \
     Grid3 g = make_grid(nx, ny, nz, dx, dy, dz);
@@ -605,9 +724,12 @@ int gpucad_normalise_four(const float *in, float *indicator, float *normalised, 
     GC_CHECK_LAUNCH();
     hipLaunchKernelGGL(minmax_final_kernel, dim3(1), dim3(256), 0, 0, part, nparts);
     GC_CHECK_LAUNCH();
-    dim3 grid((unsigned)((size + 255) / 256));
-    hipLaunchKernelGGL(band_kernel, grid, dim3(256), 0, 0, in, indicator, normalised, part, nx, ny,
-                       nz, iso1, iso2);
+    const uint64_t blocks = (size + kBandPoints - 1) / kBandPoints;
+    GC_ARG(blocks <= 0x7fffffffull, "grid too large");
+    const bool vec = (((uintptr_t)in | (uintptr_t)indicator | (uintptr_t)normalised) & 15) == 0;
+    hipLaunchKernelGGL(vec ? band_kernel<true> : band_kernel<false>, dim3((unsigned)blocks),
+                       dim3(256), 0, 0, in, indicator, normalised, part,
+                       point_steps(nx, ny, 1024), (uint32_t)nz, iso1, iso2);
     GC_CHECK_LAUNCH();
     GC_HIP(hipStreamSynchronize(0));
     return GPUCAD_OK;
