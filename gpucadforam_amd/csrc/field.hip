@@ -30,8 +30,15 @@ namespace {
 // keeps small grids spread over more workgroups.
 constexpr int rows_per_lane(bool rot) { return rot ? 4 : 1; }
 
+// Bound by its vector instructions, near the field's write rate: 512^3 with
+// every option 163 -> 158 us, 1024^3 bent 814 -> 762, a 203 x 149 x 181 part
+// 49 -> 44 after its instructions were cut (constants in vector registers, the
+// root by v_rsq and one correction, its range tested per column instead of
+// per point, sign words by v_writelane).  Seven waves per SIMD: the rotated
+// diamond's 74 registers hold six otherwise (512^3: 216 us, 208 so); with modes
+// and a box that would take a scratch store per step.
 template <bool ROT, int TPMS, bool THICK, int PRIM, int OP>
-__global__ void __launch_bounds__(64 * kFieldWaves)
+__global__ void __launch_bounds__(64 * kFieldWaves, !ROT ? 8 : (THICK && PRIM == GC_PRIM_BOX ? 6 : 7))
 lattice_field_kernel(FieldConsts c, float *__restrict__ field, uint64_t *__restrict__ signs) {
     __shared__ float ztab[kMaxLZ * kZTab];
     constexpr int RY = rows_per_lane(ROT);

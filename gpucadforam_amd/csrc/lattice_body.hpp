@@ -48,6 +48,7 @@ struct FieldConsts {
     int group_mask;               // bit k set when some mode has kz == k
     int prim, op;
     float pc[3], pr, ph[3];
+    int prim_plain;               // every squared distance stays below 2^96
 };
 
 // Field variant: which template instance evaluates a grid.
@@ -111,6 +112,9 @@ inline FieldConsts make_field_consts(const gc_lattice_params *p, float iso, int 
         c.ph[a] = p->prim_half[a];
     }
     c.pr = p->prim_radius;
+    c.prim_plain = 1;  // (false for NaN)
+    for (int a = 0; a < 3; ++a)
+        if (!(std::fabs(c.pc[a]) <= 0x1p40f && std::fabs(c.ph[a]) <= 0x1p40f)) c.prim_plain = 0;
     return c;
 }
 
@@ -166,6 +170,9 @@ constexpr uint32_t kPastPlane = 0xfffffff0u;
 constexpr int kStoreNonTemporal = 2;
 typedef uint32_t U32x2 __attribute__((ext_vector_type(2)));
 
+// v_writelane: `old` with lane `lane`'s value replaced by the scalar `v`
+__device__ int write_lane(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+
 // Primitive of a lattice field known at compile time (PRIM_ANY: read from
 // the constants at run time).
 constexpr int PRIM_ANY = -1;
@@ -173,11 +180,11 @@ constexpr int PRIM_ANY = -1;
 // The lattice value g combined with the primitive whose distance root is
 // `root` (sphere: root - r; box: root + min(max(partial, z term), 0)).
 template <int PRIM, int OP>
-__device__ __forceinline__ float prim_op(const FieldConsts &c, float g, float root, float pz,
-                                         float pbxy) {
+__device__ __forceinline__ float prim_op(const FieldConsts &c, float pr, float g, float root,
+                                         float pz, float pbxy) {
     const int prim = PRIM == PRIM_ANY ? c.prim : PRIM;
     const float s = prim == GC_PRIM_SPHERE
-                        ? root - c.pr
+                        ? root - pr
                         : root + __builtin_fminf(__builtin_fmaxf(pbxy, pz), 0.f);
     const int op = OP == PRIM_ANY ? c.op : OP;
     const float gi = __builtin_fmaxf(g, s), gu = __builtin_fminf(g, s), gs = __builtin_fmaxf(g, -s);
@@ -213,6 +220,7 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
     const int zn = min(c.lz, c.nz - z0);
 
     // ---- per-z table (one z per thread)
+    bool ztiny = false;  // a box's z distance in (0, 2^-48)
     for (int i = threadIdx.x; i < zn; i += 64 * kFieldWaves) {
         float *e = ztab + i * kZTab;
         float zf = (float)(z0 + i);
@@ -238,10 +246,12 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
         if (c.prim == GC_PRIM_SPHERE) {
             e[ZT_PRIMZ] = pz - c.pc[2];
         } else if (c.prim == GC_PRIM_BOX) {
-            e[ZT_PRIMZ] = __builtin_fabsf(pz - c.pc[2]) - c.ph[2];
+            const float bz = __builtin_fabsf(pz - c.pc[2]) - c.ph[2];
+            e[ZT_PRIMZ] = bz;
+            ztiny |= bz > 0.f && bz < 0x1p-48f;
         }
     }
-    __syncthreads();
+    const bool any_ztiny = __syncthreads_or(ztiny);
     const bool xin = x < c.nx;
 
     // ---- per-lane x quantities
@@ -364,6 +374,37 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
     // lanes whose point lies in the grid (the sign mask keeps only these)
     const uint64_t in_mask = __ballot(xin);
 
+    // The primitive's squared distances lie in [2^-96, 2^96) (a box's may be 0
+    // too) unless a column passes within 2^-48 of its centre, edge or corner
+    // axis: then the wave takes the general root at every point.
+    const int prim = PRIM == PRIM_ANY ? c.prim : PRIM;
+    bool general = !c.prim_plain || any_ztiny;
+    if (prim != GC_PRIM_NONE) {
+        bool near = false;
+#pragma unroll
+        for (int r = 0; r < RY; ++r)
+            near |= !(pxy[r] >= 0x1p-96f) && !(prim == GC_PRIM_BOX && pxy[r] == 0.0f);
+        general |= __ballot(near) != 0;
+    }
+    // a sheet takes |f| - t; otherwise nothing is masked and t is 0
+    uint32_t fmask = c.sheet ? 0x7fffffffu : ~0u;
+    asm volatile("" : "+v"(fmask));
+    if (!c.sheet) {
+#pragma unroll
+        for (int r = 0; r < RY; ++r) {
+            T0[r] = 0.f;
+            S1[r] = S2[r] = S3[r] = Cplx{0.f, 0.f};
+        }
+    }
+    const float quarter = pinned(0.25f), pr = pinned(c.pr);
+    // the lanes that store sign words: lane r stores row r's
+    uint32_t moff = kPastPlane;
+    if (BX == 64) {
+#pragma unroll
+        for (int r = 0; r < RY; ++r)
+            if (signs != nullptr && lane == r && yin[r]) moff = soff[r] + 8u * (uint32_t)(x0 >> 6);
+    }
+
     for (int i = 0; i < zn; ++i) {
         const float *e = ztab + i * kZTab;
         // (x, z) work, shared by the lane's rows
@@ -373,10 +414,10 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
             sth = e[ZT_STH];
             Zr = e[ZT_ZF] * inv_p;
             if (TPMS == GC_TPMS_SCHWARZ_P) {
-                cZ = cos_rev(Zr);
+                cZ = cos_rev(Zr, quarter);
             } else {
                 sZ = sin_rev(Zr);
-                cZ = cos_rev(Zr);
+                cZ = cos_rev(Zr, quarter);
             }
         } else {
             if (c.uniform_period) {
@@ -384,7 +425,7 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
                 sZ = e[ZT_SZ];
             } else {
                 const float Z = e[ZT_ZF] * inv_p;
-                cZ = cos_rev(Z);
+                cZ = cos_rev(Z, quarter);
                 sZ = sin_rev(Z);
             }
         }
@@ -393,13 +434,11 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
 #pragma unroll
             for (int q = 0; q < 6; ++q) E[q] = e[ZT_E1 + q];
         }
-        const int prim = PRIM == PRIM_ANY ? c.prim : PRIM;
         const float pz = prim != GC_PRIM_NONE ? e[ZT_PRIMZ] : 0.f;
         // every row's value first (straight-line code, so the rows' independent
         // chains interleave), then the stores, which are guarded per row
         float gv[RY];
         float gl[RY], px2[RY];  // the lattice value and the primitive's squared distance
-        bool small = false;     // a squared distance in (0, 2^-96) (or NaN)
 #pragma unroll
         for (int r = 0; r < RY; ++r) {
             float f;
@@ -407,9 +446,9 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
                 float X = __builtin_fmaf(cth, dxP, __builtin_fmaf(-sth, dyP[r], cxP));
                 float Y = __builtin_fmaf(sth, dxP, __builtin_fmaf(cth, dyP[r], cyP));
                 if (TPMS == GC_TPMS_SCHWARZ_P) {
-                    f = (cos_rev(X) + cos_rev(Y)) + cZ;
+                    f = (cos_rev(X, quarter) + cos_rev(Y, quarter)) + cZ;
                 } else {
-                    float sx = sin_rev(X), cx = cos_rev(X), sy = sin_rev(Y), cy = cos_rev(Y);
+                    float sx = sin_rev(X), cx = cos_rev(X, quarter), sy = sin_rev(Y), cy = cos_rev(Y, quarter);
                     if (TPMS == GC_TPMS_GYROID)
                         f = __builtin_fmaf(sZ, cx, __builtin_fmaf(sy, cZ, sx * cy));
                     else
@@ -434,26 +473,23 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
                 t = __builtin_fmaf(S3[r].re, E[4], t);
                 t = __builtin_fmaf(-S3[r].im, E[5], t);
             }
-            float g = c.sheet ? __builtin_fabsf(f) - t : f;
+            float g = __uint_as_float(__float_as_uint(f) & fmask) - t;
             gl[r] = g;
             px2[r] = 0.f;
             if (prim != GC_PRIM_NONE) {
                 const float mz = __builtin_fmaxf(pz, 0.f);
                 px2[r] = prim == GC_PRIM_SPHERE ? __builtin_fmaf(pz, pz, pxy[r])
                                                 : __builtin_fmaf(mz, mz, pxy[r]);
-                // exact zeros (a box's inside) are exact on the fast path too
-                small |= !(px2[r] >= 0x1p-96f) && px2[r] != 0.0f;
-                g = prim_op<PRIM, OP>(c, g, sqrt_rn_normal(px2[r]), pz, pbxy[r]);
+                const float root = PRIM == GC_PRIM_SPHERE ? sqrt_rn_plain<false>(px2[r])
+                                                          : sqrt_rn_plain<true>(px2[r]);
+                g = prim_op<PRIM, OP>(c, pr, g, root, pz, pbxy[r]);
             }
             gv[r] = g;
         }
-        // a squared distance in (0, 2^-96), a point within 2^-48 of the
-        // primitive's centre: the wave takes the rescaled root for every row
-        // (one uniform test per z step, after the rows' arithmetic)
-        if (prim != GC_PRIM_NONE && __ballot(small) != 0) {
+        if (prim != GC_PRIM_NONE && general) {
 #pragma unroll
             for (int r = 0; r < RY; ++r)
-                gv[r] = prim_op<PRIM, OP>(c, gl[r], sqrt_rn(px2[r]), pz, pbxy[r]);
+                gv[r] = prim_op<PRIM, OP>(c, pr, gl[r], sqrt_rn(px2[r]), pz, pbxy[r]);
         }
         if (BX == 64) {
             // buffer stores over this z plane: a lane whose point lies outside
@@ -477,16 +513,14 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
                 const __amdgpu_buffer_rsrc_t sr =
                     __builtin_amdgcn_make_buffer_rsrc(splane + (uint64_t)i * sstep, (short)0,
                                                       (int)(uint32_t)sstep, kBufferWord3);
-                uint64_t mine = 0;
-                uint32_t moff = kPastPlane;
+                int lo = 0, hi = 0;
 #pragma unroll
                 for (int r = 0; r < RY; ++r) {
                     const uint64_t m = __builtin_amdgcn_fcmpf(gv[r], c.iso, 4) & in_mask;
-                    const bool me = signs != nullptr && lane == r && yin[r];
-                    mine = me ? m : mine;
-                    moff = me ? soff[r] + 8u * (uint32_t)(x0 >> 6) : moff;
+                    lo = write_lane((int)(uint32_t)m, r, lo);
+                    hi = write_lane((int)(m >> 32), r, hi);
                 }
-                const U32x2 w = {(uint32_t)mine, (uint32_t)(mine >> 32)};
+                const U32x2 w = {(uint32_t)lo, (uint32_t)hi};
                 __builtin_amdgcn_raw_buffer_store_b64(w, sr, (int)moff, 0, 0);
             }
             continue;
