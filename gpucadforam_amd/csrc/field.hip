@@ -106,6 +106,33 @@ int validate_lattice(const gc_lattice_params *p) {
     return GPUCAD_OK;
 }
 
+// z planes per workgroup of the one-grid launch.  A long run spreads the
+// per-column work and the z table, a short one leaves more workgroups to fill
+// the chip and its last wave.  With w = columns of bricks x planes the best run
+// grew like sqrt(w) in sweeps from 33 x 47 x 61 to 1024^3 (rotated: 8 planes of
+// 128^3, 10 of 203 x 149 x 181, 20 of 320 x 300 x 310; bent or with modes: 8 of
+// 100^3, 20 of 200^3, 48 of 400^3, 80 of 512^3); 0.12 sqrt(w) is within 5 % of
+// each.  Large rotated grids, whose four rows per lane need more columns,
+// are faster when five workgroups per CU take all of it at once, in runs of
+// w / 1300 planes (512^3: 161 us in runs of 112, 173 of 47, 166 of 48: long
+// runs are multiples of 16).  A lattice with neither rotation, bend nor modes
+// has little per-column work and is fastest in runs of 16 from 200^3 on
+// (512^3: 90.6 us, 99 in runs of 32 to 80).  With an eighth of the planes (a
+// fifth when rotated) and at least 16, as before: 40^3 5.0 us, now 3.1; rotated
+// 128^3 31.9, now 17.5; 203 x 149 x 181 44.4, now 29.0; 320 x 300 x 310 76.9,
+// now 60.
+int default_z_run(const gc_lattice_params *p, int bricks_x, int bricks_y) {
+    const bool rot = p->rot0 != 0.f || p->rot1 != 0.f;
+    const bool plain = !rot && !(p->bend_radius > 0.f) && p->n_modes == 0;
+    const double w = (double)bricks_x * bricks_y * p->nz;
+    const double best = std::max(0.12 * std::sqrt(w), rot ? w / 1300.0 : 0.0);
+    int run = (int)std::min(std::max(best + 0.5, 4.0), plain ? 16.0 : (double)kMaxLZ);
+    run = std::max(run, (p->nz + 65534) / 65535);  // (a launch's third dimension)
+    if (run > 40) return (run + 15) / 16 * 16;     // (the caller bounds it by kMaxLZ)
+    const int chunks = (p->nz + run - 1) / run;
+    return (p->nz + chunks - 1) / chunks;  // the planes evenly over the runs
+}
+
 int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d_signs, float iso,
                          int lz, hipStream_t stream) {
     int st = validate_lattice(p);
@@ -113,20 +140,13 @@ int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d
     GC_ARG(d_field, "field pointer is NULL");
     const bool rot = p->rot0 != 0.f || p->rot1 != 0.f;
     const int rows = rows_per_lane(rot);
-    // default z run: long enough to amortise the per-column work (with four
-    // rows per lane that work is four rows' thickness modes, so the run is
-    // about a fifth of the grid, rounded up to 16 planes: 112 at 512^3,
-    // measured best among 32..128), short enough to leave several workgroups
-    // per z column
-    if (lz <= 0)
-        lz = rows > 1 ? std::max(16, std::min(kMaxLZ, ((p->nz + 4) / 5 + 15) / 16 * 16))
-                      : std::max(16, std::min(kMaxLZ, p->nz / 8));
+    const int brick_y = kFieldWaves * rows;
+    if (lz <= 0) lz = default_z_run(p, (p->nx + 63) / 64, (p->ny + brick_y - 1) / brick_y);
     if (lz > kMaxLZ) lz = kMaxLZ;
     const FieldConsts c = make_field_consts(p, iso, lz);
     const bool thick = p->n_modes > 0;
     FieldKernel k = rot ? pick_tpms<true>(p->tpms, thick, c.prim, c.op)
                         : pick_tpms<false>(p->tpms, thick, c.prim, c.op);
-    const int brick_y = kFieldWaves * rows;
     dim3 grid((p->nx + 63) / 64, (p->ny + brick_y - 1) / brick_y, (p->nz + lz - 1) / lz);
     GC_ARG(grid.y <= 65535 && grid.z <= 65535, "grid too large for one launch");
     hipLaunchKernelGGL(k, grid, dim3(64 * kFieldWaves), 0, stream, c, d_field, d_signs);
