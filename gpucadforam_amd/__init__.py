@@ -444,20 +444,25 @@ def f3(x, y, z):
 # ---------------------------------------------------------------------------
 # batched form
 # ---------------------------------------------------------------------------
-def _device_view(addr, count, dtype, device):
-    """A torch tensor over `count` elements of library-owned device memory
-    (valid while the owner lives)."""
-    if count == 0:
-        return torch.empty(0, dtype=dtype, device=device)
+class _Holder:
+    """Memory for torch.as_tensor through the CUDA array interface.  One class
+    for all of them: a class per view took 3.7 of a view's 4.5 us, 48 times per
+    burst of 16 served requests (703 us, 508 so)."""
+    __slots__ = ("__cuda_array_interface__",)
 
-    class _Holder:  # wraps the memory through the CUDA array interface
-        __cuda_array_interface__ = {
-            "shape": (count,),
-            "typestr": {torch.float32: "<f4", torch.int32: "<i4", torch.int64: "<i8"}[dtype],
-            "data": (addr, False),
-            "version": 2,
-        }
-    return torch.as_tensor(_Holder(), device=device)
+
+_TYPESTR = {torch.float32: "<f4", torch.int32: "<i4", torch.int64: "<i8"}
+
+
+def _device_view(addr, shape, dtype, device):
+    """A torch tensor over library-owned device memory (valid while the owner
+    lives)."""
+    if shape[0] == 0:
+        return torch.empty(shape, dtype=dtype, device=device)
+    h = _Holder()
+    h.__cuda_array_interface__ = {"shape": shape, "typestr": _TYPESTR[dtype],
+                                  "data": (addr, False), "version": 2}
+    return torch.as_tensor(h, device=device)
 
 
 class Batch:
@@ -482,11 +487,9 @@ class Batch:
         check(lib.gpucad_batch_buffers(self._h, C.byref(b)))
         self.buffers = b
         dev = torch.device("cuda", torch.cuda.current_device())
-        self.fields = _device_view(b.fields, b.field_floats, torch.float32, dev)
-        self.vertices = _device_view(b.vertices, 3 * b.vert_capacity, torch.float32,
-                                     dev).view(-1, 3)
-        self.triangles = _device_view(b.triangles, 3 * b.tri_capacity, torch.int32,
-                                      dev).view(-1, 3)
+        self.fields = _device_view(b.fields, (b.field_floats,), torch.float32, dev)
+        self.vertices = _device_view(b.vertices, (b.vert_capacity, 3), torch.float32, dev)
+        self.triangles = _device_view(b.triangles, (b.tri_capacity, 3), torch.int32, dev)
 
     def tuning(self):
         o = BatchOptions()
@@ -567,20 +570,14 @@ class Server:
 
     def result_arrays(self, r, params):
         """Host copies (field, vertices, triangles) of a finished request."""
-        f = _device_view(r.field, params.npoints(), torch.float32, self.device).cpu().numpy()
-        v = _device_view(r.vertices, 3 * r.n_vertices, torch.float32,
-                         self.device).cpu().numpy().reshape(-1, 3)
-        t = _device_view(r.triangles, 3 * r.n_triangles, torch.int32,
-                         self.device).cpu().numpy().reshape(-1, 3)
-        return f, v, t
+        return tuple(t.cpu().numpy() for t in self.result_tensors(r, params))
 
     def result_tensors(self, r, params):
         """Device views (field, vertices (V, 3), triangles (T, 3)) of a finished
         request, valid until the request is released."""
-        f = _device_view(r.field, params.npoints(), torch.float32, self.device)
-        v = _device_view(r.vertices, 3 * r.n_vertices, torch.float32, self.device).view(-1, 3)
-        t = _device_view(r.triangles, 3 * r.n_triangles, torch.int32, self.device).view(-1, 3)
-        return f, v, t
+        return (_device_view(r.field, (params.npoints(),), torch.float32, self.device),
+                _device_view(r.vertices, (r.n_vertices, 3), torch.float32, self.device),
+                _device_view(r.triangles, (r.n_triangles, 3), torch.int32, self.device))
 
     def run_trace(self, requests, arrivals):
         n = len(requests)
