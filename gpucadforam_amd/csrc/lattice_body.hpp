@@ -49,7 +49,20 @@ struct FieldConsts {
     int prim, op;
     float pc[3], pr, ph[3];
     int prim_plain;               // every squared distance stays below 2^96
+    int nt_store;                 // field stores with the non-temporal hint
 };
+
+// Whether a grid's field is stored with the non-temporal hint, given the
+// points of its launch.  Rows that end inside a 128-byte line share lines
+// between bricks, which an L2 merges only without the hint: 256 grids of
+// 32..256 points per axis 834 us with it, 652 without, 500^3 198 and 86 (with a
+// row's bricks on one XCD, which alone took 1036 to 834).  A field of the size
+// of the L2s (32 MB) is then still in them when the kernel ends and has to be
+// written back before the next one starts: a 203 x 149 x 181 edit, 22 MB,
+// 70.3 us with the hint, 71.7 without.
+inline int field_nt_store(int nx, uint64_t launch_points) {
+    return nx % 32 == 0 || launch_points < (1u << 24);
+}
 
 // Field variant: which template instance evaluates a grid.
 struct FieldVariant {
@@ -70,7 +83,8 @@ inline FieldVariant field_variant(const gc_lattice_params *p) {
 int validate_lattice(const gc_lattice_params *p);
 
 // Fills the constants of grid `p` (validated) for isovalue `iso` and z run `lz`.
-inline FieldConsts make_field_consts(const gc_lattice_params *p, float iso, int lz) {
+inline FieldConsts make_field_consts(const gc_lattice_params *p, float iso, int lz,
+                                     uint64_t launch_points) {
     FieldConsts c;
     std::memset(&c, 0, sizeof(c));
     c.nx = p->nx;
@@ -112,6 +126,7 @@ inline FieldConsts make_field_consts(const gc_lattice_params *p, float iso, int 
         c.ph[a] = p->prim_half[a];
     }
     c.pr = p->prim_radius;
+    c.nt_store = field_nt_store(p->nx, launch_points);
     c.prim_plain = 1;  // (false for NaN)
     for (int a = 0; a < 3; ++a)
         if (!(std::fabs(c.pc[a]) <= 0x1p40f && std::fabs(c.ph[a]) <= 0x1p40f)) c.prim_plain = 0;
@@ -179,14 +194,11 @@ constexpr int PRIM_ANY = -1;
 
 // The lattice value g combined with the primitive whose distance root is
 // `root` (sphere: root - r; box: root + min(max(partial, z term), 0)).
-template <int PRIM, int OP>
-__device__ __forceinline__ float prim_op(const FieldConsts &c, float pr, float g, float root,
-                                         float pz, float pbxy) {
-    const int prim = PRIM == PRIM_ANY ? c.prim : PRIM;
+__device__ __forceinline__ float prim_op(int prim, int op, float pr, float g, float root, float pz,
+                                         float pbxy) {
     const float s = prim == GC_PRIM_SPHERE
                         ? root - pr
                         : root + __builtin_fminf(__builtin_fmaxf(pbxy, pz), 0.f);
-    const int op = OP == PRIM_ANY ? c.op : OP;
     const float gi = __builtin_fmaxf(g, s), gu = __builtin_fminf(g, s), gs = __builtin_fmaxf(g, -s);
     return op == GC_OP_INTERSECT ? gi
                                  : (op == GC_OP_UNION ? gu : (op == GC_OP_SUBTRACT ? gs : g));
@@ -206,7 +218,7 @@ __device__ __forceinline__ float prim_op(const FieldConsts &c, float pr, float g
 // on (x, z) only (the z table reads, the z phase and its cos / sin) is done
 // once per RY points.  Every point's arithmetic is the same for any RY.
 template <bool ROT, int TPMS, bool THICK, int BX, int PRIM = PRIM_ANY, int OP = PRIM_ANY,
-          int RY = 1>
+          int RY = 1, bool NT = false>
 __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__restrict__ field,
                                               uint64_t *__restrict__ signs, int x0, int y0,
                                               int z0, float *ztab) {
@@ -397,6 +409,12 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
         }
     }
     const float quarter = pinned(0.25f), pr = pinned(c.pr);
+    // (the constants of a batch are in memory: read here, not in the loop,
+    // where the stores in between would have them read again at every step)
+    const float iso = c.iso;
+    const bool nt_store = NT || c.nt_store;  // (NT: known at compile time)
+    const bool uniform_period = c.uniform_period;
+    const int op = OP == PRIM_ANY ? c.op : OP;
     // the lanes that store sign words: lane r stores row r's
     uint32_t moff = kPastPlane;
     if (BX == 64) {
@@ -420,7 +438,7 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
                 cZ = cos_rev(Zr, quarter);
             }
         } else {
-            if (c.uniform_period) {
+            if (uniform_period) {
                 cZ = e[ZT_CZ];
                 sZ = e[ZT_SZ];
             } else {
@@ -482,14 +500,14 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
                                                 : __builtin_fmaf(mz, mz, pxy[r]);
                 const float root = PRIM == GC_PRIM_SPHERE ? sqrt_rn_plain<false>(px2[r])
                                                           : sqrt_rn_plain<true>(px2[r]);
-                g = prim_op<PRIM, OP>(c, pr, g, root, pz, pbxy[r]);
+                g = prim_op(prim, op, pr, g, root, pz, pbxy[r]);
             }
             gv[r] = g;
         }
         if (prim != GC_PRIM_NONE && general) {
 #pragma unroll
             for (int r = 0; r < RY; ++r)
-                gv[r] = prim_op<PRIM, OP>(c, pr, gl[r], sqrt_rn(px2[r]), pz, pbxy[r]);
+                gv[r] = prim_op(prim, op, pr, gl[r], sqrt_rn(px2[r]), pz, pbxy[r]);
         }
         if (BX == 64) {
             // buffer stores over this z plane: a lane whose point lies outside
@@ -500,11 +518,19 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
             const __amdgpu_buffer_rsrc_t fr =
                 __builtin_amdgcn_make_buffer_rsrc(fplane + (uint64_t)i * fstep, (short)0,
                                                   (int)(uint32_t)fstep, kBufferWord3);
+            if (nt_store) {
 #pragma unroll
-            for (int r = 0; r < RY; ++r)
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(gv[r]), fr,
-                                                      (int)((xin && yin[r]) ? foff[r] : kPastPlane),
-                                                      0, kStoreNonTemporal);
+                for (int r = 0; r < RY; ++r)
+                    __builtin_amdgcn_raw_buffer_store_b32(
+                        __float_as_uint(gv[r]), fr, (int)((xin && yin[r]) ? foff[r] : kPastPlane),
+                        0, kStoreNonTemporal);
+            } else {
+#pragma unroll
+                for (int r = 0; r < RY; ++r)
+                    __builtin_amdgcn_raw_buffer_store_b32(
+                        __float_as_uint(gv[r]), fr, (int)((xin && yin[r]) ? foff[r] : kPastPlane),
+                        0, 0);
+            }
             if (splane) {
                 // the rows' sign words in one store: lane r holds row r's
                 // word (one compare per row gives the wave's mask of lanes with
@@ -516,7 +542,7 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
                 int lo = 0, hi = 0;
 #pragma unroll
                 for (int r = 0; r < RY; ++r) {
-                    const uint64_t m = __builtin_amdgcn_fcmpf(gv[r], c.iso, 4) & in_mask;
+                    const uint64_t m = __builtin_amdgcn_fcmpf(gv[r], iso, 4) & in_mask;
                     lo = write_lane((int)(uint32_t)m, r, lo);
                     hi = write_lane((int)(m >> 32), r, hi);
                 }
@@ -535,7 +561,7 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
             if (splane) {
                 // one compare gives the wave's mask of lanes with g < iso (4 is
                 // the ordered less-than predicate: NaN compares false)
-                const uint64_t m = __builtin_amdgcn_fcmpf(g, c.iso, 4) & in_mask;
+                const uint64_t m = __builtin_amdgcn_fcmpf(g, iso, 4) & in_mask;
                 if (sign_lane && yin[r]) {
                     const uint64_t bits =
                         BX == 64 ? m : (m >> (ly * BX)) & ((1ull << (BX & 63)) - 1ull);
