@@ -72,6 +72,10 @@ __device__ __forceinline__ uint64_t shift1(uint64_t cur, uint64_t next) {
     return (cur >> 1) | (next << 63);
 }
 __device__ __forceinline__ uint32_t popc64(uint64_t w) { return (uint32_t)__popcll(w); }
+__device__ __forceinline__ uint32_t popc32(uint32_t w) { return (uint32_t)__popc(w); }
+__device__ __forceinline__ uint64_t load_u64(const void *base, uint32_t off) {
+    return *(const uint64_t *)((const char *)base + off);
+}
 __device__ __forceinline__ uint64_t mask_below(int64_t n) {
     if (n >= 64) return ~0ull;
     if (n <= 0) return 0ull;
@@ -121,14 +125,6 @@ __device__ __forceinline__ void store_nt(uint32_t *p, T3 t) {
 __device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv &f) {
     const uint32_t q = __umulhi(n, f.m);  // n / d or one less
     return q + (n - q * f.d >= f.d ? 1u : 0u);
-}
-
-// sign word `idx` of a grid (32-bit word index: a grid has fewer than 2^32
-// words) when `ok`, else 0.  The load is unconditional (word 0 stands in),
-// so a run of these has no branches and its loads issue back to back.
-__device__ __forceinline__ uint64_t ldw(const uint64_t *s, uint32_t idx, bool ok) {
-    const uint64_t v = s[ok ? idx : 0u];
-    return ok ? v : 0ull;
 }
 
 struct WordPos {
@@ -238,6 +234,16 @@ __device__ __forceinline__ uint32_t word_triangles(uint64_t k0, uint64_t k1, uin
     return v - 2 * f - 4 * d + 4 * inside;
 }
 
+// Block of workgroup b of n: workgroup b runs on XCD b % 8, and each XCD takes
+// runs of 1 << lr consecutive blocks, so the rows and planes next to a block's
+// own are in its L2.
+__device__ __forceinline__ uint32_t run_order(uint32_t b, uint32_t n, uint32_t lr) {
+    const uint32_t first = b >> (lr + 3) << (lr + 3);  // of the 8 runs
+    if (n - first < (8u << lr)) return b;
+    const uint32_t in = b - first;
+    return first + ((in & 7u) << lr) + (in >> 3);
+}
+
 struct CountArgs {
     const uint64_t *signs;  // sign buffer base
     uint32_t *live;         // per block: bit i: its words 8i .. 8i + 7 have something to emit
@@ -245,14 +251,17 @@ struct CountArgs {
     // per word: first vertex of its two half words (16 bits each) and its
     // first triangle, within the block (at most 49152 and 81920)
     uint2 *base;
+    uint32_t lr;            // log2 of the blocks of a run
 };
 
+// Bound by the words that it reads four times, in rows and planes, and the 8
+// bytes that it writes per word (1024^3: 134 MB each, 130 us).
 template <class Src>
 __global__ void __launch_bounds__(kBlock) count_kernel(Src src, CountArgs a) {
     __shared__ uint32_t s_sum[4][2];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     {
-        const uint32_t gb = blockIdx.x;
+        const uint32_t gb = run_order(blockIdx.x, gridDim.x, a.lr);
         const Seg s = src.get(src.seg_of(gb));
         const Grid &g = s.g;
         const uint64_t *signs = a.signs + s.sign_off;
@@ -261,33 +270,37 @@ __global__ void __launch_bounds__(kBlock) count_kernel(Src src, CountArgs a) {
         if (k < g.words) {
             const WordPos p = word_pos(k, g);
             const bool has_y = p.y + 1 < g.ny, has_z = p.z + 1 < g.nz;
-            const uint32_t kk = (uint32_t)k, W = (uint32_t)g.W, RW = (uint32_t)g.ny * W;
-            const bool hw = p.w + 1 < g.W;
-            const uint64_t wa = signs[kk];
-            const uint64_t an = ldw(signs, kk + 1, hw);
-            const uint64_t wb = ldw(signs, kk + W, has_y);
-            const uint64_t bn = ldw(signs, kk + W + 1, has_y && hw);
-            const uint64_t wc = ldw(signs, kk + RW, has_z);
-            const uint64_t cn = ldw(signs, kk + RW + 1, has_z && hw);
-            const uint64_t wd = ldw(signs, kk + RW + W, has_y && has_z);
-            const uint64_t dn = ldw(signs, kk + RW + W + 1, has_y && has_z && hw);
+            // a row or word that does not exist stands for its predecessor: no
+            // crossing between rows, and past the row's last word the masks
+            // leave no bit that a next word would reach
+            const uint32_t W8 = 8u * (uint32_t)g.W;
+            const uint32_t dy = has_y ? W8 : 0u, dz = has_z ? (uint32_t)g.ny * W8 : 0u;
+            const uint32_t dn = p.w + 1 < g.W ? 8u : 0u;
+            const uint64_t *at = signs + (gb - s.block_off) * (uint64_t)kBlock;
+            const uint32_t oa = 8u * tid, ob = oa + dy, oc = oa + dz, od = ob + dz;
+            const uint64_t wa = load_u64(at, oa), an = load_u64(at, oa + dn);
+            const uint64_t wb = load_u64(at, ob), bn = load_u64(at, ob + dn);
+            const uint64_t wc = load_u64(at, oc), cn = load_u64(at, oc + dn);
+            const uint64_t wd = load_u64(at, od), dn_ = load_u64(at, od + dn);
             // all eight loads issue before any of the arithmetic on them
             __builtin_amdgcn_sched_barrier(0);
-            const uint64_t sa = shift1(wa, an);
-            const uint64_t sb = shift1(wb, bn);
-            const uint64_t sc = shift1(wc, cn);
+            const uint64_t sa = shift1(wa, an), sb = shift1(wb, bn);
+            const uint64_t sc = shift1(wc, cn), sd = shift1(wd, dn_);
             const uint64_t vpt = mask_below((int64_t)g.nx - 64 * p.w);
             const uint64_t ved = mask_below((int64_t)g.nx - 1 - 64 * p.w);
-            const uint64_t ex = (wa ^ sa) & ved;
-            const uint64_t ey = has_y ? (wa ^ wb) & vpt : 0ull;
-            const uint64_t ez = has_z ? (wa ^ wc) & vpt : 0ull;
-            vc = popc64(ex) + popc64(ey) + popc64(ez);
-            vlo = popc64(ex & 0xffffffffull) + popc64(ey & 0xffffffffull) +
-                  popc64(ez & 0xffffffffull);
-            if (has_y && has_z) {
-                const uint64_t sd = shift1(wd, dn);
-                tc = word_triangles(wa & ved, sa & ved, sb & ved, wb & ved, wc & ved, sc & ved,
-                                    sd & ved, wd & ved);
+            const uint64_t any = (wa | sa | wb | sb | wc | sc | wd | sd) & vpt;
+            const uint64_t all = wa & sa & wb & sb & wc & sc & wd & sd;
+            // (a wave with all its signs equal, cells and own edges: nothing)
+            if (__any((any & ~all) != 0)) {
+                const uint64_t ex = (wa ^ sa) & ved;
+                const uint64_t ey = (wa ^ wb) & vpt;
+                const uint64_t ez = (wa ^ wc) & vpt;
+                vlo = popc32((uint32_t)ex) + popc32((uint32_t)ey) + popc32((uint32_t)ez);
+                vc = vlo + popc32((uint32_t)(ex >> 32)) + popc32((uint32_t)(ey >> 32)) +
+                     popc32((uint32_t)(ez >> 32));
+                if (has_y && has_z)
+                    tc = word_triangles(wa & ved, sa & ved, sb & ved, wb & ved, wc & ved, sc & ved,
+                                        sd & ved, wd & ved);
             }
         }
         const uint32_t vincl = wave_scan_incl(vc);
@@ -459,6 +472,8 @@ constexpr int kIdStride = kEmitStride; // vertex numbers of an edge: 64 cells + 
 // 42.5 us for scan and emission (4.9 of them the scan, and its launch), 35.6 so.
 constexpr int kSelfBlocks = 512;
 
+constexpr uint32_t kMixed = ~0u;
+
 struct EmitArgs {
     const float *field;     // field buffer base
     const uint64_t *signs;  // sign buffer base
@@ -472,6 +487,7 @@ struct EmitArgs {
     uint32_t *triangles;
     uint64_t tcap;
     uint32_t lw;            // log2 of the words per wave: 3, 4 or 5
+    uint32_t lr;            // log2 of the workgroups of a run, or kMixed
     uint32_t nb;            // kSelf: blocks of the grid
     uint64_t *ctl, *d_counts;  // kSelf: written by the first workgroup
 };
@@ -528,7 +544,8 @@ __device__ __forceinline__ uint32_t record_limit(uint64_t cap, uint64_t at, uint
 // lists).  Edge and triangle records leave 64 at a time on 128-byte line
 // boundaries: non-temporal stores of 12-byte records move 3.9 TB/s when every
 // store ends inside a line and 5.0 TB/s when only a wave's first and last do.
-// 1024^3: 3231 -> 2665 us, 512^3: 186 -> 172, 128^3: 25 -> 15, 40^3: 23 -> 10.
+// 1024^3: 3231 -> 2665 us, 512^3: 186 -> 172 (143 in runs of a plane, run_order),
+// 128^3: 25 -> 15, 40^3: 23 -> 10.
 //
 // Workgroups of four waves: they share the triangle table, and with eight a
 // wave that is done waits for more of the others before its LDS is free
@@ -541,11 +558,13 @@ emit_kernel(Src src, EmitArgs a) {
     constexpr uint32_t kThreads = 64 * kEmitWaves;
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    // Workgroup b runs on XCD b % 8, and so would every eighth workgroup of a
-    // plane, the same rows in every plane: mixing the higher bits in spreads a
-    // part that fills some of the rows over all XCDs (512^3: 185 -> 175 us).
+    // Few blocks: neighbours over the XCDs, mixed with the higher bits so that
+    // no XCD has the same rows of every plane (run_log2).
     uint32_t bx = blockIdx.x;
-    if ((bx | 7u) < gridDim.x) bx ^= (bx >> 3 ^ bx >> 6 ^ bx >> 9 ^ bx >> 12 ^ bx >> 15) & 7u;
+    if (a.lr != kMixed)
+        bx = run_order(bx, gridDim.x, a.lr);
+    else if ((bx | 7u) < gridDim.x)
+        bx ^= (bx >> 3 ^ bx >> 6 ^ bx >> 9 ^ bx >> 12 ^ bx >> 15) & 7u;
     // a workgroup takes 4 << lw words of a block of 256
     const uint32_t lw = a.lw, lparts = 6 - lw;
     const uint32_t gb = bx >> lparts, part = bx & ((1u << lparts) - 1u);
@@ -919,6 +938,24 @@ namespace {
 // 37.6, 35.6, 35.6 (32 words); 1.7 k blocks (16 served grids): 119.5 of 16, 126 of 32.
 uint32_t words_per_wave_log2(uint64_t nb) { return nb >= 4096 ? 5 : (nb >= 256 ? 4 : 3); }
 
+// Blocks of a run (run_order), as a logarithm: about a plane, with at least 8
+// runs per XCD.  512^3 with a sphere, count to emission: 177 us with the
+// workgroups mixed over the XCDs, 148 in runs of a plane, 144 of two, 149 of
+// four; 1024^3 full of surface 2883, 2904, 2947, 3028; 640^3 294, 292, 293, 300.
+uint32_t run_log2(uint64_t nb, uint64_t plane_blocks) {
+    uint32_t lr = 0;
+    while (lr < 20 && (1ull << lr) < plane_blocks) ++lr;
+    while (lr > 0 && (64ull << lr) > nb) --lr;
+    return lr;
+}
+
+// The order of the emission's workgroups (EmitArgs::lr).  Below 1536 blocks
+// mixing them was faster: the edit of 128^3 21.9 us, in runs 22.8; 256^3 100.2
+// and 101.1; 300^3 (1758 blocks) 183.9 and 182.2.
+uint32_t emit_order(uint64_t nb, uint64_t plane_blocks, uint32_t lw) {
+    return nb < 1536 ? kMixed : run_log2(nb, plane_blocks) + 6 - lw;
+}
+
 template <class Src, bool kSelf>
 int launch_emit(const Src &src, const EmitArgs &a, uint64_t nb, hipStream_t stream) {
     const uint64_t wgs = nb << (6 - a.lw);
@@ -972,11 +1009,12 @@ int enqueue_extract(const gc_extract_args *a, hipStream_t stream) {
     }
     uint2 *base = (uint2 *)(ws + L.base_off);
     uint32_t *live = (uint32_t *)(ws + L.live_off);
+    const uint64_t plane_blocks = ((uint64_t)s.g.W * a->ny + kBlock - 1) / kBlock;
     uint64_t *bsum = (uint64_t *)(ws + L.bsum_off);
     uint64_t *ctl = (uint64_t *)(ws + L.ctl_off);
     SegResult *res = (SegResult *)(ws + L.res_off);
     hipLaunchKernelGGL(count_kernel<OneGrid>, dim3((unsigned)L.nb), dim3(kBlock), 0, stream, one,
-                       CountArgs{signs, live, bsum, base});
+                       CountArgs{signs, live, bsum, base, run_log2(L.nb, plane_blocks)});
     GC_CHECK_LAUNCH();
     const bool self = L.nb <= (uint64_t)kSelfBlocks;
     if (!self) {
@@ -987,7 +1025,8 @@ int enqueue_extract(const gc_extract_args *a, hipStream_t stream) {
     const uint32_t lw = words_per_wave_log2(L.nb);
     const EmitArgs ea = {a->field, signs, base, live, bsum, res, tabs->emit, a->vertices,
                          a->vertices ? a->vert_capacity : 0, a->triangles,
-                         a->triangles ? a->tri_capacity : 0, lw, (uint32_t)L.nb, ctl, a->d_counts};
+                         a->triangles ? a->tri_capacity : 0, lw, emit_order(L.nb, plane_blocks, lw),
+                         (uint32_t)L.nb, ctl, a->d_counts};
     if (a->emit_event) GC_HIP(hipEventRecord((hipEvent_t)a->emit_event, stream));
     return self ? launch_emit<OneGrid, true>(one, ea, L.nb, stream)
                 : launch_emit<OneGrid, false>(one, ea, L.nb, stream);
@@ -1000,9 +1039,11 @@ int enqueue_extract_batch(const BatchExtract &b, int phases, hipStream_t stream)
     int st = device_tables(&tabs);
     if (st) return st;
     const ManyGrids src = {b.segs, b.blk2seg};
+    const uint64_t plane_blocks = 4;  // (a plane of 128..256 points; longer runs: no gain)
     if (phases & EXTRACT_COUNT) {
         hipLaunchKernelGGL(count_kernel<ManyGrids>, dim3(b.nb), dim3(kBlock), 0, stream, src,
-                           CountArgs{b.signs, b.live, b.bsum, (uint2 *)b.base});
+                           CountArgs{b.signs, b.live, b.bsum, (uint2 *)b.base,
+                                     run_log2(b.nb, plane_blocks)});
         GC_CHECK_LAUNCH();
         hipLaunchKernelGGL(scan_blocks_kernel, dim3(1), dim3(1024), 0, stream, b.bsum,
                            (uint64_t)b.nb, b.ctl, (uint64_t *)nullptr, b.segs, b.nseg, b.res);
@@ -1011,7 +1052,8 @@ int enqueue_extract_batch(const BatchExtract &b, int phases, hipStream_t stream)
     if (phases & EXTRACT_EMIT) {
         const EmitArgs ea = {b.fields, b.signs, (const uint2 *)b.base, b.live, b.bsum, b.res,
                              tabs->emit, b.vertices, b.vertices ? b.vcap : 0, b.triangles,
-                             b.triangles ? b.tcap : 0, lw, b.nb, nullptr, nullptr};
+                             b.triangles ? b.tcap : 0, lw, emit_order(b.nb, plane_blocks, lw), b.nb,
+                             nullptr, nullptr};
         if ((st = launch_emit<ManyGrids, false>(src, ea, b.nb, stream))) return st;
     }
     return GPUCAD_OK;
