@@ -440,10 +440,7 @@ __global__ void __launch_bounds__(64) bool_generate_kernel(BGenArgs a) {
             const bool fixed = f & GC_BOOL_FIXED, make = f & GC_BOOL_MAKE_REGION;
             float D[8], L[8];
             float4 G[8];
-            // (a mode's volumes exist; the loads need not wait for the cell's
-            // case.  211 x 193 x 229, 3.1 M vertices: 40.6 us when they did,
-            // 39.2 so and with stores on line boundaries)
-            const bool load = nn.f || nn.d || nn.l;
+            const bool load = nv != 0;  // (a mode's volumes exist when it yields vertices)
             if (load && !make && (fixed || !(f & GC_BOOL_DYNAMIC)))
                 corners_inside(a.v.dyn, lin, gx, gxy, D);
             if (load && !make && (fixed || (f & GC_BOOL_DYNAMIC)))
@@ -494,8 +491,9 @@ __global__ void __launch_bounds__(64) bool_generate_kernel(BGenArgs a) {
         s_tri[lane] = *(const uint4 *)(a.tri + cube * 16);
         for (uint32_t j = 0; j < nv; ++j) owner[first + j] = (uint8_t)lane;
         __syncthreads();
-        for (uint32_t k = lane - (s_base[0] & 7u); (int)k < (int)total; k += 64) {
-            if ((int)k < 0) continue;
+        // (not from a line boundary on, as the lattice's generate: 19.6 M
+        // vertices in dynamic mode 212 us, so 224)
+        for (uint32_t k = lane; k < total; k += 64) {
             const uint32_t o = owner[k];
             const uint32_t j = k - s_first[o];
             const uint32_t t0 = j - j % 3u;  // the triangle's first vertex
