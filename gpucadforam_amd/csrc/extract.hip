@@ -535,8 +535,10 @@ __device__ __forceinline__ uint32_t record_limit(uint64_t cap, uint64_t at, uint
 
 // The whole mesh of a chunk of 8, 16 or 32 words by one wave.
 //
-// Bound: at 1024^3 (222 M vertices, 445 M triangles) it moves 11.1 GB, 2.1 ms
-// at the copy rate; the vector units are busy 60 % and LDS 50 % of the time.
+// Bound by the bytes it moves: at 1024^3 (222 M vertices, 445 M triangles) 14.6
+// GB by the counters (6.2 read, 8.4 written), 2.8 ms at the rate of a large
+// copy; at 512^3 0.73 GB, 140 us.  The vector units are busy 60 % and LDS 50 %
+// of the time at 1024^3.
 // One wave makes a chunk's vertices and triangles, so the signs are loaded and
 // the crossings derived once and the edges come out of the cell steps as a
 // ring, without a pass of their own (two kinds of workgroup before: 18 % of
