@@ -292,6 +292,8 @@ SIGNATURES = {
     "gpucad_svl_matvec": ([_vp, _vp, _i32, _i32, _i32], C.c_int),
     "gpucad_svl_cg": ([_vp, _i32, _i32, _i32, _i32, _f, C.POINTER(_i32), C.POINTER(_f)],
                       C.c_int),
+    "gpucad_svl_cg_form": ([_vp, _i32, _i32, _i32, _i32, _i32, _f, _i32, _f, _f, C.POINTER(_i32),
+                            C.POINTER(_f), C.POINTER(_i32)], C.c_int),
     "gpucad_svl_axpby": ([_vp, _f, _vp, _f, _u64], C.c_int),
     "gpucad_svl_dot": ([_vp, _vp, _vp, _u64], C.c_int),
     "gpucad_svl_fillfrac": ([_vp, _vp, _i32, _i32, _i32], C.c_int),

@@ -299,7 +299,8 @@ struct CgState {
     int done;
     int iters;       // the reference's FinalIter
     float res;       // the reference's FinalRes = sqrt(r.r)
-    int pad[3];
+    uint32_t tiles;  // tiles whose part of the solution is written (cg_chip_kernel)
+    int pad[2];
 };
 
 constexpr int kCgUnroll = 2;  // points per thread and step, all their loads in flight
@@ -510,8 +511,10 @@ __global__ void cg_b_kernel(CgArgs a, int it) {
 //
 // All workgroups must be resident together: at most one per CU is launched.
 // Every wait is bounded in time: should other work hold the CUs that long, the
-// waiting workgroups leave, nothing has been written to x, and the caller
-// solves by the two-launch form.
+// waiting workgroups leave.  A tile that leaves may have posted its sums, so
+// others, the first one too, can still reach the end: the solution is complete
+// only when every tile has counted itself after writing its part.  Otherwise
+// the caller solves by the two-launch form; x has not been written.
 //
 // Measured (us per iteration, two-launch form -> this): three right-hand
 // sides of 120^3 41 -> 20.4; one of 120^3 26.8 -> 12.4, of 61 x 57 x 70 13.7 -> 8.1, of
@@ -527,7 +530,7 @@ struct ChipArgs {
     int nx, ny, nz, m, ty, tz, G;  // G = ty * tz tiles per right-hand side
     uint64_t n;
     const float *b;             // m right-hand sides
-    float *phi;                 // their solutions, complete when every `done` is set
+    float *phi;                 // their solutions, complete when each has G finished tiles
     uint64_t *faces;            // [m][G][4][face_words]: r, iteration
     uint64_t *sums;             // [m][2][G][2]: FP64 halves, iteration
     uint32_t face_words;
@@ -535,6 +538,9 @@ struct ChipArgs {
     CgState *st;
     int max_iter;
     float term;
+    // longest wait of a right-hand side's first tile and of the others, in ticks
+    // of the 100 MHz clock; negative: the first wait ends at once
+    int64_t wait_first, wait_others;
 };
 
 // The same value, unknown to the optimiser: what is computed from it inside the
@@ -562,13 +568,14 @@ __device__ __forceinline__ uint64_t read_word(const uint64_t *p) {
 
 // A bounded wait: false once the time has run out or another workgroup gave up.
 struct ChipWait {
-    int64_t start = 0;
+    int64_t limit, start = 0;
     uint32_t turns = 0;
+    __device__ __forceinline__ explicit ChipWait(int64_t ticks) : limit(ticks) {}
     __device__ __forceinline__ bool again(uint32_t *abort) {
-        if ((++turns & 63u) != 0) return true;
+        if (limit >= 0 && (++turns & 63u) != 0) return true;
         const int64_t now = (int64_t)wall_clock64();
         if (start == 0) start = now;
-        if (now - start > kChipWaitTicks)
+        if (now - start > limit)
             __hip_atomic_store(abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
     }
@@ -594,18 +601,19 @@ __device__ __forceinline__ void chip_post(double v, uint64_t *slots, int g, uint
     }
 }
 __device__ __forceinline__ bool chip_collect(const uint64_t *slots, int G, uint32_t it,
-                                             uint32_t *abort, ChipShared &sh, double *total) {
+                                             uint32_t *abort, int64_t limit, ChipShared &sh,
+                                             double *total) {
     const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6, used = (G + 63) >> 6;
     if (wave < used) {
         double w = 0.0;
         bool ok = true;
         if (t < G) {
-            ChipWait wait;
+            ChipWait wait(limit);
             uint64_t hi, lo;
             for (;;) {
                 hi = read_word(slots + 2 * t);
                 lo = read_word(slots + 2 * t + 1);
-                if ((uint32_t)(hi >> 32) == it && (uint32_t)(lo >> 32) == it) break;
+                if (limit >= 0 && (uint32_t)(hi >> 32) == it && (uint32_t)(lo >> 32) == it) break;
                 if (!wait.again(abort)) {
                     ok = false;
                     break;
@@ -663,6 +671,7 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
     const int rows = (int)blockDim.x / nx;  // tile rows a pass of the workgroup covers
     const int row = t / nx, x = t - row * nx;
     const bool own = row < by;              // (rows >= by)
+    const int64_t limit = g == 0 ? a.wait_first : a.wait_others;
     const int ty = own ? row : 0;           // threads without a column follow column 0's
     const float *b = a.b + (uint64_t)s * a.n;
     if (t == 0) sh.abort = 0;
@@ -743,7 +752,7 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
 
     double tot;
     chip_post(acc, sums_rr, g, 1u, sh);
-    if (!chip_collect(sums_rr, a.G, 1u, a.abort, sh, &tot)) return;
+    if (!chip_collect(sums_rr, a.G, 1u, a.abort, limit, sh, &tot)) return;
     float delta = (float)tot, delta_prev = 0.f, beta = 0.f;
     float hy[2][2][kYPass], hz[2][2];  // the halo's r: [side][layer][pass], [side][layer]
     int it = 0;
@@ -832,7 +841,7 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
             if (!own) acc = 0.0;
         }
         chip_post(acc, sums_dq, g, (uint32_t)it + 1u, sh);
-        if (!chip_collect(sums_dq, a.G, (uint32_t)it + 1u, a.abort, sh, &tot)) return;
+        if (!chip_collect(sums_dq, a.G, (uint32_t)it + 1u, a.abort, limit, sh, &tot)) return;
         const float alpha = delta / (float)tot;
         // phi += alpha d, r -= alpha q, the new r on the faces, r.r
         acc = 0.0;
@@ -894,7 +903,7 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
                     vz[side][l] = hasz ? read_word(pz[side] + l * by * nx + xy) : none;
                 }
             }
-            ChipWait wait;
+            ChipWait wait(limit);
             auto settle = [&](uint64_t v, const uint64_t *w) {
                 while ((uint32_t)(v >> 32) != tag) {
                     if (!wait.again(a.abort)) {
@@ -919,7 +928,7 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
                 }
         }
         if (!ok) sh.abort = 1;  // (read after the next barrier)
-        if (!chip_collect(sums_rr, a.G, (uint32_t)it + 2u, a.abort, sh, &tot)) return;
+        if (!chip_collect(sums_rr, a.G, (uint32_t)it + 2u, a.abort, limit, sh, &tot)) return;
         delta_prev = delta;
         delta = (float)tot;
         beta = delta / delta_prev;
@@ -934,8 +943,9 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
     if (g == 0 && t == 0) {
         a.st[s].iters = it + 1;
         a.st[s].res = sqrtf(delta);
-        a.st[s].done = 1;
     }
+    if (t == 0)
+        __hip_atomic_fetch_add(&a.st[s].tiles, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #undef GC_IN_RUN
 }
 
@@ -1028,11 +1038,20 @@ CgLayout cg_layout(uint64_t n, int m) {
     return l;
 }
 
+// How a solve is made (gpucad_svl_cg_form) and, after it, how it was.
+struct CgForm {
+    enum { kAuto = 0, kTwoLaunch = 1, kChip = 2 };
+    int form = kAuto;
+    int64_t wait_first = kChipWaitTicks, wait_others = kChipWaitTicks;  // ChipArgs
+    int solved_by = 0;
+};
+
 // The solve on the chip: m right-hand sides b, solutions into x (x may be b),
-// ws holding m * n floats and the exchange words.  *solved says whether it
-// ran to its end.
+// ws holding m * n floats and the exchange words.  *solved says whether every
+// tile ran to its end.
 int cg_chip_solve(const ChipPlan &p, const float *b, float *x, int m, int nx, int ny, int nz,
-                  int max_iter, float end_res, CgState *h, void *ws, bool *solved, hipStream_t st) {
+                  int max_iter, float end_res, const CgForm &f, CgState *h, void *ws, bool *solved,
+                  hipStream_t st) {
     const ChipLayout l = chip_layout(p, m);
     const uint64_t n = (uint64_t)nx * ny * nz;
     const uint64_t vec = (m * n * sizeof(float) + 255) & ~uint64_t(255);
@@ -1055,6 +1074,8 @@ int cg_chip_solve(const ChipPlan &p, const float *b, float *x, int m, int nx, in
     a.abort = (uint32_t *)(w + l.state + kMaxRhs * sizeof(CgState));
     a.max_iter = max_iter;
     a.term = end_res * end_res;
+    a.wait_first = f.wait_first;
+    a.wait_others = f.wait_others;
     *solved = false;
     typedef void (*ChipKernel)(ChipArgs);
     const int bz = (nz + p.tz - 1) / p.tz;
@@ -1074,7 +1095,7 @@ int cg_chip_solve(const ChipPlan &p, const float *b, float *x, int m, int nx, in
     GC_HIP(hipMemcpyAsync(h, a.st, m * sizeof(CgState), hipMemcpyDeviceToHost, st));
     GC_HIP(hipStreamSynchronize(st));
     for (int s = 0; s < m; ++s)
-        if (!h[s].done) return GPUCAD_OK;
+        if (h[s].tiles != (uint32_t)a.G) return GPUCAD_OK;
     GC_HIP(hipMemcpyAsync(x, a.phi, m * n * sizeof(float), hipMemcpyDeviceToDevice, st));
     *solved = true;
     return GPUCAD_OK;
@@ -1099,18 +1120,20 @@ size_t cg_bytes(int m, int nx, int ny, int nz) {
 // chunks between host checks of the done flags (a finished right-hand side
 // leaves the kernels at their first test).  x is complete in stream order.
 int cg_solve(const float *b, float *x, int m, int nx, int ny, int nz, int max_iter, float end_res,
-             int *iters, float *res, void *ws, hipStream_t st) {
+             CgForm *f, int *iters, float *res, void *ws, hipStream_t st) {
     const uint64_t n = (uint64_t)nx * ny * nz;
     CgState h[kMaxRhs];
     int cus = 0;
     int rc = cg_cus(&cus);
     if (rc) return rc;
     const ChipPlan chip = chip_plan(nx, ny, nz, m, cus);
+    GC_ARG(f->form != CgForm::kChip || chip.ty, "the grid does not fit on the chip");
     bool solved = false;
-    if (chip.ty) {
-        rc = cg_chip_solve(chip, b, x, m, nx, ny, nz, max_iter, end_res, h, ws, &solved, st);
+    if (chip.ty && f->form != CgForm::kTwoLaunch) {
+        rc = cg_chip_solve(chip, b, x, m, nx, ny, nz, max_iter, end_res, *f, h, ws, &solved, st);
         if (rc) return rc;
     }
+    f->solved_by = solved ? CgForm::kChip : CgForm::kTwoLaunch;
     if (!solved) {
         const CgLayout l = cg_layout(n, m);
         CgArgs a;
@@ -1711,23 +1734,52 @@ int gpucad_svl_matvec(const float *d_d, float *d_q, int32_t nx, int32_t ny, int3
     return GPUCAD_OK;
 }
 
-int gpucad_svl_cg(float *d_phi, int32_t nx, int32_t ny, int32_t nz, int32_t iter, float end_res,
-                  int32_t *final_iter, float *final_res) {
+static int svl_cg(float *d_phi, int m, int nx, int ny, int nz, int iter, float end_res, CgForm *f,
+                  int *final_iter, float *final_res) {
     clear_error();
     auto calls = lock_device_calls();  // shared scratch arena
     GC_ARG(d_phi, "NULL buffer");
     int st = check_dims(nx, ny, nz, 4);
     if (st) return st;
     GC_ARG(iter >= 1, "iter must be >= 1");
-    int it = 0;
-    float res = 0.f;
     void *ws = nullptr;
-    if ((st = scratch_arena(cg_bytes(1, nx, ny, nz), &ws))) return st;
-    st = cg_solve(d_phi, d_phi, 1, nx, ny, nz, iter, end_res, &it, &res, ws, 0);
+    if ((st = scratch_arena(cg_bytes(m, nx, ny, nz), &ws))) return st;
+    st = cg_solve(d_phi, d_phi, m, nx, ny, nz, iter, end_res, f, final_iter, final_res, ws, 0);
     if (st) return st;
     GC_HIP(hipStreamSynchronize(0));
-    if (final_iter) *final_iter = it;
-    if (final_res) *final_res = res;
+    return GPUCAD_OK;
+}
+
+int gpucad_svl_cg(float *d_phi, int32_t nx, int32_t ny, int32_t nz, int32_t iter, float end_res,
+                  int32_t *final_iter, float *final_res) {
+    CgForm f;
+    return svl_cg(d_phi, 1, nx, ny, nz, iter, end_res, &f, final_iter, final_res);
+}
+
+int gpucad_svl_cg_form(float *d_phi, int32_t m, int32_t nx, int32_t ny, int32_t nz, int32_t iter,
+                       float end_res, int32_t form, float wait_first_ms, float wait_ms,
+                       int32_t *final_iter, float *final_res, int32_t *how) {
+    clear_error();
+    GC_ARG(m >= 1 && m <= kMaxRhs, "m must be in [1, %d]", kMaxRhs);
+    GC_ARG(form >= CgForm::kAuto && form <= CgForm::kChip, "unknown form %d", form);
+    // (a longer wait than the default would hold the device's other work)
+    const float most = (float)kChipWaitTicks / 1e5f;
+    GC_ARG(wait_first_ms <= most && wait_ms <= most, "a wait is at most %g ms", (double)most);
+    CgForm f;
+    f.form = form;
+    const auto ticks = [](float ms) { return ms < 0.f ? (int64_t)-1 : (int64_t)(ms * 1e5f); };
+    if (wait_first_ms != 0.f) f.wait_first = ticks(wait_first_ms);
+    if (wait_ms != 0.f) f.wait_others = ticks(wait_ms);
+    int st = svl_cg(d_phi, m, nx, ny, nz, iter, end_res, &f, final_iter, final_res);
+    if (st || !how) return st;
+    int cus = 0;
+    if ((st = cg_cus(&cus))) return st;
+    const ChipPlan p = chip_plan(nx, ny, nz, m, cus);
+    how[0] = f.solved_by;
+    how[1] = p.ty;
+    how[2] = p.tz;
+    how[3] = p.ty ? ((nz + p.tz - 1) / p.tz + 3) / 4 * 4 : 0;
+    how[4] = p.ty > 1 ? ((nz + p.tz - 1) / p.tz + p.threads / nx - 1) / (p.threads / nx) : 0;
     return GPUCAD_OK;
 }
 
@@ -1850,7 +1902,8 @@ int gpucad_svl_field(const gc_svl_params *p, const float *d_period, const gc_flo
     int iters[3] = {0, 0, 0};
     float res[3] = {0.f, 0.f, 0.f};
     const float tol = p->cg_end_res / (float)(3 * std::max(1, p->range));
-    st = cg_solve(phi, phi, 3, p->nx, p->ny, p->nz, p->cg_max_iter, tol, iters, res,
+    CgForm form;
+    st = cg_solve(phi, phi, 3, p->nx, p->ny, p->nz, p->cg_max_iter, tol, &form, iters, res,
                   (char *)ws + vec, s);
     if (st) return st;
     const Up u = {p->nx, p->ny, p->nz, p->fx, p->fy, p->fz, p->fine_dx, p->fine_dy, p->fine_dz};

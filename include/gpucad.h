@@ -405,6 +405,19 @@ int gpucad_svl_matvec(const float *d_d, float *d_q, int32_t nx, int32_t ny, int3
  * device (no host round trip per iteration). */
 int gpucad_svl_cg(float *d_phi, int32_t nx, int32_t ny, int32_t nz, int32_t iter, float end_res,
                   int32_t *final_iter, float *final_res);
+/* The same for m right-hand sides (1..4; m vectors of nx*ny*nz in a row,
+ * solved together; final_iter and final_res hold m values) with the form of
+ * the solve given, for tests and timings.  form 0: as gpucad_svl_cg chooses;
+ * 1: two launches per iteration; 2: one launch with its vectors on the chip
+ * (GPUCAD_E_ARG where the grid does not fit), by two launches if that gives
+ * up.  wait_first_ms and wait_ms are the longest waits of each right-hand
+ * side's first tile and of the other tiles on the chip (0: the default, which
+ * they may not exceed; negative: the first wait ends at once).  how, if not
+ * NULL, receives the form that solved (1 or 2), the tiles along y and z, the
+ * planes of a tile rounded up to 4, and the passes over a y halo. */
+int gpucad_svl_cg_form(float *d_phi, int32_t m, int32_t nx, int32_t ny, int32_t nz, int32_t iter,
+                       float end_res, int32_t form, float wait_first_ms, float wait_ms,
+                       int32_t *final_iter, float *final_res, int32_t how[5]);
 /* Gratings::VecSMultAdd_lattice (Gratings.h:37, Gratings.cu:73-94, 977-985):
  * v = a1 v + a2 w over n points. */
 int gpucad_svl_axpby(float *d_v, float a1, const float *d_w, float a2, uint64_t n);

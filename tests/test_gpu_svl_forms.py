@@ -1,0 +1,101 @@
+"""The phase solve's two forms against each other and the oracle: a solve on the
+chip counts as done only when every tile wrote its part, a solve that gives up
+is made by two launches from the same right-hand sides, and every kernel of
+the chip form with one to three passes over a tile's y halo.
+
+Both forms do the oracle's arithmetic per point, and alpha and beta are sums
+in FP64 rounded once, so they differ from the oracle's by one rounding now and
+then (6e-8 of a coefficient): over at most 20 iterations the solutions agree
+within 1e-4 of the largest value."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TWO_LAUNCH, ON_CHIP = 1, 2
+
+
+def solve(gc, dev, b, dims, iters, end_res, form=0, wait_first=0.0, wait=0.0):
+    """b: (m, n) right-hand sides; returns x (m, n), iterations, residuals, how."""
+    m = len(b)
+    d = torch.from_numpy(np.ascontiguousarray(b)).to(dev)
+    it, res, how = (C.c_int32 * m)(), (C.c_float * m)(), (C.c_int32 * 5)()
+    gc.check(gc.lib.gpucad_svl_cg_form(gc.ptr(d), m, *dims, iters, end_res, form, wait_first, wait,
+                                       it, res, how))
+    return d.cpu().numpy(), list(it), list(res), list(how)
+
+
+def rhs(orc, dims, m):
+    ijk = ((1, -2, 1), (0, 1, 0), (2, 0, -1), (0, 0, 1))
+    return np.stack([orc.svl_finding_phi(*dims, *ijk[a], lattice_type="b", uniform_type=0,
+                                         const_period=9.0) for a in range(m)])
+
+
+@pytest.mark.parametrize("m", [1, 3])
+@pytest.mark.parametrize("first", [0.0, -1.0], ids=["first tile waits", "no tile waits"])
+def test_a_tile_that_leaves_makes_the_solve_unfinished(gc, orc, dev, m, first):
+    dims = (40, 24, 40)
+    b = rhs(orc, dims, m)
+    zero = np.zeros_like(b)
+    for c, iters, end_res in ((zero, 50, 0.01), (b, 1, 0.0), (b, 50, 1e9), (b, 12, 0.0)):
+        want = solve(gc, dev, c, dims, iters, end_res, TWO_LAUNCH)
+        # (leaves another solution where the next solve keeps its own)
+        assert solve(gc, dev, b, dims, 12, 0.0, ON_CHIP)[3][0] == ON_CHIP
+        # the other tiles post their sums and leave at their first wait
+        got = solve(gc, dev, c, dims, iters, end_res, ON_CHIP, first, -1.0)
+        assert got[3][0] == TWO_LAUNCH
+        assert np.array_equal(got[0], want[0]) and got[1:3] == want[1:3]
+
+
+# dims, m, planes of a tile rounded up to 4, passes over a y halo
+PLANS = [((12, 12, 12), 1, 4, 1), ((61, 57, 70), 1, 8, 1), ((255, 33, 80), 1, 8, 2),
+         ((90, 90, 90), 3, 12, 1), ((120, 120, 120), 1, 12, 2), ((128, 128, 128), 2, 16, 2),
+         ((119, 101, 93), 3, 16, 2), ((150, 150, 150), 1, 16, 3), ((110, 110, 110), 3, 20, 3),
+         ((120, 120, 120), 3, 24, 3), ((33, 37, 50), 4, 4, 1)]
+
+
+@pytest.mark.parametrize("dims,m,planes,passes", PLANS)
+def test_the_forms_agree(gc, orc, dev, dims, m, planes, passes):
+    b = rhs(orc, dims, m)
+    if m > 1:
+        b[-1] *= np.float32(2.0 ** -9)  # stops before the others
+    end_res = float(np.linalg.norm(b[-1].astype(np.float64))) * 0.7
+    chip = solve(gc, dev, b, dims, 9, end_res, ON_CHIP)
+    assert chip[3][0] == ON_CHIP and chip[3][3:] == [planes, passes]
+    two = solve(gc, dev, b, dims, 9, end_res, TWO_LAUNCH)
+    assert two[3][0] == TWO_LAUNCH
+    assert chip[1] == two[1]
+    for s in range(m):
+        xo, ito, reso = orc.svl_cg(b[s], *dims, iters=9, end_res=end_res)
+        for x, it, res, _ in (chip, two):
+            assert it[s] == ito
+            assert abs(res[s] - reso) <= 1e-4 * reso
+            assert np.max(np.abs(x[s] - xo)) <= 1e-4 * np.max(np.abs(xo))
+
+
+@pytest.mark.parametrize("dims,m", [((520, 40, 30), 3), ((170, 170, 170), 1)])
+def test_grids_past_the_chip(gc, orc, dev, dims, m):
+    """Rows too wide for a tile, or too many points: several right-hand sides
+    and steps per workgroup in the two-launch form."""
+    b = rhs(orc, dims, m)
+    with pytest.raises(gc.GpucadError):
+        solve(gc, dev, b, dims, 9, 0.0, ON_CHIP)
+    x, it, res, how = solve(gc, dev, b, dims, 9, 0.0)
+    assert how[:3] == [TWO_LAUNCH, 0, 0]
+    for s in range(m):
+        xo, ito, reso = orc.svl_cg(b[s], *dims, iters=9, end_res=0.0)
+        assert it[s] == ito and abs(res[s] - reso) <= 1e-4 * reso
+        assert np.max(np.abs(x[s] - xo)) <= 1e-4 * np.max(np.abs(xo))
+
+
+def test_waits_are_bounded(gc, dev):
+    d = torch.zeros(64, dtype=torch.float32, device=dev)
+    for first, others in ((1e9, 0.0), (0.0, float("inf")), (float("nan"), 0.0)):
+        assert gc.lib.gpucad_svl_cg_form(gc.ptr(d), 1, 4, 4, 4, 4, 0.0, 0, first, others, None,
+                                         None, None) == gc.E_ARG
+    for m, form in ((0, 0), (5, 0), (1, 3), (1, -1)):
+        assert gc.lib.gpucad_svl_cg_form(gc.ptr(d), m, 4, 4, 4, 4, 0.0, form, 0.0, 0.0, None, None,
+                                         None) == gc.E_ARG
