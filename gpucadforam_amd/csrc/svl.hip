@@ -524,7 +524,15 @@ constexpr int kChipThreads = 1024;            // most threads of a tile's workgr
 constexpr int kChipZ = 24;                    // longest z run of a tile
 constexpr int kYPass = 3;                     // most passes over a halo layer of a y side
 constexpr size_t kChipLds = 160 * 1024 - 1024;  // LDS of a tile's d (1 KB: the sums)
-constexpr int64_t kChipWaitTicks = 20000000;  // longest wait: 0.2 s of the 100 MHz clock
+// Longest wait: 5 ms of the 100 MHz clock, about what a whole solve takes (1 ms
+// for 61^3, 6 ms for three of 120^3) and less than the two-launch form adds to it.
+constexpr int64_t kChipWaitTicks = 500000;
+// After a solve gave up, the next ones on its device go straight to two
+// launches: what held the CUs (another process, a long kernel of another
+// stream, a CU mask) mostly still does, and a loop over 62 harmonics would wait
+// in each.  One in 64 tries again, which costs such a loop 0.1 ms per solve.
+constexpr int kChipPause = 64;
+int g_chip_pause[64];  // solves left to take so, per device; under lock_device_calls()
 
 struct ChipArgs {
     int nx, ny, nz, m, ty, tz, G;  // G = ty * tz tiles per right-hand side
@@ -1000,10 +1008,11 @@ ChipPlan chip_plan(int nx, int ny, int nz, int m, int cus) {
     return best;
 }
 
-int cg_cus(int *cus) {
+int cg_cus(int *cus, int *device = nullptr) {
     int dev = 0;
     GC_HIP(hipGetDevice(&dev));
     GC_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev));
+    if (device) *device = dev;
     return GPUCAD_OK;
 }
 
@@ -1115,23 +1124,28 @@ size_t cg_bytes(int m, int nx, int ny, int nz) {
 }
 
 // Solves A x = b for m right-hand sides (b: m vectors of n, x written over
-// b when x == b) in ws (cg_bytes).  On the chip when the grid fits there;
-// otherwise, or when that gave up waiting, iterations of two launches in
-// chunks between host checks of the done flags (a finished right-hand side
-// leaves the kernels at their first test).  x is complete in stream order.
+// b when x == b) in ws (cg_bytes).  On the chip when the grid fits there and no
+// solve gave up lately; otherwise, or when this one gives up waiting, iterations
+// of two launches in chunks between host checks of the done flags (a finished
+// right-hand side leaves the kernels at their first test).  x is complete in
+// stream order.
 int cg_solve(const float *b, float *x, int m, int nx, int ny, int nz, int max_iter, float end_res,
              CgForm *f, int *iters, float *res, void *ws, hipStream_t st) {
     const uint64_t n = (uint64_t)nx * ny * nz;
     CgState h[kMaxRhs];
-    int cus = 0;
-    int rc = cg_cus(&cus);
+    int cus = 0, dev = 0;
+    int rc = cg_cus(&cus, &dev);
     if (rc) return rc;
     const ChipPlan chip = chip_plan(nx, ny, nz, m, cus);
     GC_ARG(f->form != CgForm::kChip || chip.ty, "the grid does not fit on the chip");
+    int &pause = g_chip_pause[dev];  // (the arena is for devices 0..63)
     bool solved = false;
-    if (chip.ty && f->form != CgForm::kTwoLaunch) {
+    if (chip.ty && (f->form == CgForm::kChip || (f->form == CgForm::kAuto && pause == 0))) {
         rc = cg_chip_solve(chip, b, x, m, nx, ny, nz, max_iter, end_res, *f, h, ws, &solved, st);
         if (rc) return rc;
+        pause = solved ? 0 : kChipPause;
+    } else if (chip.ty && f->form == CgForm::kAuto) {
+        --pause;
     }
     f->solved_by = solved ? CgForm::kChip : CgForm::kTwoLaunch;
     if (!solved) {

@@ -48,6 +48,7 @@ def test_a_tile_that_leaves_makes_the_solve_unfinished(gc, orc, dev, m, first):
         got = solve(gc, dev, c, dims, iters, end_res, ON_CHIP, first, -1.0)
         assert got[3][0] == TWO_LAUNCH
         assert np.array_equal(got[0], want[0]) and got[1:3] == want[1:3]
+    assert solve(gc, dev, b, dims, 12, 0.0, ON_CHIP)[3][0] == ON_CHIP
 
 
 # dims, m, planes of a tile rounded up to 4, passes over a y halo
@@ -99,3 +100,23 @@ def test_waits_are_bounded(gc, dev):
     for m, form in ((0, 0), (5, 0), (1, 3), (1, -1)):
         assert gc.lib.gpucad_svl_cg_form(gc.ptr(d), m, 4, 4, 4, 4, 0.0, form, 0.0, 0.0, None, None,
                                          None) == gc.E_ARG
+
+
+def test_a_solve_that_gave_up_is_not_tried_at_once(gc, orc, dev):
+    dims = (40, 24, 40)
+    b = rhs(orc, dims, 1)
+    want = solve(gc, dev, b, dims, 12, 0.0, TWO_LAUNCH)
+    assert solve(gc, dev, b, dims, 12, 0.0, ON_CHIP)[3][0] == ON_CHIP
+    assert solve(gc, dev, b, dims, 12, 0.0)[3][0] == ON_CHIP
+    assert solve(gc, dev, b, dims, 12, 0.0, 0, -1.0, -1.0)[3][0] == TWO_LAUNCH
+    by = []
+    for _ in range(65):  # nothing holds the CUs any more
+        x, it, res, how = solve(gc, dev, b, dims, 12, 0.0)
+        assert np.array_equal(x, want[0]) or how[0] == ON_CHIP
+        by.append(how[0])
+    assert by == [TWO_LAUNCH] * 64 + [ON_CHIP]
+    # a solve on the chip that the caller asked for and that ends clears it too
+    assert solve(gc, dev, b, dims, 12, 0.0, 0, -1.0, -1.0)[3][0] == TWO_LAUNCH
+    assert solve(gc, dev, b, dims, 12, 0.0)[3][0] == TWO_LAUNCH
+    assert solve(gc, dev, b, dims, 12, 0.0, ON_CHIP)[3][0] == ON_CHIP
+    assert solve(gc, dev, b, dims, 12, 0.0)[3][0] == ON_CHIP
