@@ -699,19 +699,19 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
     auto face = [=](int tile, int f) {
         return a.faces + (((uint64_t)s * a.G + tile) * 4 + f) * a.face_words;
     };
-    // Past the grid's ends along z the halo holds 4 d of the point whose -d the
+    // Past the grid's ends along z the halo holds the point whose -d the
     // operator takes there (axis_terms: rows 0, 1, nz - 2, nz - 1 have -d(1),
     // -d(0), -d(nz - 1), -d(nz - 2) in the place of -0.25 d two planes off), so
-    // every plane has the one form -0.25 d(-2) - 0.25 d(+2).
+    // every plane has the one form k d(-2) + k' d(+2).
     auto ghosts = [&](int n) {  // from the thread's own column
         const int xy = here(column), c = at(xy, 0), cz = at_z(0, 0, xy);
         if (!zlo && own) {
-            lds_d[cz] = 4.0f * lds_d[c];
-            lds_d[cz + by * nx] = 4.0f * lds_d[c + ps];
+            lds_d[cz] = lds_d[c];
+            lds_d[cz + by * nx] = lds_d[c + ps];
         }
         if (!zhi && own) {
-            lds_d[cz + 2 * by * nx] = 4.0f * lds_d[c + (n - 1) * ps];
-            lds_d[cz + 3 * by * nx] = 4.0f * lds_d[c + (n - 2) * ps];
+            lds_d[cz + 2 * by * nx] = lds_d[c + (n - 1) * ps];
+            lds_d[cz + 3 * by * nx] = lds_d[c + (n - 2) * ps];
         }
     };
     // step z exists: only the last four steps can be past the run
@@ -820,6 +820,7 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
             const int ox2 = ax.o2, ox3 = ax.o3, oy2 = ay.o2 * nx, oy3 = ay.o3 * nx;
             const float wxy = ax.w + ay.w;
             const int lo_edge = here_uniform(zlo ? -1 : 2), hi_edge = here_uniform(zhi ? KZ : bz - 2);
+            const float klo = lo_edge > 0 ? -1.0f : -0.25f;
             float dm2 = lds_d[at_z(0, 1, xy)], dm1 = lds_d[at_z(0, 0, xy)];
             float dc = lds_d[c], dp1 = lds_d[c + ps];
             // two planes up: in the tile, in its halo, then past both (not used)
@@ -832,8 +833,9 @@ __global__ void __launch_bounds__(kChipThreads) cg_chip_kernel(ChipArgs a) {
                 v = v + ax.k3 * lds_d[c + ox3];
                 v = v + ay.k2 * lds_d[c + oy2];
                 v = v + ay.k3 * lds_d[c + oy3];
-                v = v + -0.25f * dm2;
-                v = v + -0.25f * dp2;
+                v = v + (z < 2 ? klo : -0.25f) * dm2;
+                // (the last two planes of a run are past KZ - 7)
+                v = v + (z >= KZ - 6 && z >= hi_edge ? -1.0f : -0.25f) * dp2;
                 asm volatile("" : "+v"(v));  // (computed here, not where it is used)
                 q[z] = v;
                 if (GC_IN_RUN(z, n)) acc += (double)dc * (double)v;

@@ -120,3 +120,18 @@ def test_a_solve_that_gave_up_is_not_tried_at_once(gc, orc, dev):
     assert solve(gc, dev, b, dims, 12, 0.0)[3][0] == TWO_LAUNCH
     assert solve(gc, dev, b, dims, 12, 0.0, ON_CHIP)[3][0] == ON_CHIP
     assert solve(gc, dev, b, dims, 12, 0.0)[3][0] == ON_CHIP
+
+
+@pytest.mark.parametrize("dims", [(8, 6, 5), (12, 20, 40), (64, 40, 24)])
+def test_the_largest_values(gc, orc, dev, dims):
+    """A constant close to the type's largest value is in the operator's null
+    space, so no term of it may overflow: d.q is 0 and the step infinite."""
+    b = np.full((1, dims[0] * dims[1] * dims[2]), 1.125 * 2.0 ** 126, np.float32)
+    with np.errstate(all="ignore"):
+        xo, ito, reso = orc.svl_cg(b[0], *dims, iters=5, end_res=0.0)
+    assert np.all(np.isposinf(xo)) and np.isnan(reso)
+    for form in (TWO_LAUNCH, ON_CHIP):
+        x, it, res, how = solve(gc, dev, b, dims, 5, 0.0, form)
+        assert how[0] == form
+        assert it == [ito] and np.isnan(res[0])
+        assert np.array_equal(x[0], xo)
