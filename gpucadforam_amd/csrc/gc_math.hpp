@@ -43,11 +43,11 @@ __device__ __forceinline__ float cos_rev(float r, float quarter = 0.25f) {
 
 // sin(2*pi*a), a = r - rint(r) in [-1/2, 1/2], reflected into [-1/4, 1/4]:
 // sin(2*pi*a) = sin(2*pi*(sign(a)/2 - a)); both steps are exact (Sterbenz).
-// The reflection is the smaller of |a| and 1/2 - |a| with a's sign.
+// The reflection is the middle one of a, 1/2 - a and -1/2 - a: a itself up to
+// |a| = 1/4, then the one of a's sign (+0 at both a = 1/2 and a = -1/2).
 __device__ __forceinline__ float sin_rev(float r) {
     float a = r - __builtin_rintf(r);
-    float m = __builtin_fminf(__builtin_fabsf(a), 0.5f - __builtin_fabsf(a));
-    return sin2pi_reduced(__builtin_copysignf(m, a));
+    return sin2pi_reduced(__builtin_amdgcn_fmed3f(a, 0.5f - a, -0.5f - a));
 }
 
 // x in a vector register from here on
