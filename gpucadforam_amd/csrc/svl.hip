@@ -1288,6 +1288,10 @@ __global__ void svl_acc_kernel(float *svl, const float2 *g, uint64_t n, const fl
 // lane: the coefficients (LDS broadcasts) and the row's taps serve all four, and
 // the rows' addresses are uniform.  240^3 from 120^3, 62 harmonics:
 // 1081 -> 150 us.
+// PACK: rows of up to 128 points, several of them in a wave, each on a power of
+// two of its lanes; longer rows are split over gridDim.y.  Calls on 262144 rows
+// of 8 points: 530 us with a row per wave, 81 so (250 with a thread per point);
+// on 16 rows of 100000: 1640 us with a wave per row, 79 so.
 // ---------------------------------------------------------------------------
 constexpr int kMaxRange = 4;  // (2r+1)^3 <= 729 coefficients
 constexpr int kSvlPoints = 4;  // fine points per lane
@@ -1302,11 +1306,11 @@ __device__ __forceinline__ Cf cmulf(Cf a, Cf b) {
 // LDS floats of one (j, k) pair: c_0, then c_i + c_-i and i (c_i - c_-i) for i = 1..R
 constexpr int svl_pair_floats(int r) { return 2 + 4 * r; }
 
-template <int R>
+template <int R, bool PACK>
 __global__ void __launch_bounds__(256) svl_field_kernel(const float *phix, const float *phiy,
                                                         const float *phiz, Up u,
                                                         const float2 *coeffs, int harmonics,
-                                                        float *svl) {
+                                                        uint32_t row_lanes_log2, float *svl) {
     constexpr int kSide = 2 * R + 1, kPair = svl_pair_floats(R), P = kSvlPoints;
     __shared__ float s_c[kSide * kSide * kPair];
     auto coeff = [&](int i, int jk) {  // 0 past the harmonics
@@ -1334,19 +1338,27 @@ __global__ void __launch_bounds__(256) svl_field_kernel(const float *phix, const
     const uint32_t nrows = (uint32_t)u.fy * (uint32_t)u.fz;
     const int64_t crow = u.nx, cplane = (int64_t)u.nx * u.ny;
     const bool wide = (u.fx & 3) == 0 && ((uintptr_t)svl & 15u) == 0;
-    for (int x0 = 0; x0 < u.fx; x0 += 64 * P) {
-        const int x = x0 + (int)lane * P;
+    // a wave's rows, the lane's one of them and its place in it
+    const uint32_t wave_rows = PACK ? 64u >> row_lanes_log2 : 1u;
+    const uint32_t lane_row = PACK ? lane >> row_lanes_log2 : 0u;
+    const uint32_t row_lane = PACK ? lane & ((1u << row_lanes_log2) - 1u) : lane;
+    for (int64_t x0 = (int64_t)blockIdx.y * 64 * P; x0 < u.fx; x0 += (int64_t)gridDim.y * 64 * P) {
+        const int64_t x = x0 + (int64_t)row_lane * P;
+        const int points = (int)min(max((int64_t)u.fx - x, (int64_t)0), (int64_t)P);
         uint32_t i0[P], i1[P];
         float w1[P], w0[P];
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            const Tap t = tap(min(x + p, u.fx - 1), u.hx, u.nx);
+            const Tap t = tap((int)min(x + p, (int64_t)u.fx - 1), u.hx, u.nx);
             i0[p] = (uint32_t)t.i0;
             i1[p] = (uint32_t)t.i1;
             w1[p] = t.w;
             w0[p] = 1.0f - t.w;
         }
-        for (uint32_t row = blockIdx.x * 4 + wave; row < nrows; row += gridDim.x * 4) {
+        for (uint64_t first = (uint64_t)(blockIdx.x * 4 + wave) * wave_rows; first < nrows;
+             first += (uint64_t)gridDim.x * 4 * wave_rows) {
+            const bool in = !PACK || first + lane_row < nrows;
+            const uint32_t row = (uint32_t)(in ? first + lane_row : first);
             const uint32_t fz = row / (uint32_t)u.fy, fy = row - fz * (uint32_t)u.fy;
             const Tap ty = tap((int)fy, u.hy, u.ny), tz = tap((int)fz, u.hz, u.nz);
             // Phi at the lane's points: lerps along x, then y, then z (sample3); a
@@ -1427,12 +1439,12 @@ __global__ void __launch_bounds__(256) svl_field_kernel(const float *phix, const
                 }
             }
             float *o = svl + (uint64_t)row * u.fx + x;
-            if (wide && x < u.fx) {
+            if (wide && points && in) {
                 *(float4 *)o = make_float4(acc[0], acc[1], acc[2], acc[3]);
             } else {
 #pragma unroll
                 for (int p = 0; p < P; ++p)
-                    if (x + p < u.fx) o[p] = acc[p];
+                    if (p < points && in) o[p] = acc[p];
             }
         }
     }
@@ -1924,14 +1936,25 @@ int gpucad_svl_field(const gc_svl_params *p, const float *d_period, const gc_flo
     if (st) return st;
     const Up u = {p->nx, p->ny, p->nz, p->fx, p->fy, p->fz, p->fine_dx, p->fine_dy, p->fine_dz};
     typedef void (*FieldKernel)(const float *, const float *, const float *, Up, const float2 *,
-                                int, float *);
-    static const FieldKernel kField[kMaxRange + 1] = {svl_field_kernel<0>, svl_field_kernel<1>,
-                                                      svl_field_kernel<2>, svl_field_kernel<3>,
-                                                      svl_field_kernel<4>};
+                                int, uint32_t, float *);
+    static const FieldKernel kField[2][kMaxRange + 1] = {
+        {svl_field_kernel<0, false>, svl_field_kernel<1, false>, svl_field_kernel<2, false>,
+         svl_field_kernel<3, false>, svl_field_kernel<4, false>},
+        {svl_field_kernel<0, true>, svl_field_kernel<1, true>, svl_field_kernel<2, true>,
+         svl_field_kernel<3, true>, svl_field_kernel<4, true>}};
+    // lanes of a row, workgroups along a row and over the rows (about 4096 in all)
     const uint64_t rows = (uint64_t)p->fy * p->fz;
-    hipLaunchKernelGGL(kField[p->range], dim3((unsigned)std::min<uint64_t>((rows + 3) / 4, 4096)),
-                       dim3(256), 0, s, phi, phi + n, phi + 2 * n, u, (const float2 *)d_coeffs,
-                       p->harmonics, d_svl);
+    const uint64_t lanes = ((uint64_t)p->fx + kSvlPoints - 1) / kSvlPoints;
+    const bool pack = lanes <= 32;
+    uint32_t lanes_log2 = 0;
+    while ((1ull << lanes_log2) < lanes) ++lanes_log2;
+    const uint64_t along = (lanes + 63) / 64;
+    const uint64_t wave_rows = pack ? 64 >> lanes_log2 : 1;
+    const uint64_t over = (rows + 4 * wave_rows - 1) / (4 * wave_rows);
+    const dim3 wgs((unsigned)std::min<uint64_t>(over, std::max<uint64_t>(1, 4096 / along)),
+                   (unsigned)std::min<uint64_t>(along, 4096));
+    hipLaunchKernelGGL(kField[pack][p->range], wgs, dim3(256), 0, s, phi, phi + n, phi + 2 * n, u,
+                       (const float2 *)d_coeffs, p->harmonics, lanes_log2, d_svl);
     GC_CHECK_LAUNCH();
     GC_HIP(hipStreamSynchronize(s));
     if (result) {

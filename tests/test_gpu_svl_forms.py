@@ -135,3 +135,30 @@ def test_the_largest_values(gc, orc, dev, dims):
         assert how[0] == form
         assert it == [ito] and np.isnan(res[0])
         assert np.array_equal(x[0], xo)
+
+
+@pytest.mark.parametrize("r", [0, 2, 4])
+@pytest.mark.parametrize("fine", [(1, 9, 70), (3, 70, 5), (4, 33, 9), (5, 7, 37), (8, 40, 8),
+                                  (17, 5, 13), (31, 8, 8), (64, 3, 5), (65, 6, 7), (127, 9, 2),
+                                  (128, 3, 11), (129, 3, 11), (256, 2, 5), (1030, 2, 3),
+                                  (40000, 1, 2)], ids=lambda f: "x".join(map(str, f)))
+def test_synthesis_rows(gc, orc, dev, fine, r):
+    """Fine rows of every share of a wave and longer than several, against the
+    same points of a synthesis that has them in the middle of longer rows:
+    the same taps and arithmetic, so the same bits."""
+    c = np.random.default_rng(23).standard_normal(((2 * r + 1) ** 3, 2)).astype(np.float32)
+
+    def run(fx):
+        p = gc.svl_params(9, lattice_type="b", const_period=7.0, range_=r, cg_max_iter=12,
+                          harmonics=(2 * r + 1) ** 3, cg_end_res=1e-6)
+        p.ny, p.nz, p.fx, p.fy, p.fz = 6, 5, fx, fine[1], fine[2]
+        p.fine_dx = 8.0 / fine[0]
+        svl, _ = gc.svl_field(p, torch.from_numpy(c).to(dev))
+        return svl.cpu().numpy().reshape(fine[2], fine[1], fx), p
+
+    got, p = run(fine[0])
+    longer, _ = run(fine[0] + 300)
+    assert np.array_equal(got.view(np.uint32), longer[:, :, :fine[0]].copy().view(np.uint32))
+    if fine[0] <= 256:
+        ref, _, _ = orc.svl_field(p, c, None)
+        assert np.max(np.abs(got.reshape(-1) - ref)) < 2e-2 * max(1e-3, np.max(np.abs(ref)))
