@@ -1031,7 +1031,10 @@ ChipLayout chip_layout(const ChipPlan &p, int m) {
     return l;
 }
 
-// Vectors of the two-launch form: 5 slots of m vectors, partial sums, states.
+// Workspace of a solve: slots of m vectors, phi in slot 0, r in slot 1 (where
+// the caller may have put b), q, d0 and d1 of the two-launch form in 2 to 4
+// and its partial sums and states behind them; the chip form's exchange words
+// begin at slot 2.
 struct CgLayout {
     uint64_t slot, bytes;
     int G;
@@ -1057,16 +1060,15 @@ struct CgForm {
     int solved_by = 0;
 };
 
-// The solve on the chip: m right-hand sides b, solutions into x (x may be b),
-// ws holding m * n floats and the exchange words.  *solved says whether every
-// tile ran to its end.
+// The solve on the chip: m right-hand sides b, solutions into x (x may be b) or
+// left in slot 0 of ws (x == ws).  *solved says whether every tile ran to its
+// end.
 int cg_chip_solve(const ChipPlan &p, const float *b, float *x, int m, int nx, int ny, int nz,
                   int max_iter, float end_res, const CgForm &f, CgState *h, void *ws, bool *solved,
                   hipStream_t st) {
     const ChipLayout l = chip_layout(p, m);
     const uint64_t n = (uint64_t)nx * ny * nz;
-    const uint64_t vec = (m * n * sizeof(float) + 255) & ~uint64_t(255);
-    char *w = (char *)ws + vec;
+    char *w = (char *)ws + 2 * cg_layout(n, m).slot;
     ChipArgs a;
     a.nx = nx;
     a.ny = ny;
@@ -1107,26 +1109,29 @@ int cg_chip_solve(const ChipPlan &p, const float *b, float *x, int m, int nx, in
     GC_HIP(hipStreamSynchronize(st));
     for (int s = 0; s < m; ++s)
         if (h[s].tiles != (uint32_t)a.G) return GPUCAD_OK;
-    GC_HIP(hipMemcpyAsync(x, a.phi, m * n * sizeof(float), hipMemcpyDeviceToDevice, st));
+    if (x != a.phi)
+        GC_HIP(hipMemcpyAsync(x, a.phi, m * n * sizeof(float), hipMemcpyDeviceToDevice, st));
     *solved = true;
     return GPUCAD_OK;
 }
+
+// b's place in the workspace ws of a solve, for a caller without its own
+float *cg_rhs(void *ws, uint64_t n, int m) { return (float *)((char *)ws + cg_layout(n, m).slot); }
 
 // Workspace of cg_solve.
 size_t cg_bytes(int m, int nx, int ny, int nz) {
     const uint64_t n = (uint64_t)nx * ny * nz;
     int cus = 0;
     if (cg_cus(&cus)) cus = 0;
-    size_t bytes = cg_layout(n, m).bytes;
+    const CgLayout l = cg_layout(n, m);
+    size_t bytes = l.bytes;
     const ChipPlan p = chip_plan(nx, ny, nz, m, cus);
-    if (p.ty)
-        bytes = std::max<size_t>(bytes, ((m * n * sizeof(float) + 255) & ~uint64_t(255)) +
-                                            chip_layout(p, m).bytes);
+    if (p.ty) bytes = std::max<size_t>(bytes, 2 * l.slot + chip_layout(p, m).bytes);
     return bytes;
 }
 
-// Solves A x = b for m right-hand sides (b: m vectors of n, x written over
-// b when x == b) in ws (cg_bytes).  On the chip when the grid fits there and no
+// Solves A x = b for m right-hand sides (b: m vectors of n, also at cg_rhs; x
+// written over b when x == b, or left in ws when x == ws) in ws (cg_bytes).  On the chip when the grid fits there and no
 // solve gave up lately; otherwise, or when this one gives up waiting, iterations
 // of two launches in chunks between host checks of the done flags (a finished
 // right-hand side leaves the kernels at their first test).  x is complete in
@@ -1191,7 +1196,8 @@ int cg_solve(const float *b, float *x, int m, int nx, int ny, int nz, int max_it
         for (int s = 0; s < m; ++s)
             if (!h[s].done)
                 return fail(GPUCAD_E_HIP, "internal: CG did not stop by iteration %d", max_iter);
-        GC_HIP(hipMemcpyAsync(x, a.phi, m * n * sizeof(float), hipMemcpyDeviceToDevice, st));
+        if (x != a.phi)
+            GC_HIP(hipMemcpyAsync(x, a.phi, m * n * sizeof(float), hipMemcpyDeviceToDevice, st));
     }
     for (int s = 0; s < m; ++s) {
         if (iters) iters[s] = h[s].iters;
@@ -1472,6 +1478,9 @@ __device__ __forceinline__ double2 cmuld(double2 a, double2 b) {
     return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
 }
 constexpr int kDftRows = 4;  // rows per wave: a wave's twiddles serve all of them
+// Rows whose sums are held at a time (16 bytes per row and i: at most 21 MB; a
+// cell of 512^3 has this many).
+constexpr uint32_t kDftPiece = 1u << 18;
 
 // rows[i * nrows + row] = sum over x of f(x, row) e^{-2 pi i ix/nx}, i = 0..R
 template <int R>
@@ -1511,17 +1520,19 @@ __global__ void __launch_bounds__(256) dft_rows_kernel(const float *cell, int nx
         }
 }
 
-// workgroup (i, j, k): the rows' sums over y and z; writes (i, j, k) and its
-// mirror image (-i, -j, -k)
-__global__ void __launch_bounds__(256) dft_planes_kernel(const double2 *rows, int ny, int nz,
-                                                         int range, double cells, float2 *out) {
+// workgroup (i, j, k): the sums of rows first .. first + nrows over y and z,
+// added to the earlier pieces' in sum; after the last piece it writes (i, j, k)
+// and its mirror image (-i, -j, -k)
+__global__ void __launch_bounds__(256) dft_planes_kernel(const double2 *rows, uint32_t first,
+                                                         uint32_t nrows, bool last, int ny, int nz,
+                                                         int range, double cells, double2 *sum,
+                                                         float2 *out) {
     const int side = 2 * range + 1;
     const int j = (int)(blockIdx.x % side) - range, k = (int)(blockIdx.x / side) - range;
     const int i = (int)blockIdx.y;
-    const uint32_t nrows = (uint32_t)ny * (uint32_t)nz;
     double re = 0.0, im = 0.0;
     for (uint32_t t = threadIdx.x; t < nrows; t += 256) {
-        const uint32_t z = t / (uint32_t)ny, y = t - z * (uint32_t)ny;
+        const uint32_t z = (first + t) / (uint32_t)ny, y = first + t - z * (uint32_t)ny;
         // the angle in periods (at most 2 range of them, so rounded to about 1e-15)
         const double a = (double)((int64_t)j * y) / (double)ny + (double)((int64_t)k * z) / (double)nz;
         double s, c;
@@ -1539,8 +1550,19 @@ __global__ void __launch_bounds__(256) dft_planes_kernel(const double2 *rows, in
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        const float vr = (float)(((sr[0] + sr[1]) + (sr[2] + sr[3])) / cells);
-        const float vi = (float)(((si[0] + si[1]) + (si[2] + si[3])) / cells);
+        double2 v = make_double2((sr[0] + sr[1]) + (sr[2] + sr[3]),
+                                 (si[0] + si[1]) + (si[2] + si[3]));
+        double2 *before = sum + blockIdx.x + gridDim.x * blockIdx.y;
+        if (first > 0) {
+            v.x += before->x;
+            v.y += before->y;
+        }
+        if (!last) {
+            *before = v;
+            return;
+        }
+        const float vr = (float)(v.x / cells);
+        const float vi = (float)(v.y / cells);
         auto at = [=](int a, int b, int c) {
             return (a + range) + side * ((b + range) + side * (c + range));
         };
@@ -1917,13 +1939,12 @@ int gpucad_svl_field(const gc_svl_params *p, const float *d_period, const gc_flo
     // the three unit right-hand sides, solved together; a harmonic's residual
     // is at most (|i| + |j| + |k|) times theirs, so they are solved to
     // cg_end_res / (3 range) to meet cg_end_res for every harmonic
-    const uint64_t vec = (3 * n * sizeof(float) + 255) & ~uint64_t(255);
     void *ws = nullptr;
-    if ((st = scratch_arena(vec + cg_bytes(3, p->nx, p->ny, p->nz), &ws))) return st;
-    float *phi = (float *)ws;
+    if ((st = scratch_arena(cg_bytes(3, p->nx, p->ny, p->nz), &ws))) return st;
+    float *phi = (float *)ws, *b = cg_rhs(ws, n, 3);
     const int unit[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
     for (int a = 0; a < 3; ++a) {
-        hipLaunchKernelGGL(finding_phi_kernel, stride_grid(n), dim3(256), 0, s, phi + a * n,
+        hipLaunchKernelGGL(finding_phi_kernel, stride_grid(n), dim3(256), 0, s, b + a * n,
                            d_period, phi_args(p, unit[a][0], unit[a][1], unit[a][2]));
         GC_CHECK_LAUNCH();
     }
@@ -1931,9 +1952,11 @@ int gpucad_svl_field(const gc_svl_params *p, const float *d_period, const gc_flo
     float res[3] = {0.f, 0.f, 0.f};
     const float tol = p->cg_end_res / (float)(3 * std::max(1, p->range));
     CgForm form;
-    st = cg_solve(phi, phi, 3, p->nx, p->ny, p->nz, p->cg_max_iter, tol, &form, iters, res,
-                  (char *)ws + vec, s);
-    if (st) return st;
+    st = cg_solve(b, phi, 3, p->nx, p->ny, p->nz, p->cg_max_iter, tol, &form, iters, res, ws, s);
+    if (st) {
+        (void)hipStreamSynchronize(s);  // (the next call may have the arena on another stream)
+        return st;
+    }
     const Up u = {p->nx, p->ny, p->nz, p->fx, p->fy, p->fz, p->fine_dx, p->fine_dy, p->fine_dz};
     typedef void (*FieldKernel)(const float *, const float *, const float *, Up, const float2 *,
                                 int, uint32_t, float *);
@@ -1975,22 +1998,26 @@ int gpucad_unit_spectrum(const float *d_cell, int32_t nx, int32_t ny, int32_t nz
     if (st) return st;
     GC_ARG(range >= 0 && range <= kMaxRange, "range must be in [0, %d]", kMaxRange);
     const int side = 2 * range + 1;
-    const uint32_t nrows = (uint32_t)((uint64_t)ny * nz);
+    const uint32_t nrows = (uint32_t)((uint64_t)ny * nz), piece = std::min(nrows, kDftPiece);
+    const uint64_t nsums = (uint64_t)side * side * (range + 1);
     void *ws = nullptr;
-    st = scratch_arena((uint64_t)(range + 1) * nrows * sizeof(double2), &ws);
+    st = scratch_arena((nsums + (uint64_t)(range + 1) * piece) * sizeof(double2), &ws);
     if (st) return st;
-    double2 *rows = (double2 *)ws;
+    double2 *sums = (double2 *)ws, *rows = sums + nsums;
     typedef void (*RowsKernel)(const float *, int, uint32_t, double2 *);
     static const RowsKernel kRows[kMaxRange + 1] = {dft_rows_kernel<0>, dft_rows_kernel<1>,
                                                     dft_rows_kernel<2>, dft_rows_kernel<3>,
                                                     dft_rows_kernel<4>};
-    hipLaunchKernelGGL(kRows[range], dim3((nrows - 1) / (4 * kDftRows) + 1), dim3(256), 0, 0, d_cell,
-                       nx, nrows, rows);
-    GC_CHECK_LAUNCH();
-    hipLaunchKernelGGL(dft_planes_kernel, dim3((unsigned)(side * side), (unsigned)(range + 1)),
-                       dim3(256), 0, 0, rows, ny, nz, range, (double)nx * ny * nz,
-                       (float2 *)d_coeffs);
-    GC_CHECK_LAUNCH();
+    for (uint64_t r = 0; r < nrows; r += piece) {
+        const uint32_t first = (uint32_t)r, m = std::min(piece, nrows - first);
+        hipLaunchKernelGGL(kRows[range], dim3((m - 1) / (4 * kDftRows) + 1), dim3(256), 0, 0,
+                           d_cell + r * nx, nx, m, rows);
+        GC_CHECK_LAUNCH();
+        hipLaunchKernelGGL(dft_planes_kernel, dim3((unsigned)(side * side), (unsigned)(range + 1)),
+                           dim3(256), 0, 0, rows, first, m, r + m == nrows, ny, nz, range,
+                           (double)nx * ny * nz, sums, (float2 *)d_coeffs);
+        GC_CHECK_LAUNCH();
+    }
     GC_HIP(hipStreamSynchronize(0));
     return GPUCAD_OK;
 }
