@@ -130,22 +130,44 @@ int validate_lattice(const gc_lattice_params *p) {
 // the chip and its last wave.  With w = columns of bricks x planes the best run
 // grew like sqrt(w) in sweeps from 33 x 47 x 61 to 1024^3 (rotated: 8 planes of
 // 128^3, 10 of 203 x 149 x 181, 20 of 320 x 300 x 310; bent or with modes: 8 of
-// 100^3, 20 of 200^3, 48 of 400^3, 80 of 512^3); 0.12 sqrt(w) is within 5 % of
-// each.  Large rotated grids, whose four rows per lane need more columns,
-// are faster when five workgroups per CU take all of it at once, in runs of
-// w / 1300 planes (512^3: 161 us in runs of 112, 173 of 47, 166 of 48: long
-// runs are multiples of 16).  A lattice with neither rotation, bend nor modes
-// has little per-column work and is fastest in runs of 16 from 200^3 on
-// (512^3: 90.6 us, 99 in runs of 32 to 80).  With an eighth of the planes (a
-// fifth when rotated) and at least 16, as before: 40^3 5.0 us, now 3.1; rotated
-// 128^3 31.9, now 17.5; 203 x 149 x 181 44.4, now 29.0; 320 x 300 x 310 76.9,
-// now 60.
+// 100^3, 20 of 200^3); 0.12 sqrt(w) is within 5 % of each, up to the longest run
+// that pays (longest_z_run).  Large rotated grids, whose four rows per lane need
+// more columns, are faster when five workgroups per CU take all of it at once,
+// in runs of w / 1300 planes (512^3: 161 us in runs of 112, 173 of 47, 166 of 48:
+// long runs are multiples of 16).  With an eighth of the planes (a fifth when
+// rotated) and at least 16, as before: 40^3 5.0 us, now 3.1; rotated 128^3
+// 31.9, now 17.5; 203 x 149 x 181 44.4, now 29.0; 320 x 300 x 310 76.9, now 60.
+//
+// Without rotation the longest run goes by what a column costs before its first
+// point.  us at 512^3 and 1024^3 in runs of 16, 32, 80 and 96 (before: an eighth):
+//   nothing           97.7  100  101  104 (102)     741  803  778  776 (782)
+//   a primitive        109 96.2 97.4 99.2 (104)     842  775  770  759 (795)
+//   bend, primitive    116  105 99.4 99.7 (110)     934  826  773  770 (820)
+//   modes              158  125  101  104 (115)    1237  963  815  802 (807)
+// Past the 256 MB of the memory-side cache, rows that end inside a line need
+// shorter runs: the parts of a line that two bricks share meet in the L2, which
+// the active workgroups of an XCD, 1 KB each per plane, fill in 16 planes.  The
+// more a plane costs the closer together they run.  us of 620^3 in runs of
+// 12, 16, 24, 32 and 48 planes (before):
+//   nothing            179  238  302  320  332 (477)
+//   a primitive        211  201  180  309  330 (480)
+//   bend, primitive    238  219  198  191  327 (483)
+//   modes              323  289  247  221  325 (481)
+//   all three          375  327  285  267  236 (487)
+// and of 860^3 12 to 24 planes: 599 733 900; 548 514 824; 632 581 540.
+int longest_z_run(const gc_lattice_params *p) {
+    const bool bend = p->bend_radius > 0.f, prim = p->prim != GC_PRIM_NONE;
+    const bool cut = p->nx % 32 != 0 && (uint64_t)p->nx * p->ny * p->nz >= (1u << 26);
+    if (p->n_modes > 0) return !cut ? 96 : (prim ? 48 : 32);
+    if (prim) return bend ? (cut ? 24 : 80) : (cut ? 16 : 32);
+    return cut ? 12 : 16;
+}
+
 int default_z_run(const gc_lattice_params *p, int bricks_x, int bricks_y) {
     const bool rot = p->rot0 != 0.f || p->rot1 != 0.f;
-    const bool plain = !rot && !(p->bend_radius > 0.f) && p->n_modes == 0;
     const double w = (double)bricks_x * bricks_y * p->nz;
     const double best = std::max(0.12 * std::sqrt(w), rot ? w / 1300.0 : 0.0);
-    int run = (int)std::min(std::max(best + 0.5, 4.0), plain ? 16.0 : (double)kMaxLZ);
+    int run = (int)std::min(std::max(best + 0.5, 4.0), (double)(rot ? kMaxLZ : longest_z_run(p)));
     run = std::max(run, (p->nz + 65534) / 65535);  // (a launch's third dimension)
     if (run > 40) return (run + 15) / 16 * 16;     // (the caller bounds it by kMaxLZ)
     const int chunks = (p->nz + run - 1) / run;
@@ -154,14 +176,14 @@ int default_z_run(const gc_lattice_params *p, int bricks_x, int bricks_y) {
 
 // Whether a launch puts the bricks of a row on one XCD, where the lines and
 // sign words that they share are merged in its L2: rows that end inside a line
-// (500^3: 198 us plain and 228 rotated, 86 and 158 so), and without rotation
-// whole lines as well (512^3 93, so 85; the edit of 1024^3 3.73 ms, so 3.66).
-// Not rotated grids of whole lines (the edit of 512^3 337 us, so 342) nor fields
-// of the size of the L2s (128^3 edit 22.1 us, so 22.4).  The other launches
-// store with the non-temporal hint always (field_nt_store).
-bool rows_by_xcd(const gc_lattice_params *p, bool rot) {
-    const uint64_t points = (uint64_t)p->nx * p->ny * p->nz;
-    return points >= (1u << 24) && (!rot || p->nx % 32 != 0);
+// (500^3: 198 us plain and 228 rotated, 86 and 158 so).  Not rows of
+// whole lines, which share none: bent 512^3 107 us so, 94 without; 640^3 216
+// and 182; with a primitive 205 and 186, with modes 220 and 197 (each in its
+// launch's runs).  Not fields of the size of the L2s (128^3 edit 22.1 us, so
+// 22.4).  The other launches store with the non-temporal hint always
+// (field_nt_store).
+bool rows_by_xcd(const gc_lattice_params *p) {
+    return (uint64_t)p->nx * p->ny * p->nz >= (1u << 24) && p->nx % 32 != 0;
 }
 
 int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d_signs, float iso,
@@ -176,7 +198,7 @@ int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d
     if (lz > kMaxLZ) lz = kMaxLZ;
     const FieldConsts c = make_field_consts(p, iso, lz, (uint64_t)p->nx * p->ny * p->nz);
     const bool thick = p->n_modes > 0;
-    const bool by_xcd = rows_by_xcd(p, rot);
+    const bool by_xcd = rows_by_xcd(p);
     const auto pick = by_xcd ? (rot ? pick_tpms<true, true> : pick_tpms<true, false>)
                              : (rot ? pick_tpms<false, true> : pick_tpms<false, false>);
     FieldKernel k = pick(p->tpms, thick, c.prim, c.op);

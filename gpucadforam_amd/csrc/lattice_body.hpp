@@ -232,7 +232,6 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
     const int zn = min(c.lz, c.nz - z0);
 
     // ---- per-z table (one z per thread)
-    bool ztiny = false;  // a box's z distance in (0, 2^-48)
     for (int i = threadIdx.x; i < zn; i += 64 * kFieldWaves) {
         float *e = ztab + i * kZTab;
         float zf = (float)(z0 + i);
@@ -258,12 +257,10 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
         if (c.prim == GC_PRIM_SPHERE) {
             e[ZT_PRIMZ] = pz - c.pc[2];
         } else if (c.prim == GC_PRIM_BOX) {
-            const float bz = __builtin_fabsf(pz - c.pc[2]) - c.ph[2];
-            e[ZT_PRIMZ] = bz;
-            ztiny |= bz > 0.f && bz < 0x1p-48f;
+            e[ZT_PRIMZ] = __builtin_fabsf(pz - c.pc[2]) - c.ph[2];
         }
     }
-    const bool any_ztiny = __syncthreads_or(ztiny);
+    __syncthreads();
     const bool xin = x < c.nx;
 
     // ---- per-lane x quantities
@@ -390,9 +387,16 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
     // too) unless a column passes within 2^-48 of its centre, edge or corner
     // axis: then the wave takes the general root at every point.
     const int prim = PRIM == PRIM_ANY ? c.prim : PRIM;
-    bool general = !c.prim_plain || any_ztiny;
+    bool general = !c.prim_plain;
     if (prim != GC_PRIM_NONE) {
         bool near = false;
+        // (a box's z distances in (0, 2^-48): every wave looks at the table, since
+        // a vote of the workgroup takes two more barriers, 1 us of a 128^3 launch)
+        if (prim == GC_PRIM_BOX)
+            for (int i = lane; i < zn; i += 64) {
+                const float bz = ztab[i * kZTab + ZT_PRIMZ];
+                near |= bz > 0.f && bz < 0x1p-48f;
+            }
 #pragma unroll
         for (int r = 0; r < RY; ++r)
             near |= !(pxy[r] >= 0x1p-96f) && !(prim == GC_PRIM_BOX && pxy[r] == 0.0f);
