@@ -198,16 +198,18 @@ int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d
     if (lz > kMaxLZ) lz = kMaxLZ;
     const FieldConsts c = make_field_consts(p, iso, lz, (uint64_t)p->nx * p->ny * p->nz);
     const bool thick = p->n_modes > 0;
-    const bool by_xcd = rows_by_xcd(p);
+    dim3 grid((p->nx + 63) / 64, (p->ny + brick_y - 1) / brick_y, (p->nz + lz - 1) / lz);
+    GC_ARG(grid.y <= 65535 && grid.z <= 65535, "grid too large for one launch");
+    // (a launch holds fewer than 2^32 threads along x)
+    const bool by_xcd =
+        rows_by_xcd(p) && (rot || (uint64_t)grid.x * 8 * 64 * kFieldWaves <= 0xffffffffull);
     const auto pick = by_xcd ? (rot ? pick_tpms<true, true> : pick_tpms<true, false>)
                              : (rot ? pick_tpms<false, true> : pick_tpms<false, false>);
     FieldKernel k = pick(p->tpms, thick, c.prim, c.op);
-    dim3 grid((p->nx + 63) / 64, (p->ny + brick_y - 1) / brick_y, (p->nz + lz - 1) / lz);
     if (!rot && by_xcd) {  // (lattice_field_kernel)
         grid.x *= 8;
         grid.y = (grid.y + 7) / 8;
     }
-    GC_ARG(grid.y <= 65535 && grid.z <= 65535, "grid too large for one launch");
     hipLaunchKernelGGL(k, grid, dim3(64 * kFieldWaves), 0, stream, c, d_field, d_signs);
     GC_CHECK_LAUNCH();
     return GPUCAD_OK;
