@@ -139,11 +139,16 @@ int validate_lattice(const gc_lattice_params *p) {
 // 31.9, now 17.5; 203 x 149 x 181 44.4, now 29.0; 320 x 300 x 310 76.9, now 60.
 //
 // Without rotation the longest run goes by what a column costs before its first
-// point.  us at 512^3 and 1024^3 in runs of 16, 32, 80 and 96 (before: an eighth):
-//   nothing           97.7  100  101  104 (102)     741  803  778  776 (782)
-//   a primitive        109 96.2 97.4 99.2 (104)     842  775  770  759 (795)
-//   bend, primitive    116  105 99.4 99.7 (110)     934  826  773  770 (820)
-//   modes              158  125  101  104 (115)    1237  963  815  802 (807)
+// point.  us at 512^3 in runs of 8, 16, 32, 64 and 96 (before: an eighth):
+//   nothing            101  97.7  100  101  104 (102)
+//   a primitive        125   109 96.2 99.4 99.2 (104)
+//   bend, primitive    146   116  105  101 99.7 (110)
+//   modes              225   158  125  110  104 (115)
+// and with a row's bricks on one XCD, over 24 grids of 256^3 to 1024^3, against
+// an eighth: nothing 0.88 in runs of 12, 0.90 of 16; bend 0.88 of 16, 0.95 of 12;
+// primitive 0.93 of 24, 0.93 of 32, 0.98 of 16; bend and primitive 0.92 of 48,
+// 0.93 of 64 (1024^3 827 and 785); modes 0.98 of 48 and 64, 1.06 of 32.  They
+// differ by up to 10 % from one size to the next; edits, with their mesh, by 2 %.
 // Past the 256 MB of the memory-side cache, rows that end inside a line need
 // shorter runs: the parts of a line that two bricks share meet in the L2, which
 // the active workgroups of an XCD, 1 KB each per plane, fill in 16 planes.  The
@@ -158,9 +163,10 @@ int validate_lattice(const gc_lattice_params *p) {
 int longest_z_run(const gc_lattice_params *p) {
     const bool bend = p->bend_radius > 0.f, prim = p->prim != GC_PRIM_NONE;
     const bool cut = p->nx % 32 != 0 && (uint64_t)p->nx * p->ny * p->nz >= (1u << 26);
-    if (p->n_modes > 0) return !cut ? 96 : (prim ? 48 : 32);
-    if (prim) return bend ? (cut ? 24 : 80) : (cut ? 16 : 32);
-    return cut ? 12 : 16;
+    if (p->n_modes > 0) return cut && !prim ? 32 : (cut ? 48 : 64);
+    if (prim && bend) return cut ? 24 : 64;
+    if (prim) return cut ? 16 : 24;
+    return bend && !cut ? 16 : 12;
 }
 
 int default_z_run(const gc_lattice_params *p, int bricks_x, int bricks_y) {
@@ -176,14 +182,17 @@ int default_z_run(const gc_lattice_params *p, int bricks_x, int bricks_y) {
 
 // Whether a launch puts the bricks of a row on one XCD, where the lines and
 // sign words that they share are merged in its L2: rows that end inside a line
-// (500^3: 198 us plain and 228 rotated, 86 and 158 so).  Not rows of
-// whole lines, which share none: bent 512^3 107 us so, 94 without; 640^3 216
-// and 182; with a primitive 205 and 186, with modes 220 and 197 (each in its
-// launch's runs).  Not fields of the size of the L2s (128^3 edit 22.1 us, so
-// 22.4).  The other launches store with the non-temporal hint always
-// (field_nt_store).
-bool rows_by_xcd(const gc_lattice_params *p) {
-    return (uint64_t)p->nx * p->ny * p->nz >= (1u << 24) && p->nx % 32 != 0;
+// (500^3: 198 us plain and 228 rotated, 86 and 158 so), and without rotation
+// whole lines as well, whose sign words share lines (edits: 1024^3 4.76 ms with
+// the bricks over the XCDs, 4.67 so; 512^3 596 us, 582 so; 256 x 1024 x 1024 929,
+// 886 so).  Not rotated grids of whole lines (the edit of 512^3 337 us, so 342).
+// From 64 MB on: an edit of 128^3 took 22.1 us, so 22.4.  (Between them rows that
+// end inside a line gain too: 203^3 17.3 us, so 12.1; 252^3 28.1, so 15.0; rotated
+// 22.9 and 23.3, 34.1 and 29.2.)  The other launches store with the
+// non-temporal hint always (field_nt_store).
+bool rows_by_xcd(const gc_lattice_params *p, bool rot) {
+    const uint64_t points = (uint64_t)p->nx * p->ny * p->nz;
+    return points >= (1u << 24) && (!rot || p->nx % 32 != 0);
 }
 
 int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d_signs, float iso,
@@ -202,7 +211,7 @@ int launch_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d
     GC_ARG(grid.y <= 65535 && grid.z <= 65535, "grid too large for one launch");
     // (a launch holds fewer than 2^32 threads along x)
     const bool by_xcd =
-        rows_by_xcd(p) && (rot || (uint64_t)grid.x * 8 * 64 * kFieldWaves <= 0xffffffffull);
+        rows_by_xcd(p, rot) && (rot || (uint64_t)grid.x * 8 * 64 * kFieldWaves <= 0xffffffffull);
     const auto pick = by_xcd ? (rot ? pick_tpms<true, true> : pick_tpms<true, false>)
                              : (rot ? pick_tpms<false, true> : pick_tpms<false, false>);
     FieldKernel k = pick(p->tpms, thick, c.prim, c.op);

@@ -232,6 +232,7 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
     const int zn = min(c.lz, c.nz - z0);
 
     // ---- per-z table (one z per thread)
+    bool ztiny = false;  // a box's z distance in (0, 2^-48)
     for (int i = threadIdx.x; i < zn; i += 64 * kFieldWaves) {
         float *e = ztab + i * kZTab;
         float zf = (float)(z0 + i);
@@ -257,10 +258,17 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
         if (c.prim == GC_PRIM_SPHERE) {
             e[ZT_PRIMZ] = pz - c.pc[2];
         } else if (c.prim == GC_PRIM_BOX) {
-            e[ZT_PRIMZ] = __builtin_fabsf(pz - c.pc[2]) - c.ph[2];
+            const float bz = __builtin_fabsf(pz - c.pc[2]) - c.ph[2];
+            e[ZT_PRIMZ] = bz;
+            ztiny |= bz > 0.f && bz < 0x1p-48f;
         }
     }
-    __syncthreads();
+    // The batched form votes, which takes two more barriers: its uneven grids are
+    // faster so (256 of them 4.12 ms, 4.18 without).  A one-grid launch does not
+    // (160^3 with modes 13.3 us so, 12.0 without): its waves look at the table.
+    bool any_ztiny = false;
+    if (PRIM == PRIM_ANY) any_ztiny = __syncthreads_or(ztiny);
+    else __syncthreads();
     const bool xin = x < c.nx;
 
     // ---- per-lane x quantities
@@ -387,12 +395,11 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
     // too) unless a column passes within 2^-48 of its centre, edge or corner
     // axis: then the wave takes the general root at every point.
     const int prim = PRIM == PRIM_ANY ? c.prim : PRIM;
-    bool general = !c.prim_plain;
+    bool general = !c.prim_plain || any_ztiny;
     if (prim != GC_PRIM_NONE) {
         bool near = false;
-        // (a box's z distances in (0, 2^-48): every wave looks at the table, since
-        // a vote of the workgroup takes two more barriers, 1 us of a 128^3 launch)
-        if (prim == GC_PRIM_BOX)
+        // (z distances of a box in (0, 2^-48))
+        if (PRIM != PRIM_ANY && prim == GC_PRIM_BOX)
             for (int i = lane; i < zn; i += 64) {
                 const float bz = ztab[i * kZTab + ZT_PRIMZ];
                 near |= bz > 0.f && bz < 0x1p-48f;
