@@ -263,11 +263,13 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
             ztiny |= bz > 0.f && bz < 0x1p-48f;
         }
     }
-    // The batched form votes, which takes two more barriers: its uneven grids are
-    // faster so (256 of them 4.12 ms, 4.18 without).  A one-grid launch does not
-    // (160^3 with modes 13.3 us so, 12.0 without): its waves look at the table.
+    // The batched form and rotated grids vote, which takes two more barriers:
+    // they are faster so (256 uneven grids 4.12 ms, 4.18 without; a rotated diamond
+    // with modes less a sphere, 203 x 149 x 181, 28.1 us, 29.3 without).  Other
+    // one-grid launches are not (160^3 with modes 13.3 us so, 12.0 without): their
+    // waves look at the table.
     bool any_ztiny = false;
-    if (PRIM == PRIM_ANY) any_ztiny = __syncthreads_or(ztiny);
+    if (PRIM == PRIM_ANY || ROT) any_ztiny = __syncthreads_or(ztiny);
     else __syncthreads();
     const bool xin = x < c.nx;
 
@@ -399,7 +401,7 @@ __device__ __forceinline__ void lattice_brick(const FieldConsts &c, float *__res
     if (prim != GC_PRIM_NONE) {
         bool near = false;
         // (z distances of a box in (0, 2^-48))
-        if (PRIM != PRIM_ANY && prim == GC_PRIM_BOX)
+        if (PRIM != PRIM_ANY && !ROT && prim == GC_PRIM_BOX)
             for (int i = lane; i < zn; i += 64) {
                 const float bz = ztab[i * kZTab + ZT_PRIMZ];
                 near |= bz > 0.f && bz < 0x1p-48f;
