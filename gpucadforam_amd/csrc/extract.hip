@@ -951,9 +951,12 @@ uint32_t run_log2(uint64_t nb, uint64_t plane_blocks) {
     return lr;
 }
 
-// The order of the emission's workgroups (EmitArgs::lr).  Below 1536 blocks
-// mixing them was faster: the edit of 128^3 21.9 us, in runs 22.8; 256^3 100.2
-// and 101.1; 300^3 (1758 blocks) 183.9 and 182.2.
+// The order of the emission's workgroups (EmitArgs::lr).  Small launches gain
+// nothing from runs: over 40 grids of 128 to 5488 blocks the two orders were within
+// 2 % of each other (most often within 1 %), but for grids whose surface leaves
+// part of the planes empty: 272^3 less all but a sphere (1445 blocks) 47.7 us
+// mixed and 51.2 in runs, 340^3 (2710 blocks) 94.9 and 75.3, 192^3 (432) 23.9 and 22.4.
+// 1536 is a line between the first two; where exactly it lies matters little.
 uint32_t emit_order(uint64_t nb, uint64_t plane_blocks, uint32_t lw) {
     return nb < 1536 ? kMixed : run_log2(nb, plane_blocks) + 6 - lw;
 }

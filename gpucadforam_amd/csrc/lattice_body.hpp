@@ -56,10 +56,11 @@ struct FieldConsts {
 // points of its launch.  Rows that end inside a 128-byte line share lines
 // between bricks, which an L2 merges only without the hint: 256 grids of
 // 32..256 points per axis 834 us with it, 652 without, 500^3 198 and 86 (with a
-// row's bricks on one XCD, which alone took 1036 to 834).  A field of the size
-// of the L2s (32 MB) is then still in them when the kernel ends and has to be
-// written back before the next one starts: a 203 x 149 x 181 edit, 22 MB,
-// 70.3 us with the hint, 71.7 without.
+// row's bricks on one XCD, which alone took 1036 to 834).  A field that the L2s
+// hold (32 MB) is then still in them when the kernel ends and has to be written
+// back before the next one starts: a 203 x 149 x 181 edit, 22 MB, 70.3 us with
+// the hint, 71.7 without.  The line at 64 MB is on the safe side of that
+// (rows_by_xcd has both sides between them).
 inline int field_nt_store(int nx, uint64_t launch_points) {
     return nx % 32 == 0 || launch_points < (1u << 24);
 }

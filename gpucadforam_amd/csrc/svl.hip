@@ -501,7 +501,10 @@ __global__ void cg_b_kernel(CgArgs a, int it) {
 // exchange r on their faces (two layers; each tile updates its halo of d by the
 // same d = r + beta d as the owner, so d needs no exchange) and meet twice, in
 // the sums d.q and r.r.  Every element sees the arithmetic of the two-launch
-// form in the same order; the sums are FP64 over the same products.
+// form in the same order.  The sums are FP64 over the same products, in tiles'
+// order instead of ranges', so alpha and beta are the same floats unless the two
+// round to different ones (in none of 13 solves compared, of 4^3 to 162^3 with one
+// and three right-hand sides, up to 391 iterations: all bits the same).
 //
 // There are no fences: an exchanged value travels in one 8-byte word with the
 // number of its iteration, written and read by relaxed agent-scope atomics,
@@ -516,10 +519,12 @@ __global__ void cg_b_kernel(CgArgs a, int it) {
 // only when every tile has counted itself after writing its part.  Otherwise
 // the caller solves by the two-launch form; x has not been written.
 //
-// Measured (us per iteration, two-launch form -> this): three right-hand
-// sides of 120^3 41 -> 20.4; one of 120^3 26.8 -> 12.4, of 61 x 57 x 70 13.7 -> 8.1, of
-// 12^3 (one tile) 13.1 -> 7.2.  What is left is latency: two exchanges of about 2 us each
-// and the barriers of a workgroup that fills its CU.
+// Measured (us per iteration of whole calls, two-launch form -> this): three
+// right-hand sides of 120^3 50 -> 20.3 (41 in its kernels alone), of 100^3 35.6 -> 12.9;
+// one of 162^3 45.4 -> 21.0, of 120^3 26.6 -> 12.4, of 61 x 57 x 70 13.7 -> 8.0, of 12^3
+// (12 tiles) 12.1 -> 6.0, of 4^3 (one tile, nothing to wait for) 11.7 -> 4.2.
+// What is left is latency: two exchanges of about 2 us each and the barriers of a
+// workgroup that fills its CU.
 constexpr int kChipThreads = 1024;            // most threads of a tile's workgroup
 constexpr int kChipZ = 24;                    // longest z run of a tile
 constexpr int kYPass = 3;                     // most passes over a halo layer of a y side

@@ -131,8 +131,8 @@ uint64_t gpucad_sign_words(int32_t nx, int32_t ny, int32_t nz);
  * words), which lets gpucad_extract skip its own classification read. */
 int gpucad_lattice_field(const gc_lattice_params *p, float *d_field, uint64_t *d_signs,
                          float iso, void *stream);
-/* Same, with the number of z planes each workgroup walks (1..128; 0 = default
- * 32).  The batch autotuner sweeps it. */
+/* Same, with the number of z planes each workgroup walks (1..128; 0 = by the
+ * grid's size and options, as gpucad_lattice_field). */
 int gpucad_lattice_field_lz(const gc_lattice_params *p, float *d_field, uint64_t *d_signs,
                             float iso, int32_t lz, void *stream);
 
